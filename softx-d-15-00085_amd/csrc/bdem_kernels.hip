@@ -14,7 +14,7 @@
  *   k_forces             the same code paths writing intermediate results
  *                        (contact lists, per-particle forces) for parity.
  */
-#include "bdem_kernels.hpp"
+#include "bdem_step.hpp"
 
 namespace bdem {
 
@@ -83,84 +83,12 @@ void launch_hash_batch(const DevParams* Pv, const uint32_t* tile_sim, const Step
                      b.omg_cur, b.keys_new, b.status);
 }
 
-/* ------------------------------------------------------------------------ */
-/* Pair forces of one particle (all laws).                                    */
-/* ------------------------------------------------------------------------ */
-struct PairHistCtx {
-  const HistRec* in; int in_cnt; int cursor;
-  HistRec* out; int out_cnt;
-};
-
-/* Force and torque on particle A from contact partner j (all laws), and the
- * spring record of that contact.  The caller accumulates Fc and Tc. */
-template <int LAW>
-__device__ __forceinline__ void contact_force(const DevParams& P, int j, const float4* __restrict__ pos_r,
-                                              const float4* __restrict__ vel_m,
-                                              const float4* __restrict__ omg_t, f3 pa, float ra, f3 va,
-                                              float ma, f3 wa, int ta, const HistRec* hin, int hin_cnt,
-                                              int cursor, HistRec* hrec, f3& Fc, f3& Tc,
-                                              float* tally = nullptr) {
-  const float4 pb = pos_r[j];
-  const float4 vb = vel_m[j];
-  const float4 ob = omg_t[j];
-  HistRec first = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (LAW != BDEM_LAW_REFERENCE && hin_cnt > 0) first = hin[spring_start(hin_cnt, cursor)];
-  if (LAW == BDEM_LAW_REFERENCE) {
-    pair_ref(P, pa, ra, va, ma, wa, ta, xyz(pb), pb.w, xyz(vb), vb.w, xyz(ob), packed_type(ob.w), Fc, Tc,
-             tally);
-  } else {
-    const f3 rel = pa - xyz(pb);
-    const float d = length(rel);
-    const f3 n = rel * (1.0f / d);
-    const float delta = (ra + pb.w) - d;
-    const f3 la = (-1.0f * n) * ra;
-    const f3 lb = n * pb.w;
-    const f3 vc = (va + cross(wa, la)) - (xyz(vb) + cross(xyz(ob), lb));
-    /* R* and m* from one division */
-    const float sr = ra + pb.w, sm = ma + vb.w;
-    const float q = 1.0f / (sr * sm);
-    const float rstar = ((ra * pb.w) * sm) * q;
-    const float mstar = ((ma * vb.w) * sr) * q;
-    const int idb = packed_pid(ob.w);
-    f3 xi = find_spring_first(hin, hin_cnt, idb, cursor, first);
-    /* one type: a wave-uniform address, read by scalar loads that need not
-     * wait for the partner's type word */
-    float e = 0.0f;
-    Fc = history_law(P, n, delta, vc, rstar, mstar, P.one_type ? P.law_pp[0][0] : P.law_pp[ta][packed_type(ob.w)],
-                     xi, tally ? &e : nullptr);
-    /* half the pair's dissipation from each side (the pair is met from both) */
-    if (tally) atomicAdd(tally + TALLY_PP, (0.5f * e) * P.dt);
-    Tc = cross(la, Fc);
-    if (hrec) *hrec = make_float4(xi.x, xi.y, xi.z, __int_as_float(idb));
-  }
-}
-
-/* Per-particle (uncompacted) loop over the contacts found by the scan. */
-template <int LAW>
-__device__ __forceinline__ void particle_contact(const DevParams& P, int j, const float4* __restrict__ pos_r,
-                                                 const float4* __restrict__ vel_m,
-                                                 const float4* __restrict__ omg_t, f3 pa, float ra, f3 va,
-                                                 float ma, f3 wa, int ta, f3& F, f3& T, PairHistCtx* hc,
-                                                 float* tally = nullptr) {
-  f3 Fc, Tc;
-  HistRec* rec = (LAW != BDEM_LAW_REFERENCE && hc->out_cnt < HMAX) ? hc->out + hc->out_cnt : nullptr;
-  contact_force<LAW>(P, j, pos_r, vel_m, omg_t, pa, ra, va, ma, wa, ta, hc->in, hc->in_cnt,
-                     hc->out_cnt, rec, Fc, Tc, tally);
-  if (LAW != BDEM_LAW_REFERENCE && hc->out_cnt < HMAX) ++hc->out_cnt;
-  F = F + Fc;
-  if (P.rotation) T = T + Tc;
-}
-
 /* Pair forces of one particle in two phases: the candidate scan only
  * records contact partners (in the reference order) into this thread's
  * column of an LDS list, then the force loop walks the list.  A wave's force
  * body then runs max(contacts) times instead of max(candidates) times.
  * Particles with more than CLIST contacts (beyond the reference's 32-entry
  * list) finish the tail with a second scan, in the same order. */
-constexpr int CLIST = 12;   /* LDS list entries per thread: 12 KiB + wave staging fits 6 blocks per CU */
-static_assert(CLIST <= HMAX, "springs of the listed contacts are stored first");
-constexpr int STEP_THREADS = 256;
-
 template <int LAW>
 __device__ __forceinline__ int particle_pair_forces(const DevParams& P, const uint2* __restrict__ cells,
                                                     const float4* __restrict__ pos_r,
@@ -271,22 +199,6 @@ __device__ __forceinline__ void wave_pair_forces(const DevParams& P, const float
 /* discharge check -> next key.  Reads the sorted scratch, writes the state.  */
 /* ------------------------------------------------------------------------ */
 
-#define BDEM_STEP_PARAMS                                                                            \
-  int n, const float4* __restrict__ pos_in, const float4* __restrict__ vel_in,                      \
-      const float4* __restrict__ omg_in, const float4* __restrict__ quat_in,                        \
-      float4* __restrict__ pos_out, float4* __restrict__ vel_out, float4* __restrict__ omg_out,     \
-      float4* __restrict__ quat_out, uint32_t* __restrict__ keys_out,                               \
-      const uint32_t* __restrict__ sorted_keys, uint8_t* __restrict__ changed,                      \
-      unsigned long long* __restrict__ sbuf, uint32_t* __restrict__ append,                         \
-      const uint32_t* __restrict__ hwc_in, uint32_t* __restrict__ hwc_out,                          \
-      const HistRec* __restrict__ hr_in, HistRec* __restrict__ hr_out,                              \
-      const HistRec* __restrict__ wr_in, HistRec* __restrict__ wr_out, int hist_cap,                \
-      float* __restrict__ wall_force, int do_kill, uint32_t *status, int *kill_count
-#define BDEM_STEP_ARGS                                                                               \
-  n, pos_in, vel_in, omg_in, quat_in, pos_out, vel_out, omg_out, quat_out, keys_out, sorted_keys, changed, \
-      sbuf, append, hwc_in, hwc_out, hr_in, hr_out, wr_in, wr_out, hist_cap, wall_force, do_kill, status,  \
-      kill_count
-
 /* One wave's 64 consecutive sorted slots (lane i & 63 of the wave).  P and
  * cells are the slot range's simulation: its parameter block and its cell
  * table (indexed by the simulation's own hash); key_base is added to every
@@ -352,117 +264,27 @@ __device__ __forceinline__ void step_wave(const DevParams& P, const uint2* __res
   wave_pair_forces<LAW, BT>(P, pos_in, vel_in, omg_in, clist, nl, base_i, pr, vm, ot, hwc, hr_in, hr_out, hist_cap,
                         *reinterpret_cast<WaveScratch*>(wl), Fpp, Tpp, tally);
 
-  bool chg = false;
+  WallOut wo;
   float dmove = 0.0f;
-  if (alive) {
-    const bool hist_slot = LAW != BDEM_LAW_REFERENCE && pid < hist_cap;
-    if (nc > CLIST) {
-      /* beyond the list: rescan, same order (rare).  Springs of contacts
-       * CLIST .. HMAX-1 are stored after the list's, as in the restatement */
-      PairHistCtx hc{nullptr, 0, 0, nullptr, HMAX};   /* no slot: looked up, not stored */
-      if (hist_slot) {
-        hc.in = hr_in + (size_t)pid * HMAX;
-        hc.in_cnt = min((int)(hwc & 0xFFFFu), HMAX);
-        hc.out = hr_out + (size_t)pid * HMAX;
-        hc.out_cnt = CLIST;
-      }
-      for_each_contact(P, cells, pos_in, i, p, r, [&](int j, float4, int k) {
-        if (k >= CLIST)
-          particle_contact<LAW>(P, j, pos_in, vel_in, omg_in, p, r, v, m, w, ta, Fpp, Tpp, &hc, tally);
-        if (dbg_list && k >= CLIST && k < LIST_STRIDE) dbg_list[(size_t)i * LIST_STRIDE + k] = (uint32_t)j;
-      });
-      /* the reference's 32-entry list overflows (Collision_Detection_BroadPhase.cuh:481) */
-      if (nc > LIST_STRIDE) atomicOr(status, ST_LIST_OVERFLOW);
-    }
-    if (LAW != BDEM_LAW_REFERENCE && nc > HMAX) atomicOr(status, ST_HIST_OVERFLOW);
-    if (!P.rotation) Tpp = mk3(0.f, 0.f, 0.f);
-
-    WallHist wh{nullptr, 0, nullptr, 0};
-    if (LAW != BDEM_LAW_REFERENCE) {
-      if (hist_slot) {
-        wh.in = wr_in + (size_t)pid * WMAX;
-        wh.in_cnt = min((int)((hwc >> 16) & 0xFFu), WMAX);
-        wh.out = wr_out + (size_t)pid * WMAX;
-      } else {
-        wh.out = nullptr; wh.out_cnt = WMAX;   /* no slot: springs are not kept (full count: never written) */
-      }
-    }
-    f3 Fw, Tw;
-    wall_forces(P, ta, p, r, v, w, m, Fw, Tw, &wh, tally);
-    if (wall_force) {
-      wall_force[3 * i] = Fw.x; wall_force[3 * i + 1] = Fw.y; wall_force[3 * i + 2] = Fw.z;
-    }
-    /* a9: lifters; the contact type of the last check is kept for the next step */
-    f3 Fl = mk3(0.f, 0.f, 0.f), Tl = Fl;
-    uint32_t ltype = 0u;
-    if (P.num_dobj > 0)
-      ltype = (uint32_t)lifter_forces(P, ta, p, r, v, w, m, (int)((hwc >> 24) & 3u), Fl, Tl, tally);
-    if (hwc_out) {
-      uint32_t h = ltype << 24;
-      if (LAW != BDEM_LAW_REFERENCE && hist_slot)
-        h |= (uint32_t)(nc < HMAX ? nc : HMAX) | ((uint32_t)wh.out_cnt << 16);
-      hwc_out[i] = h;
-    }
-
-    const float inv_inertia = P.per_particle ? 1.0f / (0.4f * r * r * m) : P.t_inertia[ta];
-    QuatF q{1.f, 0.f, 0.f, 0.f};
-    if (ORIENT) { const float4 q4 = quat_in[i]; q = QuatF{q4.x, q4.y, q4.z, q4.w}; }
-    integrate(P, inv_inertia, m, Fpp, Tpp, Fw, Tw, Fl, Tl, p, v, w, ORIENT ? &q : nullptr);
-    if (SKIN) {
-      /* |p_new - p_old| <= sum |v dt| (1 + 2^-20) + sum |p| 2^-22 (rounding of p += v dt) */
-      dmove = ((fabsf(v.x) + fabsf(v.y) + fabsf(v.z)) * P.dt) * 1.00000095367431640625f +
-              (fabsf(p.x) + fabsf(p.y) + fabsf(p.z)) * 2.384185791015625e-07f;
-    }
-
-    /* a11: Remove_Silo_Discharged_Particles, GPU_Memory_Transfer.cuh:650-664 */
-    if (do_kill && p.y < P.kill_height) {
-      p = cvt(P.max_size);
-      pid = -1;
-      atomicAdd(kill_count, 1);
-    }
-    pos_out[i] = make_float4(p.x, p.y, p.z, r);
-    vel_out[i] = make_float4(v.x, v.y, v.z, m);
-    omg_out[i] = make_float4(w.x, w.y, w.z, __int_as_float(pack_id_type(pid, ta)));
-    if (ORIENT) quat_out[i] = make_float4(q.w, q.x, q.y, q.z);
-    if (SKIN) sk.mask_out[i] = new_mask;
-  } else if (in) {
-    /* dead: inert, copied through */
-    pos_out[i] = pr;
-    vel_out[i] = vm;
-    omg_out[i] = ot;
-    if (ORIENT) quat_out[i] = quat_in[i];
-    if (SKIN) sk.mask_out[i] = 0ull;
-    if (hwc_out) hwc_out[i] = hwc;
-    if (wall_force) { wall_force[3 * i] = 0.f; wall_force[3 * i + 1] = 0.f; wall_force[3 * i + 2] = 0.f; }
-  }
   uint32_t new_key = 0u;
-  if (in) {
-    new_key = key_base + key_of(P, p, pid, status);
-    keys_out[i] = new_key;
-    chg = new_key != sorted_keys[i];
-    changed[i] = chg ? 1 : 0;
+  bool chg = false;
+  if (alive) {
+    contact_tail<LAW>(P, cells, pos_in, vel_in, omg_in, i, p, r, v, w, m, ta, pid, nc, hwc, hr_in, hr_out, hist_cap,
+                      dbg_list, status, Fpp, Tpp, tally);
+    walls_and_lifters<LAW>(P, i, pid, ta, p, r, v, w, m, hwc, wr_in, wr_out, hist_cap, wall_force, wo, tally);
   }
+  if (in)
+    chg = particle_finish<LAW, ORIENT, SKIN>(P, key_base, i, alive, pr, vm, ot, hwc, nc, Fpp, Tpp, wo, new_mask, sk,
+                                             quat_in, pos_out, vel_out, omg_out, quat_out, keys_out, sorted_keys,
+                                             changed, hwc_out, hist_cap, wall_force, do_kill, status, kill_count,
+                                             new_key, dmove);
   if (SKIN) {
     /* the step's largest displacement bound, for the next step's epoch test */
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) dmove = fmaxf(dmove, __shfl_xor(dmove, o, 64));
     if ((threadIdx.x & 63) == 0 && dmove > 0.0f) atomicMax(&sk.vmeta[VM_DMAX + sk.par], __float_as_uint(dmove));
   }
-  /* append changed slots for the next incremental sort (one atomic per wave) */
-  const uint64_t mask = __ballot(chg);
-  if (mask) {
-    const int lane = threadIdx.x & 63;
-    const int leader = __ffsll((unsigned long long)mask) - 1;
-    uint32_t base = 0u;
-    if (lane == leader) base = atomicAdd(append, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader, 64);
-    const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-    const uint32_t at = base + (uint32_t)__popcll(mask & lt);
-    if (chg) {
-      if (at < (uint32_t)n) sbuf[at] = ((unsigned long long)new_key << 32) | (uint32_t)i;
-      else atomicOr(status, ST_SORT_ERROR);   /* a counter left uncleared: never write past the list */
-    }
-  }
+  append_changed(chg, new_key, i, n, sbuf, append, status);
 }
 
 /* One simulation: block b (renumbered XCD-aware) owns sorted slots
@@ -567,6 +389,10 @@ static void launch_batch_l(const BatchLaunch& L, const StepBuffers& b, const uin
 
 void launch_step_batch(const BatchLaunch& L, const StepBuffers& b, const uint32_t* sorted_keys, int hp, int ap,
                        hipStream_t s) {
+  if (L.blocks == 0 && b.n <= TEAM_STEP_MAX) {
+    launch_step_team_batch(L, b, sorted_keys, hp, ap, s);
+    return;
+  }
   if (L.law == BDEM_LAW_REFERENCE) launch_batch_l<BDEM_LAW_REFERENCE>(L, b, sorted_keys, hp, ap, s);
   else if (L.law == BDEM_LAW_LSD_COULOMB) launch_batch_l<BDEM_LAW_LSD_COULOMB>(L, b, sorted_keys, hp, ap, s);
   else launch_batch_l<BDEM_LAW_HERTZ_MINDLIN>(L, b, sorted_keys, hp, ap, s);
@@ -599,6 +425,10 @@ static void launch_step_s(const DevParams* dP, const StepBuffers& b, const uint3
 void launch_step(const DevParams* dP, const StepBuffers& b, const uint32_t* sk, int law, bool orient,
                  int hp, int ap, bool do_kill, bool want_wf, bool energy, const SkinArgs& sa, uint32_t* dl,
                  uint32_t* dn, hipStream_t s) {
+  if (!sa.on && b.n <= TEAM_STEP_MAX) {
+    launch_step_team(dP, b, sk, law, orient, hp, ap, do_kill, want_wf, energy, dl, dn, s);
+    return;
+  }
   if (law == BDEM_LAW_REFERENCE) {
     if (orient) launch_step_s<BDEM_LAW_REFERENCE, true>(dP, b, sk, hp, ap, do_kill, want_wf, energy, sa, dl, dn, s);
     else launch_step_s<BDEM_LAW_REFERENCE, false>(dP, b, sk, hp, ap, do_kill, want_wf, energy, sa, dl, dn, s);

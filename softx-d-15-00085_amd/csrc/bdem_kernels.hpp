@@ -143,6 +143,14 @@ hipError_t launch_sort(const SortArgs& a, bool incremental, int par, hipStream_t
 void launch_step(const DevParams* dP, const StepBuffers& b, const uint32_t* sorted_keys, int law,
                  bool orient, int hist_par, int append_par, bool do_kill, bool want_wall_force, bool energy,
                  const SkinArgs& sk, uint32_t* dbg_list, uint32_t* dbg_nn, hipStream_t s);
+/* The same step by k_step_team (a team of lanes per particle, no skin masks):
+ * launch_step takes it up to TEAM_STEP_MAX slots, where one wave per 64
+ * particles leaves the chip waiting on each wave's serial chain (figures in
+ * bdem_team.hip). */
+constexpr int TEAM_STEP_MAX = 131072;
+void launch_step_team(const DevParams* dP, const StepBuffers& b, const uint32_t* sorted_keys, int law, bool orient,
+                      int hist_par, int append_par, bool do_kill, bool want_wall_force, bool energy,
+                      uint32_t* dbg_list, uint32_t* dbg_nn, hipStream_t s);
 /* Many simulations in one persistent launch (k_step_batch): params[s] is
  * simulation s's parameter block (its key_base offsets its keys and cell
  * table inside the shared sort), tile_sim[t] the simulation owning sorted
@@ -164,6 +172,9 @@ struct BatchLaunch {
 };
 /* Keys of a batch (n a multiple of 64): tile_sim[i / 64] owns slot i. */
 void launch_hash_batch(const DevParams* Pv, const uint32_t* tile_sim, const StepBuffers& b, hipStream_t s);
+/* A plain-grid batch of at most TEAM_STEP_MAX slots, by k_step_team. */
+void launch_step_team_batch(const BatchLaunch& L, const StepBuffers& b, const uint32_t* sorted_keys, int hist_par,
+                            int append_par, hipStream_t s);
 void launch_step_batch(const BatchLaunch& L, const StepBuffers& b, const uint32_t* sorted_keys, int hist_par,
                        int append_par, hipStream_t s);
 /* Rotate_VolObject_Inc on the device: every lifter attached to the drum in
