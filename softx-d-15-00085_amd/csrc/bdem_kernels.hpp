@@ -89,10 +89,8 @@ constexpr int SORT_THREADS = 256;
 constexpr int SORT_ITEMS = 16;
 constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;
 constexpr int RADIX = 256;
-/* incremental resort: 1024 threads own 4096 consecutive slots; the changed
- * composites of a block's window are sorted in LDS up to RS_LCAP */
-constexpr int RS_THREADS = 1024;
-constexpr int RS_TILE = 4096;
+/* incremental resort: the changed composites of a block's window are sorted
+ * in LDS up to RS_LCAP */
 constexpr int RS_LCAP = 4096;
 /* meta words: two append counters used on alternate steps, the size of the
  * last changed set */
