@@ -65,11 +65,15 @@ void dfree(bdem_ctx* c, T*& p) {
 }
 
 void drop_graphs(bdem_ctx* c) {
-  if ((c->graph[0] || c->graph[1]) && c->stream) (void)hipStreamSynchronize(c->stream);
-  for (auto& g : c->graph) {
-    if (g) (void)hipGraphExecDestroy(g);
-    g = nullptr;
-  }
+  bool any = false;
+  for (const auto& by_par : c->graph)
+    for (const auto& g : by_par) any = any || g.exec;
+  if (any && c->stream) (void)hipStreamSynchronize(c->stream);
+  for (auto& by_par : c->graph)
+    for (auto& g : by_par) {
+      if (g.exec) (void)hipGraphExecDestroy(g.exec);
+      g.exec = nullptr;
+    }
 }
 
 void free_all(bdem_ctx* c) {
@@ -609,34 +613,33 @@ int prepare_sorted(bdem_ctx* c, hipEvent_t* ev = nullptr) {
   return BDEM_OK;
 }
 
-/* Two steps whose launches are the same every time: the incremental path
- * of a sphere context with no discharge check, skin masks, stage timing or
- * recording in them.  Every per-step alternation (sorted keys, append
- * counters, spring buffers) has period two, so such a pair is captured
- * once per parity and replayed. */
-bool graph_pair_ok(const bdem_ctx* c) {
+/* A run of `steps` (even) steps whose launches are the same every time: the
+ * incremental path of a sphere context with no discharge check, skin masks,
+ * stage timing or recording in them.  Every per-step alternation (sorted
+ * keys, append counters, spring buffers) has period two, so such a run is
+ * captured once per parity and replayed. */
+bool graph_run_ok(const bdem_ctx* c, int steps) {
   if (!c->graphs_on || c->poly || c->tev.size() || c->dbg_list || c->dbg_nn) return false;
   if (!(c->keys_valid && c->flags_valid && !c->full_next)) return false;
   if (c->b.skin > 0.0f) return false;
   if (c->sim.Kill_Particles) {
     const int interval = (c->has_ext && c->ext.kill_check_interval > 0) ? c->ext.kill_check_interval : 1000;
-    if (c->stepc + 2 >= interval) return false;   /* a check falls in the pair */
+    if (c->stepc + steps >= interval) return false;   /* a check falls in the run */
   }
   return true;
 }
 
-int graph_pair(bdem_ctx* c) {
-  const int key = c->append_par;
-  hipGraphExec_t& g = c->graph[key];
-  if (g && (c->graph_hist[key] != c->hist_par || c->graph_sorted[key] != c->sorted_par)) {
-    (void)hipGraphExecDestroy(g);
-    g = nullptr;
+int graph_run(bdem_ctx* c, int steps) {
+  bdem_ctx::StepGraph& G = c->graph[steps == GRAPH_STEPS ? 1 : 0][c->append_par];
+  if (G.exec && (G.hist != c->hist_par || G.sorted != c->sorted_par)) {
+    (void)hipGraphExecDestroy(G.exec);
+    G.exec = nullptr;
   }
-  if (!g) {
+  if (!G.exec) {
     const int hp = c->hist_par, sp = c->sorted_par, ap = c->append_par, st = c->stepc;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    int rc = bdem_update_sim(c);
-    if (rc == BDEM_OK) rc = bdem_update_sim(c);
+    int rc = BDEM_OK;
+    for (int s = 0; s < steps && rc == BDEM_OK; ++s) rc = bdem_update_sim(c);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (rc != BDEM_OK) {
@@ -646,20 +649,20 @@ int graph_pair(bdem_ctx* c) {
     if (e != hipSuccess) return fail(c, BDEM_EHIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
     if (c->hist_par != hp || c->sorted_par != sp || c->append_par != ap) {
       (void)hipGraphDestroy(graph);
-      return fail(c, BDEM_ESTATE, "internal: a step pair did not return to its parity");
+      return fail(c, BDEM_ESTATE, "internal: a run of steps did not return to its parity");
     }
-    const hipError_t ei = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
+    const hipError_t ei = hipGraphInstantiate(&G.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     if (ei != hipSuccess) {
-      g = nullptr;
+      G.exec = nullptr;
       return fail(c, BDEM_EHIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(ei));
     }
-    c->graph_hist[key] = hp;
-    c->graph_sorted[key] = sp;
-    c->stepc = st;   /* captured, not run: the replay below runs the pair */
+    G.hist = hp;
+    G.sorted = sp;
+    c->stepc = st;   /* captured, not run: the replay below runs the steps */
   }
-  HIPCHK(c, hipGraphLaunch(g, c->stream));
-  if (c->sim.Kill_Particles) c->stepc += 2;
+  HIPCHK(c, hipGraphLaunch(G.exec, c->stream));
+  if (c->sim.Kill_Particles) c->stepc += steps;
   if (c->lift_on && !c->dobj.empty()) c->dobj_dirty = true;
   return BDEM_OK;
 }
@@ -1425,10 +1428,13 @@ int bdem_step(bdem_ctx* c, int nsteps) {
   if (rc) return rc;
   int s = 0;
   while (s < nsteps) {
-    if (nsteps - s >= 2 && graph_pair_ok(c)) {
+    const int run = nsteps - s >= GRAPH_STEPS && graph_run_ok(c, GRAPH_STEPS) ? GRAPH_STEPS
+                    : nsteps - s >= 2 && graph_run_ok(c, 2)                   ? 2
+                                                                              : 0;
+    if (run > 0) {
       HIPCHK(c, hipSetDevice(c->device));
-      if ((rc = graph_pair(c)) != BDEM_OK) return rc;
-      s += 2;
+      if ((rc = graph_run(c, run)) != BDEM_OK) return rc;
+      s += run;
     } else {
       if ((rc = bdem_update_sim(c)) != BDEM_OK) return rc;
       s += 1;

@@ -67,8 +67,12 @@ struct bdem_batch {
 
   bool keys_valid = false;        /* false: the next step hashes and fully sorts */
   int hist_par = 0, sorted_par = 0, append_par = 0, qpar = 0;
-  hipGraphExec_t graph[2] = {nullptr, nullptr};   /* two-step graph per parity */
-  bdem_batch_tuning graph_tune[2]{};
+  /* graphs of 2 and of GRAPH_STEPS steps, per parity */
+  struct StepGraph {
+    hipGraphExec_t exec = nullptr;
+    bdem_batch_tuning tune{};
+  };
+  StepGraph graph[2][2];
 };
 
 namespace {
@@ -96,10 +100,11 @@ int balloc(bdem_batch* B, T** p, size_t count) {
 }
 
 void drop_graphs(bdem_batch* B) {
-  for (auto& g : B->graph) {
-    if (g) (void)hipGraphExecDestroy(g);
-    g = nullptr;
-  }
+  for (auto& by_par : B->graph)
+    for (auto& g : by_par) {
+      if (g.exec) (void)hipGraphExecDestroy(g.exec);
+      g.exec = nullptr;
+    }
 }
 
 void free_buffers(bdem_batch* B) {
@@ -195,20 +200,20 @@ bool same_launch(const bdem_batch_tuning& a, const bdem_batch_tuning& b) {
   return a.threads == b.threads && a.waves_per_cu == b.waves_per_cu && a.grab == b.grab;
 }
 
-/* Two steady-state steps, captured once per parity and launch shape. */
-int graph_pair(bdem_batch* B) {
-  const int key = B->append_par;
-  if (B->graph[key] && !same_launch(B->graph_tune[key], B->tune)) {
-    (void)hipGraphExecDestroy(B->graph[key]);
-    B->graph[key] = nullptr;
+/* `steps` (even) steady-state steps, captured once per parity and launch shape. */
+int graph_run(bdem_batch* B, int steps) {
+  bdem_batch::StepGraph& G = B->graph[steps == GRAPH_STEPS ? 1 : 0][B->append_par];
+  if (G.exec && !same_launch(G.tune, B->tune)) {
+    (void)hipGraphExecDestroy(G.exec);
+    G.exec = nullptr;
   }
-  if (!B->graph[key]) {
+  if (!G.exec) {
     /* the launches advance the host-side parities; capture from a copy of
-     * them and check that two steps bring them back */
+     * them and check that the steps bring them back */
     const int hp = B->hist_par, sp = B->sorted_par, ap = B->append_par, qp = B->qpar;
     BHIP(B, hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
-    int rc = launch_one(B);
-    if (rc == BDEM_OK) rc = launch_one(B);
+    int rc = BDEM_OK;
+    for (int s = 0; s < steps && rc == BDEM_OK; ++s) rc = launch_one(B);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(B->stream, &g);
     if (rc != BDEM_OK) {
@@ -218,17 +223,17 @@ int graph_pair(bdem_batch* B) {
     if (e != hipSuccess) return bfail(B, BDEM_EHIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
     if (B->hist_par != hp || B->sorted_par != sp || B->append_par != ap || B->qpar != qp) {
       (void)hipGraphDestroy(g);
-      return bfail(B, BDEM_ESTATE, "internal: a step pair did not return to its parity");
+      return bfail(B, BDEM_ESTATE, "internal: a run of steps did not return to its parity");
     }
-    e = hipGraphInstantiate(&B->graph[key], g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&G.exec, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (e != hipSuccess) {
-      B->graph[key] = nullptr;
+      G.exec = nullptr;
       return bfail(B, BDEM_EHIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
     }
-    B->graph_tune[key] = B->tune;
+    G.tune = B->tune;
   }
-  BHIP(B, hipGraphLaunch(B->graph[key], B->stream));
+  BHIP(B, hipGraphLaunch(G.exec, B->stream));
   return BDEM_OK;
 }
 
@@ -461,8 +466,9 @@ int bdem_batch_step(bdem_batch* B, int nsteps) {
   int s = 0;
   while (s < nsteps) {
     if (B->keys_valid && B->tune.use_graph && nsteps - s >= 2) {
-      if ((rc = graph_pair(B)) != BDEM_OK) return rc;
-      s += 2;
+      const int run = nsteps - s >= GRAPH_STEPS ? GRAPH_STEPS : 2;
+      if ((rc = graph_run(B, run)) != BDEM_OK) return rc;
+      s += run;
     } else {
       if ((rc = launch_one(B)) != BDEM_OK) return rc;
       s += 1;

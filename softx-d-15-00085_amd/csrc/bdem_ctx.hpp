@@ -15,6 +15,10 @@ using bdem::PolyBuffers;
 using bdem::StatsWords;
 using bdem::StepBuffers;
 
+/* Steps per long graph: replays follow each other with about 8 us between
+ * them whatever their length, so two-step graphs lose 4 us a step. */
+constexpr int GRAPH_STEPS = 16;
+
 struct bdem_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -66,10 +70,13 @@ struct bdem_ctx {
   uint32_t* dbg_list = nullptr;  /* debug: the contacts the step kernel used */
   uint32_t* dbg_nn = nullptr;
   int stepc = 0;
-  /* two steady-state steps captured as a HIP graph, one per parity of the
-   * per-step alternations (see bdem_step) */
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
-  int graph_hist[2] = {0, 0}, graph_sorted[2] = {0, 0};
+  /* runs of steady-state steps captured as HIP graphs, by length (2 or
+   * GRAPH_STEPS) and parity of the per-step alternations (see bdem_step) */
+  struct StepGraph {
+    hipGraphExec_t exec = nullptr;
+    int hist = 0, sorted = 0;
+  };
+  StepGraph graph[2][2];
   bool graphs_on = true;
   /* stage timing: one event per stage boundary per recorded step */
   std::vector<hipEvent_t> tev;
