@@ -1574,7 +1574,7 @@ int bdem_debug_forces(bdem_ctx* c, float* fpp, float* tpp, float* fw, float* tw,
   float* d = nullptr;
   HIPCHK(c, hipMalloc((void**)&d, (size_t)n * 12 * sizeof(float)));
   if (c->poly)
-    launch_poly_forces(c->dp, c->dshape, c->b, c->pb, d, d + 3 * (size_t)n, d + 6 * (size_t)n, d + 9 * (size_t)n,
+    launch_poly_forces(c->dp, c->dshape, c->b, c->pb, c->b.keys_sorted[c->sorted_par], d, d + 3 * (size_t)n, d + 6 * (size_t)n, d + 9 * (size_t)n,
                        c->stream);
   else
     launch_forces(c->dp, c->b, c->hp.law, c->hist_par, d, d + 3 * (size_t)n, d + 6 * (size_t)n,

@@ -194,7 +194,7 @@ void launch_poly_step(const DevParams* dP, const bdem_poly_shape* dshape, const 
 void launch_poly_world_shapes(const DevParams* dP, const bdem_poly_shape* dshape, const StepBuffers& b,
                               const PolyBuffers& pb, hipStream_t s);
 void launch_poly_forces(const DevParams* dP, const bdem_poly_shape* dshape, const StepBuffers& b, const PolyBuffers& pb,
-                        float* fpp, float* tpp, float* fw, float* tw, hipStream_t s);
+                        const uint32_t* sorted_keys, float* fpp, float* tpp, float* fw, float* tw, hipStream_t s);
 
 /* Ensemble statistics of the current state (bdem_stats.hip): live
  * particles with y > min_y (count, sum of |v|*0.01, the fastest as

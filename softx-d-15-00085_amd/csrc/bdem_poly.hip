@@ -9,8 +9,9 @@
  *                   face-centroid slot): world-frame shapes into `rot`,
  *                   written coalesced (RotatePolyhedra, Utilities.cuh:420-479)
  *   k_poly_list     bounding-sphere contact list in the reference order (the
- *                   sphere broad phase), plus a queue of (particle, slot)
- *                   work items appended one atomic per wave
+ *   k_poly_list2    sphere broad phase; the second form for larger counts),
+ *                   plus a queue of (particle, slot) work items appended one
+ *                   atomic per block
  *   k_poly_pairs    one thread per queued pair, grid-stride over the queue:
  *                   the separating-plane test of the two facing faces; the
  *                   pairs it does not separate go to a second queue
@@ -30,7 +31,7 @@
  */
 #include <atomic>
 
-#include "bdem_kernels.hpp"
+#include "bdem_step.hpp"
 
 namespace bdem {
 
@@ -1219,10 +1220,59 @@ __global__ __launch_bounds__(256) void k_poly_rotate(const DevParams* __restrict
   rot[t] = make_float4(out.x, out.y, out.z, 0.0f);
 }
 
-constexpr int LIST_LANES = 32;   /* particles per wave in the polyhedra list kernel (a power of two) */
+/* A particle's list (m of its c contacts, in LDS) to memory by its G lanes,
+ * and its pairs to the work queue, one reservation per block of `WAVES`
+ * waves.  Every thread of the block calls. */
+template <int G, int WAVES>
+__device__ __forceinline__ void list_store(int n, int i, bool in, int c, const uint32_t* mine,
+                                           uint32_t* __restrict__ list32, uint32_t* __restrict__ nn,
+                                           uint32_t* __restrict__ queue, uint32_t* __restrict__ qcount,
+                                           uint32_t* status) {
+  __shared__ uint32_t wtotal[WAVES], qbase;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane & (G - 1);
+  if (in && sub == 0) {
+    nn[i] = (uint32_t)c;
+    if (c > LIST_STRIDE) atomicOr(status, ST_LIST_OVERFLOW);
+  }
+  const int m = in ? min(c, LIST_STRIDE) : 0;
+  /* queue places: the wave's particles in order, each lane's entries k = sub, sub + G, ... */
+  const int own = m > sub ? (m - sub + G - 1) / G : 0;
+  int incl = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += v;
+  }
+  if (lane == 63) wtotal[wave] = (uint32_t)incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t t = 0u;
+    for (int w = 0; w < WAVES; ++w) t += wtotal[w];
+    qbase = t ? atomicAdd(qcount, t) : 0u;
+  }
+  __syncthreads();
+  uint32_t at = qbase + (uint32_t)(incl - own);
+  for (int w = 0; w < wave; ++w) at += wtotal[w];
+  const uint32_t cap = (uint32_t)n * LIST_STRIDE;
+  for (int k = sub; k < m; k += G, ++at) {
+    const uint32_t slot = (uint32_t)i * LIST_STRIDE + (uint32_t)k;
+    list32[slot] = mine[k];
+    if (at < cap) queue[at] = slot;
+  }
+}
 
 /* Bounding-sphere contact list (the sphere broad phase: Kernel_BroadCollision-
- * Detection_NonSymmetry, 32 slots, full count) and the pair work queue. */
+ * Detection_NonSymmetry, 32 slots, full count) and the pair work queue.
+ *
+ * A grid cell (2 x the largest bounding radius) holds about seven hulls, so
+ * a hull tests some 190 candidates to list 12.  Sixteen lanes share them,
+ * four particles to a wave: a lane per stencil row, then a candidate per
+ * lane and round (team_contacts).  One lane per particle walked the rows one
+ * after another with half its lanes idle: 137 us at 200,000 hulls (VALU
+ * issue), 68 us at 3,001, where the chain is all there is. */
+constexpr int LIST_G = 16, LIST_NP = 64 / LIST_G;
+constexpr int LIST_CAND = 256;
+constexpr int LIST_BLOCK = 4 * LIST_NP;   /* particles per 256-thread block */
 __global__ __launch_bounds__(256) void k_poly_list(const DevParams* __restrict__ Pp, int n,
                                                    const uint2* __restrict__ cells,
                                                    const float4* __restrict__ pos_r,
@@ -1231,39 +1281,165 @@ __global__ __launch_bounds__(256) void k_poly_list(const DevParams* __restrict__
                                                    uint32_t* __restrict__ queue, uint32_t* __restrict__ qcount,
                                                    uint32_t* status) {
   const DevParams& P = *Pp;
-  __shared__ __align__(16) unsigned char wlds[4][sizeof(WaveStage)];
-  /* 32 consecutive particles per wave (lanes 32-63 idle): twice the waves
-   * of one particle per lane, to hide the scan's memory latency at the
-   * particle counts of a polyhedra run */
-  const int lane = threadIdx.x & 63;
-  const bool own = lane < LIST_LANES;
-  const int i = (blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)) * LIST_LANES + (lane & (LIST_LANES - 1));
-  const bool live = own && i < n && packed_pid(omg[i].w) >= 0;
+  __shared__ uint32_t cand[4][LIST_NP][LIST_CAND];
+  __shared__ uint32_t list[4][LIST_NP][LIST_STRIDE];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int ps = lane / LIST_G, sub = lane & (LIST_G - 1);
+  const int i = xcd_block(blockIdx.x, gridDim.x) * LIST_BLOCK + wave * LIST_NP + ps;
+  const bool in = i < n;
+  const bool live = in && packed_pid(omg[i].w) >= 0;
   const float4 pr = live ? pos_r[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-  /* the staged stencil scan of a wave of consecutive particles */
-  int c = for_each_contact_wave(P, cells, pos_r, (uint32_t)n, i, xyz(pr), pr.w, live,
-                                *reinterpret_cast<WaveStage*>(wlds[threadIdx.x >> 6]), [&](int j, float4, int k) {
-                                  if (k < LIST_STRIDE) list32[(size_t)i * LIST_STRIDE + k] = (uint32_t)j;
-                                });
-  if (!live) c = 0;
-  if (c > LIST_STRIDE) atomicOr(status, ST_LIST_OVERFLOW);
-  if (own && i < n) nn[i] = (uint32_t)c;
-  const int m = c < LIST_STRIDE ? c : LIST_STRIDE;
-  /* wave prefix of the per-lane pair counts, one atomic per wave */
-  int incl = m;
+  uint32_t* const mine = list[wave][ps];
+  const int c = team_contacts<LIST_G, LIST_CAND>(P, cells, pos_r, (uint32_t)n, i, xyz(pr), pr.w, live, cand[wave][ps],
+                                                 [&](int j, int k) {
+                                                   if (k < LIST_STRIDE) mine[k] = (uint32_t)j;
+                                                 });
+  __builtin_amdgcn_wave_barrier();
+  list_store<LIST_G, 4>(n, i, in, c, mine, list32, nn, queue, qcount, status);
+}
+
+/* The same list for larger counts, two lanes per particle and 32 particles
+ * per wave: the gathers of k_poly_list are bound by their addresses there.
+ * The wave stages the three rows of one y layer (cells, then candidates) by
+ * coalesced loads into LDS; a particle's two lanes test one half each of a
+ * row's candidates into a bit mask, and the masks' set bits, the first
+ * half's before the second's, are the contacts in order. */
+constexpr int LIST_TEAM_MAX = 24576;
+constexpr int LIST2_POS = 96;
+struct ListStage {
+  float4 pos[3][LIST2_POS];
+  uint2 cell[3][64];
+  uint32_t list[32][LIST_STRIDE + 1];   /* odd stride: both lanes of 32 particles write it */
+};
+constexpr int LIST2_WAVES = 4, LIST2_BLOCK = 32 * LIST2_WAVES;
+__global__ __launch_bounds__(64 * LIST2_WAVES) void k_poly_list2(const DevParams* __restrict__ Pp, int n,
+                                                                 const uint2* __restrict__ cells,
+                                                                 const float4* __restrict__ pos_r,
+                                                                 const float4* __restrict__ omg,
+                                                                 const uint32_t* __restrict__ sorted_keys,
+                                                                 uint32_t* __restrict__ list32,
+                                                                 uint32_t* __restrict__ nn,
+                                                                 uint32_t* __restrict__ queue,
+                                                                 uint32_t* __restrict__ qcount, uint32_t* status) {
+  const DevParams& P = *Pp;
+  __shared__ ListStage stage[LIST2_WAVES];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  ListStage& st = stage[wave];
+  const int ps = lane >> 1, sub = lane & 1;
+  const int i = xcd_block(blockIdx.x, gridDim.x) * LIST2_BLOCK + wave * 32 + ps;
+  const bool in = i < n;
+  const bool live = in && packed_pid(omg[i].w) >= 0;
+  const float4 pr = live ? pos_r[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  const f3 pa = xyz(pr);
+  const float ra = pr.w;
+  /* the particles' keys ascend: the wave's first and last key of a cell */
+  const uint32_t key = in ? sorted_keys[i] : 0xFFFFFFFFu;
+  const uint64_t gm = __ballot(key < P.C);
+  const uint32_t hmin = __builtin_amdgcn_readfirstlane(key);
+  const uint32_t hmax = gm ? (uint32_t)__builtin_amdgcn_readlane((int)key, 63 - __clzll((long long)gm)) : 0u;
+  const bool narrow = gm != 0ull && hmax - hmin + 3u <= 64u;   /* a row's cells fit one load */
+  int g[3];
+  grid_pos(P, pa, g);
+  const int xs = max(g[0] - 1, 0), xe = min(g[0] + 1, P.nx - 1);
+  const uint2 none = make_uint2(0xFFFFFFFFu, 0u);
+  uint32_t* const mine = st.list[ps];
+  int count = 0;
+  for (int dy = 0; dy < 3; ++dy) {
+    RowWin w[3];
+    uint2 ce[3];
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int o = __shfl_up(incl, d, 64);
-    if (lane >= d) incl += o;
+    for (int z = 0; z < 3; ++z) {
+      w[z] = row_window(P, hmin, hmax, 3 * dy + z);
+      ce[z] = none;
+      if (narrow && w[z].ok && (uint32_t)lane < w[z].wn) ce[z] = cells[w[z].w0 + lane];
+    }
+    uint32_t pmin[3], pcnt[3];
+    float4 q0[3], q1[3];
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      const RowStage rs = row_stage(ce[z], none, (uint32_t)n);
+      pmin[z] = rs.pmin;
+      pcnt[z] = rs.any && rs.pmax - rs.pmin <= (uint32_t)LIST2_POS ? rs.pmax - rs.pmin : 0u;
+      q0[z] = make_float4(0.f, 0.f, 0.f, 0.f);
+      q1[z] = q0[z];
+      if ((uint32_t)lane < pcnt[z]) q0[z] = pos_r[pmin[z] + lane];
+      if ((uint32_t)lane + 64u < pcnt[z]) q1[z] = pos_r[pmin[z] + 64u + lane];
+    }
+    __builtin_amdgcn_wave_barrier();   /* the previous layer's reads are done */
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      st.cell[z][lane] = ce[z];
+      st.pos[z][lane] = q0[z];
+      if (lane + 64 < LIST2_POS) st.pos[z][lane + 64] = q1[z];
+    }
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t y = (uint32_t)g[1] + (uint32_t)dy - 1u;
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      const uint32_t zz = (uint32_t)g[2] + (uint32_t)z - 1u;
+      uint32_t lo = 0u, cnt = 0u;
+      if (live && xs <= xe && y < (uint32_t)P.ny && zz < (uint32_t)P.nz) {
+        const uint32_t h0 = hash_of(P, xs, (int)y, (int)zz), h1 = hash_of(P, xe, (int)y, (int)zz);
+        if (h1 < P.C) {   /* at most three cells, first and last occupied entry */
+          uint2 c0 = none, c1 = none, c2 = none;
+          if (narrow && h0 >= w[z].w0 && h1 < w[z].w0 + w[z].wn) {
+            const uint2* const row = st.cell[z] - w[z].w0;
+            c0 = row[h0];
+            if (h0 + 1u <= h1) c1 = row[h0 + 1u];
+            if (h0 + 2u <= h1) c2 = row[h0 + 2u];
+          } else {   /* spread keys, or a particle outside the grid */
+            c0 = cells[h0];
+            if (h0 + 1u <= h1) c1 = cells[h0 + 1u];
+            if (h0 + 2u <= h1) c2 = cells[h0 + 2u];
+          }
+          const uint32_t a = min(min(c0.x, c1.x), c2.x);
+          if (a != 0xFFFFFFFFu) {
+            uint32_t b = c2.x != 0xFFFFFFFFu ? c2.y : (c1.x != 0xFFFFFFFFu ? c1.y : c0.y);
+            b = min(b, (uint32_t)n);   /* table entries never exceed n; kept in range regardless */
+            lo = a;
+            cnt = b > a ? b - a : 0u;
+          }
+        }
+      }
+      const bool staged = lo >= pmin[z] && lo + cnt <= pmin[z] + pcnt[z];
+      for (uint32_t base = 0u; __any((int)(base < cnt)); base += 64u) {
+        const uint32_t rem = base < cnt ? min(cnt - base, 64u) : 0u;
+        const uint32_t half = (rem + 1u) >> 1;
+        const uint32_t j0 = lo + base + (sub ? half : 0u), len = sub ? rem - half : half;
+        uint32_t mask = 0u;
+        if (__all((int)(staged || len == 0u))) {
+          /* four reads in flight; past the end the last entry is read again */
+          const uint32_t at = j0 - pmin[z], last = len ? len - 1u : 0u;
+          const float4* const src = st.pos[z] + (len ? at : 0u);
+          for (uint32_t t = 0u; t < len; t += 4u) {
+            float4 pb[4];
+#pragma unroll
+            for (uint32_t u = 0u; u < 4u; ++u) pb[u] = src[min(t + u, last)];
+#pragma unroll
+            for (uint32_t u = 0u; u < 4u; ++u) mask |= (overlaps(pa, ra, pb[u]) && t + u < len ? 1u : 0u) << (t + u);
+          }
+        } else {
+          for (uint32_t t = 0u; t < len; ++t) {
+            const bool hit = overlaps(pa, ra, pos_r[j0 + t]);
+            mask |= (hit ? 1u : 0u) << t;
+          }
+        }
+        const uint32_t self = (uint32_t)i - j0;
+        if (self < len) mask &= ~(1u << self);
+        const int c = __popc(mask), other = __shfl_xor(c, 1, 64);
+        int k = count + (sub ? other : 0);
+        count += c + other;
+        while (mask) {
+          const int t = __ffs(mask) - 1;
+          mask &= mask - 1u;
+          if (k < LIST_STRIDE) mine[k] = j0 + (uint32_t)t;
+          ++k;
+        }
+      }
+    }
   }
-  const int total = __shfl(incl, 63, 64);
-  uint32_t base = 0u;
-  if (lane == 63 && total > 0) base = atomicAdd(qcount, (uint32_t)total);
-  base = __shfl(base, 63, 64);
-  const uint32_t at = base + (uint32_t)(incl - m);
-  const uint32_t cap = (uint32_t)n * LIST_STRIDE;
-  for (int k = 0; k < m; ++k)
-    if (at + (uint32_t)k < cap) queue[at + k] = (uint32_t)i * LIST_STRIDE + (uint32_t)k;
+  __builtin_amdgcn_wave_barrier();
+  list_store<2, LIST2_WAVES>(n, i, in, count, mine, list32, nn, queue, qcount, status);
 }
 
 /* One queued pair per thread, grid-stride so that every wave exits once the
@@ -1613,13 +1789,19 @@ static unsigned resident_blocks(K kernel, int slot) {
 }
 
 static void launch_poly_forces_common(const DevParams* dP, const bdem_poly_shape* dshape, const StepBuffers& b,
-                                      const PolyBuffers& pb, bool energy, hipStream_t s) {
+                                      const PolyBuffers& pb, const uint32_t* sk, bool energy, hipStream_t s) {
   const size_t rot_threads = (size_t)b.n * pb.L.stride;
   hipLaunchKernelGGL(k_poly_rotate, dim3((unsigned)((rot_threads + 255) / 256)), dim3(256), 0, s, dP, pb.local,
                      b.n, pb.L, b.pos_srt, b.omg_srt, b.quat_srt, pb.rot, pb.qcount);
-  hipLaunchKernelGGL(k_poly_list, dim3((b.n + 4 * LIST_LANES - 1) / (4 * LIST_LANES)), dim3(256), 0, s, dP, b.n,
-                     b.cells, b.pos_srt,
-                     b.omg_srt, pb.list, pb.nn, pb.queue, pb.qcount, b.status);
+  /* sixteen lanes a particle while the chip holds their waves (8,192) a few
+   * times over: 11 against 36 us at 3,001 hulls, level near 30,000, 41
+   * against 20 us at 50,000 */
+  if (b.n <= LIST_TEAM_MAX)
+    hipLaunchKernelGGL(k_poly_list, dim3((b.n + LIST_BLOCK - 1) / LIST_BLOCK), dim3(256), 0, s, dP, b.n, b.cells,
+                       b.pos_srt, b.omg_srt, pb.list, pb.nn, pb.queue, pb.qcount, b.status);
+  else
+    hipLaunchKernelGGL(k_poly_list2, dim3((b.n + LIST2_BLOCK - 1) / LIST2_BLOCK), dim3(64 * LIST2_WAVES), 0, s, dP,
+                       b.n, b.cells, b.pos_srt, b.omg_srt, sk, pb.list, pb.nn, pb.queue, pb.qcount, b.status);
   /* both pair kernels loop over their queues with the resident grid; the
    * first splits its queue by XCD (a grid of whole XCD multiples) */
   static_assert(POLY_PAIR_BLOCKS % NUM_XCD == 0, "the pair kernel splits its queue by XCD");
@@ -1644,7 +1826,7 @@ void launch_poly_world_shapes(const DevParams* dP, const bdem_poly_shape* dshape
 void launch_poly_step(const DevParams* dP, const bdem_poly_shape* dshape, const StepBuffers& b, const PolyBuffers& pb,
                       const uint32_t* sk, int ap, bool do_kill, bool want_wf, bool lifters, bool energy,
                       hipStream_t s) {
-  launch_poly_forces_common(dP, dshape, b, pb, energy, s);
+  launch_poly_forces_common(dP, dshape, b, pb, sk, energy, s);
   /* the lifter search needs private arrays (scratch): only its own instantiation carries it */
   auto k = lifters ? k_poly_finish<false, true> : k_poly_finish<false, false>;
   hipLaunchKernelGGL(k, dim3((b.n + 255) / 256), dim3(256), 0, s, dP, dshape, b.n, pb.L,
@@ -1655,8 +1837,8 @@ void launch_poly_step(const DevParams* dP, const bdem_poly_shape* dshape, const 
 }
 
 void launch_poly_forces(const DevParams* dP, const bdem_poly_shape* dshape, const StepBuffers& b, const PolyBuffers& pb,
-                        float* fpp, float* tpp, float* fw, float* tw, hipStream_t s) {
-  launch_poly_forces_common(dP, dshape, b, pb, false, s);
+                        const uint32_t* sk, float* fpp, float* tpp, float* fw, float* tw, hipStream_t s) {
+  launch_poly_forces_common(dP, dshape, b, pb, sk, false, s);
   hipLaunchKernelGGL((k_poly_finish<true, false>), dim3((b.n + 255) / 256), dim3(256), 0, s, dP, dshape, b.n, pb.L,
                      pb.rot, pb.nn, pb.pf, pb.pt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, nullptr, nullptr,
                      nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0,

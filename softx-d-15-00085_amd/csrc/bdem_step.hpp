@@ -1,6 +1,6 @@
 /*
- * bdem_step.hpp - the pieces of one sphere step that its kernels share: a
- * contact's force, the contacts past the list, walls and lifters, the
+ * bdem_step.hpp - the pieces of one step that its kernels share: a team's
+ * contact search, a contact's force, the contacts past the list, walls and lifters, the
  * integration with the next key, and the changed-list append (internal).
  */
 #pragma once
@@ -242,6 +242,92 @@ __device__ __forceinline__ void append_changed(bool chg, uint32_t new_key, int i
       else atomicOr(status, ST_SORT_ERROR);   /* a counter left uncleared: never write past the list */
     }
   }
+}
+
+/* The contacts of one particle by its team (the G consecutive lanes that
+ * hold the same arguments): visit(j, k) on the lane that found contact k,
+ * k counting in the traversal order of for_each_contact.  Returns the count
+ * (team-uniform).  `active` is team-uniform; every lane of the wave calls.
+ * cand: the team's LDS list, CAND candidates at a time. */
+template <int G, int CAND, class Visit>
+__device__ __forceinline__ int team_contacts(const DevParams& P, const uint2* __restrict__ cells,
+                                             const float4* __restrict__ pos_r, uint32_t n, int i, f3 pa, float ra,
+                                             bool active, uint32_t* cand, Visit&& visit) {
+  constexpr int NR = (9 + G - 1) / G;
+  const int lane = threadIdx.x & 63, sub = lane & (G - 1), lead = lane & ~(G - 1);
+  int g[3];
+  grid_pos(P, pa, g);
+  const int xs = max(g[0] - 1, 0), xe = min(g[0] + 1, P.nx - 1);
+  uint32_t lo[NR], cnt[NR];
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    const int r = sub + G * q;
+    const uint32_t y = (uint32_t)g[1] + (uint32_t)(r / 3) - 1u, z = (uint32_t)g[2] + (uint32_t)(r % 3) - 1u;
+    lo[q] = 0u;
+    cnt[q] = 0u;
+    if (active && r < 9 && xs <= xe && y < (uint32_t)P.ny && z < (uint32_t)P.nz) {
+      const uint32_t h0 = hash_of(P, xs, (int)y, (int)z), h1 = hash_of(P, xe, (int)y, (int)z);
+      if (h1 < P.C) {   /* at most three cells, first and last occupied entry */
+        const uint2 none = make_uint2(0xFFFFFFFFu, 0u);
+        const uint2 c0 = cells[h0];
+        uint2 c1 = none, c2 = none;
+        if (h0 + 1u <= h1) c1 = cells[h0 + 1u];
+        if (h0 + 2u <= h1) c2 = cells[h0 + 2u];
+        const uint32_t a = min(min(c0.x, c1.x), c2.x);
+        if (a != 0xFFFFFFFFu) {
+          uint32_t b = c2.x != 0xFFFFFFFFu ? c2.y : (c1.x != 0xFFFFFFFFu ? c1.y : c0.y);
+          b = min(b, n);   /* table entries never exceed n; kept in range regardless */
+          lo[q] = a;
+          cnt[q] = b > a ? b - a : 0u;
+        }
+      }
+    }
+  }
+  /* offsets of the rows in the numbering of all candidates */
+  uint32_t off[NR], total = 0u;
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    uint32_t incl = cnt[q];
+#pragma unroll
+    for (int o = 1; o < G; o <<= 1) {
+      const uint32_t v = (uint32_t)__shfl_up((int)incl, o, G);
+      if (sub >= o) incl += v;
+    }
+    off[q] = total + incl - cnt[q];
+    total += (uint32_t)__shfl((int)incl, G - 1, G);
+  }
+  int count = 0;
+  const uint32_t self = i < (int)n ? (uint32_t)i : 0u;
+  for (uint32_t c0 = 0u; __any((int)(c0 < total)); c0 += (uint32_t)CAND) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q)
+      for (uint32_t k = 0u; k < cnt[q]; ++k) {
+        const uint32_t at = off[q] + k - c0;
+        if (at < (uint32_t)CAND) cand[at] = lo[q] + k;
+      }
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t m = total > c0 ? min(total - c0, (uint32_t)CAND) : 0u;
+    for (uint32_t t0 = 0u; __any((int)(t0 < m)); t0 += 4u * G) {
+      uint32_t j[4];
+      float4 pb[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t t = t0 + (uint32_t)(u * G + sub);
+        j[u] = t < m ? cand[t] : self;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) pb[u] = pos_r[j[u]];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool hit = j[u] != self && overlaps(pa, ra, pb[u]);
+        const uint32_t bits = (uint32_t)(__ballot(hit) >> lead) & ((1u << G) - 1u);
+        if (hit) visit((int)j[u], count + __popc(bits & ((1u << sub) - 1u)));
+        count += __popc(bits);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  return count;
 }
 
 }  // namespace bdem
