@@ -788,13 +788,15 @@ int bdem_set_simulation_data(bdem_ctx* c, const bdem_WOBJ* wobj, const bdem_POBJ
     ALLOC(pb.rot, (size_t)n * pb.L.stride);
     ALLOC(pb.list, (size_t)n * LIST_STRIDE);
     ALLOC(pb.nn, (size_t)n);
-    ALLOC(pb.queue, (size_t)n * LIST_STRIDE);
-    ALLOC(pb.equeue, (size_t)n * LIST_STRIDE);
-    ALLOC(pb.qcount, 4);
+    ALLOC(pb.equeue, (size_t)POLY_SUBQ * poly_subqueue_capacity(n));
+    ALLOC(pb.qcount, POLY_QCOUNTS * POLY_QSTRIDE);
+    ALLOC(pb.hitf, (size_t)n * LIST_STRIDE);
     ALLOC(pb.pf, (size_t)n * LIST_STRIDE);
     ALLOC(pb.pt, (size_t)n * LIST_STRIDE);
     ALLOC(pb.hint, (size_t)n * LIST_STRIDE);
     launch_fill_u32(reinterpret_cast<uint32_t*>(pb.hint), (size_t)n * LIST_STRIDE * 2, 0xFFFFFFFFu, c->stream);
+    launch_fill_u32(pb.nn, (size_t)n, 0u, c->stream);
+    launch_fill_u32(pb.qcount, POLY_QCOUNTS * POLY_QSTRIDE, 0u, c->stream);
   }
 #undef ALLOC
   HIPCHK(c, hipMemset(b.status, 0, sizeof(uint32_t)));
@@ -1617,7 +1619,12 @@ int bdem_debug_poly_queues(bdem_ctx* c, unsigned int* counts) {
   if (!c->poly) return fail(c, BDEM_EINVAL, "not a polyhedra context (particle_type 1)");
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  HIPCHK(c, hipMemcpy(counts, c->pb.qcount, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost));
+  std::vector<uint32_t> nn((size_t)c->b.n), q(POLY_QCOUNTS * POLY_QSTRIDE);
+  HIPCHK(c, hipMemcpy(nn.data(), c->pb.nn, nn.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+  HIPCHK(c, hipMemcpy(q.data(), c->pb.qcount, q.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+  counts[0] = counts[1] = 0u;
+  for (uint32_t v : nn) counts[0] += std::min(v, (uint32_t)LIST_STRIDE);
+  for (int s = 0; s < POLY_SUBQ; ++s) counts[1] += 2u * q[(size_t)s * POLY_QSTRIDE];   /* a pair is listed from both sides */
   return BDEM_OK;
 }
 

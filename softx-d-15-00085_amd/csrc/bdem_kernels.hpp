@@ -77,13 +77,25 @@ struct PolyBuffers {
   float4* rot;                         /* n * stride */
   uint32_t* list;                      /* n * 32 partner slots */
   uint32_t* nn;                        /* full contact count per particle */
-  uint32_t* queue;                     /* (particle * 32 + k) work items */
-  uint2* equeue;                       /* (slot, partner) of the pairs for the wave-per-pair kernel */
-  uint32_t* qcount;                    /* [0] queue length, [1] edge queue length, [2] its chunk counter */
-  float4 *pf, *pt;                     /* n * 32: pair force (w = 1 when in contact), torque */
+  uint2* equeue;                       /* (slot, partner) of the pairs for the wave-per-pair kernel, POLY_SUBQ parts */
+  uint32_t* qcount;                    /* POLY_QCOUNTS counters, POLY_QSTRIDE words apart: the parts' lengths, then
+                                          the wave-per-pair kernel's slice counters */
+  uint8_t* hitf;                       /* n * 32: 1 where the slot's pair is in contact */
+  float4 *pf, *pt;                     /* n * 32: pair force, torque, where hitf is set */
   uint2* hint;                         /* n * 32 by P_ID and list slot: (partner P_ID, separating face code) */
 };
-constexpr int POLY_PAIR_BLOCKS = 2048;   /* a multiple of the 8 XCDs */
+constexpr int POLY_SUBQ = 64, POLY_SLICES = 8;
+constexpr int POLY_QCOUNTS = POLY_SUBQ + POLY_SLICES, POLY_QSTRIDE = 32;   /* a counter per 128-byte line */
+/* Particles per block of the separating-plane kernel.  Up to
+ * POLY_PAIRS_SMALL particles the smaller blocks spread them over the CUs. */
+constexpr int POLY_PPB = 128, POLY_PPB_SMALL = 16, POLY_PAIRS_SMALL = 16384;
+/* Entries one part of the pair queue can receive: its blocks' listed slots
+ * (a block's are consecutive, block w fills part w mod POLY_SUBQ). */
+inline uint32_t poly_subqueue_capacity(int n) {
+  const int ppb = n <= POLY_PAIRS_SMALL ? POLY_PPB_SMALL : POLY_PPB;
+  const int blocks = (n + ppb - 1) / ppb;
+  return (uint32_t)((blocks + POLY_SUBQ - 1) / POLY_SUBQ) * (uint32_t)(ppb * LIST_STRIDE);
+}
 
 constexpr int SORT_THREADS = 256;
 constexpr int SORT_ITEMS = 16;

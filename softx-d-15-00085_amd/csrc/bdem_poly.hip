@@ -375,15 +375,25 @@ __device__ __forceinline__ PColl vertex_faces_select(f3 PosA, const Shape& A, co
   return res;   /* face logic fall-through: depth 0, zero normal */
 }
 
-/* Vertices of A in B, and if none, vertices of B in A (normal reversed). */
-__device__ __forceinline__ PColl vertex_faces_pair(f3 PosA, const Shape& A, f3 PosB, const Shape& B,
-                                                   const PairDirs& D) {
-  PColl c = vertex_faces_select(PosA, A, B, vertices_inside(A, B, D.fB));
-  if (!c.hit) {
-    c = vertex_faces_select(PosB, B, A, vertices_inside(B, A, D.fA));
-    c.n = c.n * -1.0f;   /* B into A: normal reversed */
+/* Vertices of A in B, and if none, vertices of B in A (normal reversed), for
+ * the contact of A (ab) and, with the roles swapped, that of B (ba): both
+ * need the same two inside tests and selections.  False when no vertex of
+ * either body is inside the other. */
+__device__ __forceinline__ bool vertex_faces_both(f3 PosA, const Shape& A, f3 PosB, const Shape& B, const PairDirs& D,
+                                                  PColl& ab, PColl& ba) {
+  const uint32_t mab = vertices_inside(A, B, D.fB), mba = vertices_inside(B, A, D.fA);
+  if ((mab | mba) == 0u) return false;
+  if (mab) ab = vertex_faces_select(PosA, A, B, mab);
+  if (mba) ba = vertex_faces_select(PosB, B, A, mba);
+  if (!mab) {
+    ab = ba;
+    ab.n = ab.n * -1.0f;
   }
-  return c;
+  if (!mba) {
+    ba = ab;
+    ba.n = ba.n * -1.0f;
+  }
+  return true;
 }
 
 /* One edge pair of Collision_Detection_Polyhedra_Polyhedra_Edges
@@ -453,7 +463,7 @@ __device__ __forceinline__ float edge_bound(f3 p0, f3 p1, f3 c, float vb, f3 n, 
  * minimum selects the serial loop's pair, whose points every lane then
  * recomputes with the same arithmetic.  The result is wave-uniform. */
 __device__ __forceinline__ PColl edges_wave(const Shape& A, const uint2* EA, int ea, const Shape& B, const uint2* EB,
-                                            int eb, f3 RelPos, f3 PosA, f3 PosB, float vbA, float vbB, float slA,
+                                            int eb, f3 PosA, f3 PosB, float vbA, float vbB, float slA,
                                             float slB, unsigned char* ia, unsigned char* ib, int fA, int fB) {
   const int lane = threadIdx.x & 63;
   float la = 3.0e38f, lb = 3.0e38f;
@@ -464,7 +474,7 @@ __device__ __forceinline__ PColl edges_wave(const Shape& A, const uint2* EA, int
   const float size = fabsf(PosA.x) + fabsf(PosA.y) + fabsf(PosA.z) + fabsf(PosB.x) + fabsf(PosB.y) + fabsf(PosB.z);
   const float margin = 0.001f + 4.0e-6f * size;
   float best = 5.0f;
-  int bt = 0x7FFFFFFF;
+  int bt = 0x7FFFFFFF, bu = 0x7FFFFFFF;
   const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
   /* the pairs of SA x SB, from compacted index lists; lane u takes pairs
    * u, u + 64, ... in row-major order (64 = qa nb + rb) */
@@ -485,8 +495,15 @@ __device__ __forceinline__ PColl edges_wave(const Shape& A, const uint2* EA, int
       if (b >= nb) { b -= nb; ++a; }
       float dis;
       if (edge_pair_dis(A, EA[i], B, EB[j], dis) && dis < 5.0f) {
-        const int t = i * eb + j;
-        if (dis < best || (dis == best && t < bt)) { best = dis; bt = t; }
+        const int t = i * eb + j, u2 = j * ea + i;
+        if (dis < best) {
+          best = dis;
+          bt = t;
+          bu = u2;
+        } else if (dis == best) {
+          bt = min(bt, t);
+          bu = min(bu, u2);
+        }
       }
     }
   };
@@ -500,18 +517,26 @@ __device__ __forceinline__ PColl edges_wave(const Shape& A, const uint2* EA, int
   const uint64_t SA2 = __ballot(lane < ea && la <= w2), SB2 = __ballot(lane < eb && lb <= w2);
   if ((SA2 & ~SA1) && SB2) sweep(SA2 & ~SA1, SB2);
   if ((SA2 & SA1) && (SB2 & ~SB1)) sweep(SA2 & SA1, SB2 & ~SB1);
-  /* wave minimum of (distance, t) */
+  /* wave minimum of (distance, t), then of (distance, t') */
   const float m = wave_min(best);
   const int tm = wave_min_i32((best == m) ? bt : 0x7FFFFFFF);
+  const int um = wave_min_i32((best == m) ? bu : 0x7FFFFFFF);
   PColl res{false, C_SP, 0.0f, mk3(0.f, 0.f, 0.f), mk3(0.0f, 0.0f, 0.0f)};
   if (!(m < 5.0f) || tm == 0x7FFFFFFF) return res;
-  /* the selected pair, recomputed by every lane */
-  const int si = tm / eb, sj = tm - (tm / eb) * eb;
-  const f3 PA = ld3(A.V + EA[si].x);
-  const f3 DA = ld3(A.V + EA[si].y) - PA;
+  /* the selected pair, by each half for its own body X against Y */
+  const bool hb = lane >= 32;
+  const Shape& X = hb ? B : A;
+  const Shape& Y = hb ? A : B;
+  const uint2* const EX = hb ? EB : EA;
+  const uint2* const EY = hb ? EA : EB;
+  const f3 PosX = hb ? PosB : PosA, PosY = hb ? PosA : PosB;
+  const int ts = hb ? um : tm, ey = hb ? ea : eb;
+  const int si = ts / ey, sj = ts - si * ey;
+  const f3 PA = ld3(X.V + EX[si].x);
+  const f3 DA = ld3(X.V + EX[si].y) - PA;
   const float DEAD = dot(DA, DA);
-  const f3 PB = ld3(B.V + EB[sj].x);
-  const f3 DB = ld3(B.V + EB[sj].y) - PB;
+  const f3 PB = ld3(Y.V + EY[sj].x);
+  const f3 DB = ld3(Y.V + EY[sj].y) - PB;
   const f3 DV = PA - PB;
   const float DEBD = dot(DB, DB);
   const float DEABD = dot(DA, DB);
@@ -522,23 +547,26 @@ __device__ __forceinline__ PColl edges_wave(const Shape& A, const uint2* EA, int
   const float dB = detJinv * (DEABD * DEADAB - DEAD * DEBDAB);
   const f3 selA = PA + DA * dA;
   const f3 selB = PB + DB * dB;
+  /* isPointinPoly (Utilities.cuh:63-98), a lane of the half per face of Y */
+  const int f = lane & 31;
+  const bool fv = f < Y.nf;
+  const bool inside_test = length(PosY - selB) < length(PosY - selA);
+  const uint64_t out = __ballot(inside_test && fv &&
+                                !(dot(ld3(Y.Fn + (fv ? f : 0)), selA - ld3(Y.Fc + (fv ? f : 0))) <= 0.000100f));
+  if ((uint32_t)(hb ? out >> 32 : out) != 0u) return res;
   res.cp = selA;
   res.n = cross(DA, DB);
   res.n = res.n * (1.0f / length(res.n));
-  if (length(PosB - selB) < length(PosB - selA)) {
-    /* isPointinPoly (Utilities.cuh:63-98), a lane per face of B */
-    const int f = lane < B.nf ? lane : 0;
-    if (__ballot(lane < B.nf && !(dot(ld3(B.Fn + f), selA - ld3(B.Fc + f)) <= 0.000100f))) return res;
-  }
   res.hit = true;
   res.cls = C_EE;
+  const f3 RelPos = (PosX - PosY) / length(PosX - PosY);
   const float dn = dot(RelPos, res.n);
   if (fabsf(dn) > 0.0f) {
     res.n = (dot(RelPos, res.n) / fabsf(dot(RelPos, res.n))) * res.n;
     res.dis = fabsf(dot(res.n, (selB - selA))) + 0.000010f;
   } else {
     res.n = RelPos / length(RelPos);
-    res.cp = PosB;
+    res.cp = PosY;
     res.dis = fabsf(dot(res.n, (selB - selA))) + 0.000010f;
   }
   return res;
@@ -687,27 +715,7 @@ struct PairOps {
   f3 PosA, PosB, va, vb, wa, wb;
   float ma, mb;
 };
-__device__ __forceinline__ PairOps pair_ops(const DevParams& P, uint32_t slot, const uint32_t* __restrict__ list32,
-                                            const float4* __restrict__ pos, const float4* __restrict__ vel,
-                                            const float4* __restrict__ omg) {
-  PairOps o;
-  o.a = (int)(slot / LIST_STRIDE);
-  o.b = (int)list32[slot];
-  const float4 oa = omg[o.a], ob = omg[o.b];
-  o.ta = packed_type(oa.w);
-  o.tb = packed_type(ob.w);
-  o.sa = shape_index(P, oa.w);
-  o.sb = shape_index(P, ob.w);
-  const float4 va4 = vel[o.a], vb4 = vel[o.b];
-  o.PosA = xyz(pos[o.a]);
-  o.PosB = xyz(pos[o.b]);
-  o.va = xyz(va4); o.vb = xyz(vb4);
-  o.ma = va4.w; o.mb = vb4.w;
-  o.wa = xyz(oa); o.wb = xyz(ob);
-  return o;
-}
-
-/* The operands of a queued pair whose partner is known. */
+/* The operands of slot's particle and its partner b. */
 __device__ __forceinline__ PairOps pair_ops_ab(const DevParams& P, uint32_t slot, uint32_t b,
                                                const float4* __restrict__ pos, const float4* __restrict__ vel,
                                                const float4* __restrict__ omg) {
@@ -728,21 +736,17 @@ __device__ __forceinline__ PairOps pair_ops_ab(const DevParams& P, uint32_t slot
   return o;
 }
 
-/* Clamps, then the reference pair law into the pair's slot. */
+/* Clamps, then the reference pair law into the contact's slot, marked in
+ * hitf (the list kernel clears it). */
 __device__ __forceinline__ void pair_store(const DevParams& P, const bdem_poly_shape& pa, const PairOps& o, PColl c,
                                            uint32_t slot, float4* __restrict__ pf, float4* __restrict__ pt,
-                                           float* tally = nullptr) {
-  float4 F4 = make_float4(0.f, 0.f, 0.f, 0.f), T4 = F4;
-  if (c.hit) {
-    depth_clamps(c, pa.radius, o.PosA, o.PosB, o.va - o.vb);
-    f3 F, T;
-    pair_resp(P, o.va, o.ma, o.wa, o.ta, o.vb, o.mb, o.wb, o.tb, c.n, c.dis, c.cp - o.PosA, c.cp - o.PosB, F, T,
-              tally);
-    F4 = make_float4(F.x, F.y, F.z, 1.0f);
-    T4 = make_float4(T.x, T.y, T.z, 0.0f);
-  }
-  pf[slot] = F4;
-  pt[slot] = T4;
+                                           uint8_t* __restrict__ hitf, float* tally = nullptr) {
+  depth_clamps(c, pa.radius, o.PosA, o.PosB, o.va - o.vb);
+  f3 F, T;
+  pair_resp(P, o.va, o.ma, o.wa, o.ta, o.vb, o.mb, o.wb, o.tb, c.n, c.dis, c.cp - o.PosA, c.cp - o.PosB, F, T, tally);
+  pf[slot] = make_float4(F.x, F.y, F.z, 1.0f);
+  pt[slot] = make_float4(T.x, T.y, T.z, 0.0f);
+  hitf[slot] = 1;
 }
 
 /* ---------------------------------------------------------------- walls */
@@ -1201,7 +1205,7 @@ __global__ __launch_bounds__(256) void k_poly_rotate(const DevParams* __restrict
                                                      float4* __restrict__ rot, uint32_t* __restrict__ qcount) {
   const DevParams& P = *Pp;
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t == 0) { qcount[0] = 0u; qcount[1] = 0u; qcount[2] = 0u; }   /* this step's queues start empty */
+  if (t < POLY_QCOUNTS) qcount[t * POLY_QSTRIDE] = 0u;   /* this step's queues start empty */
   const size_t i = t / (size_t)L.stride;
   const int e = (int)(t - i * (size_t)L.stride);
   if (i >= (size_t)n) return;
@@ -1220,49 +1224,25 @@ __global__ __launch_bounds__(256) void k_poly_rotate(const DevParams* __restrict
   rot[t] = make_float4(out.x, out.y, out.z, 0.0f);
 }
 
-/* A particle's list (m of its c contacts, in LDS) to memory by its G lanes,
- * and its pairs to the work queue, one reservation per block of `WAVES`
- * waves.  Every thread of the block calls. */
-template <int G, int WAVES>
-__device__ __forceinline__ void list_store(int n, int i, bool in, int c, const uint32_t* mine,
-                                           uint32_t* __restrict__ list32, uint32_t* __restrict__ nn,
-                                           uint32_t* __restrict__ queue, uint32_t* __restrict__ qcount,
-                                           uint32_t* status) {
-  __shared__ uint32_t wtotal[WAVES], qbase;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane & (G - 1);
-  if (in && sub == 0) {
+/* A particle's list (its c contacts, in LDS) to memory by its G lanes, and
+ * its slots' contact marks cleared. */
+template <int G>
+__device__ __forceinline__ void list_store(int i, bool in, int c, const uint32_t* mine, uint32_t* __restrict__ list32,
+                                           uint32_t* __restrict__ nn, uint8_t* __restrict__ hitf, uint32_t* status) {
+  if (!in) return;
+  const int sub = threadIdx.x & (G - 1);
+  if (sub == 0) {
     nn[i] = (uint32_t)c;
     if (c > LIST_STRIDE) atomicOr(status, ST_LIST_OVERFLOW);
   }
-  const int m = in ? min(c, LIST_STRIDE) : 0;
-  /* queue places: the wave's particles in order, each lane's entries k = sub, sub + G, ... */
-  const int own = m > sub ? (m - sub + G - 1) / G : 0;
-  int incl = own;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += v;
-  }
-  if (lane == 63) wtotal[wave] = (uint32_t)incl;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t t = 0u;
-    for (int w = 0; w < WAVES; ++w) t += wtotal[w];
-    qbase = t ? atomicAdd(qcount, t) : 0u;
-  }
-  __syncthreads();
-  uint32_t at = qbase + (uint32_t)(incl - own);
-  for (int w = 0; w < wave; ++w) at += wtotal[w];
-  const uint32_t cap = (uint32_t)n * LIST_STRIDE;
-  for (int k = sub; k < m; k += G, ++at) {
-    const uint32_t slot = (uint32_t)i * LIST_STRIDE + (uint32_t)k;
-    list32[slot] = mine[k];
-    if (at < cap) queue[at] = slot;
-  }
+  const int m = min(c, LIST_STRIDE);
+  for (int k = sub; k < m; k += G) list32[(size_t)i * LIST_STRIDE + k] = mine[k];
+  uint32_t* const marks = reinterpret_cast<uint32_t*>(hitf + (size_t)i * LIST_STRIDE);
+  for (int k = sub; k < LIST_STRIDE / 4; k += G) marks[k] = 0u;
 }
 
 /* Bounding-sphere contact list (the sphere broad phase: Kernel_BroadCollision-
- * Detection_NonSymmetry, 32 slots, full count) and the pair work queue.
+ * Detection_NonSymmetry, 32 slots, full count).
  *
  * A grid cell (2 x the largest bounding radius) holds about seven hulls, so
  * a hull tests some 190 candidates to list 12.  Sixteen lanes share them,
@@ -1278,8 +1258,7 @@ __global__ __launch_bounds__(256) void k_poly_list(const DevParams* __restrict__
                                                    const float4* __restrict__ pos_r,
                                                    const float4* __restrict__ omg,
                                                    uint32_t* __restrict__ list32, uint32_t* __restrict__ nn,
-                                                   uint32_t* __restrict__ queue, uint32_t* __restrict__ qcount,
-                                                   uint32_t* status) {
+                                                   uint8_t* __restrict__ hitf, uint32_t* status) {
   const DevParams& P = *Pp;
   __shared__ uint32_t cand[4][LIST_NP][LIST_CAND];
   __shared__ uint32_t list[4][LIST_NP][LIST_STRIDE];
@@ -1295,7 +1274,7 @@ __global__ __launch_bounds__(256) void k_poly_list(const DevParams* __restrict__
                                                    if (k < LIST_STRIDE) mine[k] = (uint32_t)j;
                                                  });
   __builtin_amdgcn_wave_barrier();
-  list_store<LIST_G, 4>(n, i, in, c, mine, list32, nn, queue, qcount, status);
+  list_store<LIST_G>(i, in, c, mine, list32, nn, hitf, status);
 }
 
 /* The same list for larger counts, two lanes per particle and 32 particles
@@ -1305,22 +1284,21 @@ __global__ __launch_bounds__(256) void k_poly_list(const DevParams* __restrict__
  * row's candidates into a bit mask, and the masks' set bits, the first
  * half's before the second's, are the contacts in order. */
 constexpr int LIST_TEAM_MAX = 24576;
-constexpr int LIST2_POS = 96;
+constexpr int LIST2_POS = 80;
 struct ListStage {
   float4 pos[3][LIST2_POS];
   uint2 cell[3][64];
   uint32_t list[32][LIST_STRIDE + 1];   /* odd stride: both lanes of 32 particles write it */
 };
 constexpr int LIST2_WAVES = 4, LIST2_BLOCK = 32 * LIST2_WAVES;
-__global__ __launch_bounds__(64 * LIST2_WAVES) void k_poly_list2(const DevParams* __restrict__ Pp, int n,
+__global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void k_poly_list2(const DevParams* __restrict__ Pp, int n,
                                                                  const uint2* __restrict__ cells,
                                                                  const float4* __restrict__ pos_r,
                                                                  const float4* __restrict__ omg,
                                                                  const uint32_t* __restrict__ sorted_keys,
                                                                  uint32_t* __restrict__ list32,
                                                                  uint32_t* __restrict__ nn,
-                                                                 uint32_t* __restrict__ queue,
-                                                                 uint32_t* __restrict__ qcount, uint32_t* status) {
+                                                                 uint8_t* __restrict__ hitf, uint32_t* status) {
   const DevParams& P = *Pp;
   __shared__ ListStage stage[LIST2_WAVES];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1439,85 +1417,132 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) void k_poly_list2(const DevParams
     }
   }
   __builtin_amdgcn_wave_barrier();
-  list_store<2, LIST2_WAVES>(n, i, in, count, mine, list32, nn, queue, qcount, status);
+  list_store<2>(i, in, count, mine, list32, nn, hitf, status);
 }
 
-/* One queued pair per thread, grid-stride so that every wave exits once the
- * queue (at most n * 32 entries) is drained: the separating-plane test of
- * each body's face turned most towards the other.  The pairs it does not
- * separate (about 1 in 5 in a dense pack of hulls) go to a second queue,
- * where a wave per pair runs the full separating-plane test, then the
- * vertex-face and edge-edge searches. */
+/* Whether particle i is among the listed contacts of j. */
+__device__ __forceinline__ bool is_listed(const uint32_t* __restrict__ list32, int j, uint32_t i) {
+  bool found = false;
+  for (int k = 0; k < LIST_STRIDE; ++k) found = found || list32[(size_t)j * LIST_STRIDE + k] == i;
+  return found;
+}
+
+/* The separating-plane test of the pairs listed by PPB consecutive
+ * particles.  Whether a face separates two bodies is the same question from
+ * both sides, so a pair is tested once, by the particle with the lower
+ * sorted slot (the other only when the first one's list overflowed without
+ * it).  First every pair takes the face that separated it at the last step;
+ * those it does not separate are gathered in LDS and take the two facing
+ * faces with full waves; the rest go to a queue for k_poly_narrow.
+ *
+ * A reservation in one shared counter costs about 10 ns, one after another
+ * (1,172 more of them added 12 us to a launch): 35,700 per launch held an
+ * earlier form of this kernel at 457 us for 200,000 hulls.  Here a block
+ * makes one, in one of POLY_SUBQ counters, each with its own part of the
+ * queue. */
+template <int PPB>
 __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict__ Pp,
-                                                    const bdem_poly_shape* __restrict__ shapes,
                                                     const ShapeHdr* __restrict__ hdr, int n, PolyLayout L,
                                                     const float4* __restrict__ rot,
-                                                    const float4* __restrict__ pos, const float4* __restrict__ vel,
-                                                    const float4* __restrict__ omg,
+                                                    const float4* __restrict__ pos, const float4* __restrict__ omg,
                                                     const uint32_t* __restrict__ list32,
-                                                    const uint32_t* __restrict__ queue,
-                                                    uint32_t* __restrict__ qcount, uint2* __restrict__ equeue,
-                                                    float4* __restrict__ pf, float4* __restrict__ pt,
+                                                    const uint32_t* __restrict__ nn, uint32_t* __restrict__ qcount,
+                                                    uint2* __restrict__ equeue, uint32_t subcap,
                                                     uint2* __restrict__ hint) {
+  static_assert(PPB * LIST_STRIDE <= 65536, "slots of a block fit 16 bits");
   const DevParams& P = *Pp;
-  const uint32_t total = qcount[0];
-  const uint32_t cap = (uint32_t)n * LIST_STRIDE;
-  const uint32_t cnt = total < cap ? total : cap;
+  __shared__ uint16_t items[PPB * LIST_STRIDE], left[PPB * LIST_STRIDE];
+  __shared__ uint32_t nitems, nleft, nout, qbase;
   const int lane = threadIdx.x & 63;
-  /* Each XCD (workgroup w runs on XCD w mod 8) takes one contiguous eighth
-   * of the queue, and its blocks stride through it together, so the turned
-   * shapes of neighbouring particles are read through that XCD's L2.  Every
-   * lane of a wave runs the same number of iterations (the bounds are whole
-   * waves) so that the append below sees the whole wave. */
-  const uint32_t xcd = blockIdx.x % NUM_XCD, per = gridDim.x / NUM_XCD;
-  const uint32_t cnt_w = (cnt + 63u) & ~63u;
-  const uint32_t chunk = ((cnt_w / 64u + NUM_XCD - 1u) / NUM_XCD) * 64u;
-  const uint32_t lo = xcd * chunk, hi = lo + chunk < cnt_w ? lo + chunk : cnt_w;
-  const uint32_t stride = per * blockDim.x;
-  for (uint32_t q = lo + (blockIdx.x / NUM_XCD) * blockDim.x + threadIdx.x; q < hi; q += stride) {
-    bool need = false;
-    uint32_t slot = 0u, partner = 0u;
+  const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+  const int base = xcd_block(blockIdx.x, gridDim.x) * PPB;
+  auto push = [&](uint16_t* list, uint32_t* count, bool want, uint32_t e) {
+    const uint64_t m = __ballot(want);
+    if (m == 0ull) return;
+    uint32_t at = 0u;
+    if (lane == 0) at = atomicAdd(count, (uint32_t)__popcll(m));
+    at = __builtin_amdgcn_readfirstlane(at);
+    if (want) list[at + (uint32_t)__popcll(m & lt)] = (uint16_t)e;
+  };
+  /* a pair of the block: its slot, bodies and hint */
+  struct Pair { uint32_t slot; int a, b, ida; uint32_t idb; ShapeHdr ha, hb; f3 PosA, PosB; Shape A, B; float vbA, vbB; };
+  auto load = [&](uint32_t e) {
+    Pair p;
+    p.slot = (uint32_t)base * LIST_STRIDE + e;
+    p.a = base + (int)(e / LIST_STRIDE);
+    p.b = (int)list32[p.slot];
+    const float oa = omg[p.a].w, ob = omg[p.b].w;
+    p.PosA = xyz(pos[p.a]);
+    p.PosB = xyz(pos[p.b]);
+    p.ida = packed_pid(oa);
+    p.idb = (uint32_t)packed_pid(ob);
+    p.ha = hdr[shape_index(P, oa)];
+    p.hb = hdr[shape_index(P, ob)];
+    p.A = shape_of(rot, L, p.a, p.ha);
+    p.B = shape_of(rot, L, p.b, p.hb);
+    p.vbA = p.ha.vbound * P.vbound_scale;
+    p.vbB = p.hb.vbound * P.vbound_scale;
+    return p;
+  };
+  if (threadIdx.x == 0) { nitems = 0u; nleft = 0u; nout = 0u; }
+  __syncthreads();
+  for (uint32_t e = threadIdx.x; e < (uint32_t)(PPB * LIST_STRIDE); e += 256u) {
+    const int i = base + (int)(e / LIST_STRIDE), k = (int)(e % LIST_STRIDE);
+    bool want = false;
+    if (i < n && (uint32_t)k < min(nn[i], (uint32_t)LIST_STRIDE)) {
+      const int j = (int)list32[(size_t)i * LIST_STRIDE + k];
+      want = j > i || (nn[j] > (uint32_t)LIST_STRIDE && !is_listed(list32, j, (uint32_t)i));
+    }
+    push(items, &nitems, want, e);
+  }
+  __syncthreads();
+  const uint32_t cnt = nitems;
+  for (uint32_t q0 = 0u; q0 < cnt; q0 += 256u) {
+    const uint32_t q = q0 + threadIdx.x;
+    bool rest = false;
+    uint32_t e = 0u;
     if (q < cnt) {
-      slot = queue[q];
-      const PairOps o = pair_ops(P, slot, list32, pos, vel, omg);
-      partner = (uint32_t)o.b;
-      const ShapeHdr ha = hdr[o.sa], hb = hdr[o.sb];
-      const Shape A = shape_of(rot, L, o.a, ha);
-      const Shape B = shape_of(rot, L, o.b, hb);
-      const float vbA = ha.vbound * P.vbound_scale, vbB = hb.vbound * P.vbound_scale;
-      /* the pair's hint, kept by P_ID and list slot (rows past n: no hint) */
-      const int ida = packed_pid(omg[o.a].w);
-      const uint32_t idb = (uint32_t)packed_pid(omg[o.b].w);
-      uint2* hp = (ida >= 0 && ida < n) ? hint + (size_t)ida * LIST_STRIDE + (slot % LIST_STRIDE) : nullptr;
+      e = items[q];
+      const Pair p = load(e);
+      /* hints are kept by P_ID and list slot (rows past n: none) */
+      const bool row = p.ida >= 0 && p.ida < n;
+      const uint2 h = row ? hint[(size_t)p.ida * LIST_STRIDE + (p.slot % LIST_STRIDE)] : make_uint2(0u, HINT_NONE);
+      rest = !hint_separates(h, p.idb, p.A, p.B, p.PosA, p.PosB, p.vbA, p.vbB);
+    }
+    push(left, &nleft, rest, e);
+  }
+  __syncthreads();
+  const uint32_t cl = nleft;
+  for (uint32_t q0 = 0u; q0 < cl; q0 += 256u) {
+    const uint32_t q = q0 + threadIdx.x;
+    bool rest = false;
+    uint32_t e = 0u;
+    if (q < cl) {
+      e = left[q];
+      const Pair p = load(e);
       uint32_t code = HINT_NONE;
-      bool sep = false;
-      if (hp) {
-        const uint2 h = *hp;
-        if (hint_separates(h, idb, A, B, o.PosA, o.PosB, vbA, vbB)) { sep = true; code = h.y; }
-      }
-      if (!sep) sep = quick_separated(A, B, o.PosA, o.PosB, vbA, vbB, code);
-      if (hp) *hp = make_uint2(idb, sep ? code : HINT_NONE);
-      need = !sep;
-      if (!need)
-        pair_store(P, shapes[o.sa], o, PColl{false, C_SP, 0.0f, mk3(0.f, 0.f, 0.f), mk3(0.f, 0.f, 0.f)}, slot, pf, pt);
+      rest = !quick_separated(p.A, p.B, p.PosA, p.PosB, p.vbA, p.vbB, code);
+      if (p.ida >= 0 && p.ida < n)
+        hint[(size_t)p.ida * LIST_STRIDE + (p.slot % LIST_STRIDE)] = make_uint2(p.idb, rest ? HINT_NONE : code);
     }
-    const uint64_t mask = __ballot(need);
-    if (mask) {
-      const int leader = __ffsll((unsigned long long)mask) - 1;
-      uint32_t base = 0u;
-      if (lane == leader) base = atomicAdd(&qcount[1], (uint32_t)__popcll(mask));
-      base = __shfl(base, leader, 64);
-      const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-      const uint32_t at = base + (uint32_t)__popcll(mask & lt);
-      if (need && at < cap) equeue[at] = make_uint2(slot, partner);
-    }
+    push(items, &nout, rest, e);   /* the first list has been read */
+  }
+  __syncthreads();
+  const uint32_t co = nout, sq = blockIdx.x % POLY_SUBQ;
+  if (co == 0u) return;
+  if (threadIdx.x == 0) qbase = atomicAdd(&qcount[sq * POLY_QSTRIDE], co);
+  __syncthreads();
+  for (uint32_t q = threadIdx.x; q < co; q += 256u) {
+    const uint32_t slot = (uint32_t)base * LIST_STRIDE + items[q], at = qbase + q;
+    if (at < subcap) equeue[(size_t)sq * subcap + at] = make_uint2(slot, list32[slot]);
   }
 }
 
 /* One pair's bodies staged in LDS by its wave: turned vertices, face
  * normals and centroids, and edge lists of A (row 0) and B (row 1). */
 /* A pair's contact, kept until the chunk's pair law runs. */
-struct PairHit { uint32_t hit; float dis, nx, ny, nz, cx, cy, cz; };
+struct PairHit { uint32_t slot; float dis, nx, ny, nz, cx, cy, cz; };   /* slot NO_SLOT: no contact */
+constexpr uint32_t NO_SLOT = 0xFFFFFFFFu;
 constexpr uint32_t NARROW_CHUNK = 32;   /* largest chunk of the narrow kernel's queue */
 
 struct PairStage {
@@ -1531,18 +1556,23 @@ struct PairStage {
   unsigned char ia[BDEM_SHAPE_MAX_EDGE], ib[BDEM_SHAPE_MAX_EDGE];   /* edge lists of the pruned search */
 };
 
-/* The pairs the first pass could not separate, one wave per pair,
- * grid-stride over the queue by waves: vertices of A in B, vertices of B in
- * A (normal reversed), then edge-edge with its depth limited to 0.025 rA
- * (DEM_Kernels_Compute.cuh:852-904).  The wave first copies both bodies
- * into its LDS stage, so the searches read LDS instead of chains of
- * dependent global loads.
+/* The pairs k_poly_pairs could not separate, one wave per pair, for both
+ * bodies' contacts at once: vertices of A in B, vertices of B in A, then
+ * edge-edge with its depth limited to 0.025 r (DEM_Kernels_Compute.cuh:
+ * 852-904).  The wave first copies both bodies into its LDS stage, so the
+ * searches read LDS instead of chains of dependent global loads.  The inside
+ * tests and the edge search are the same for the contact of A with B and of
+ * B with A (vertex_faces_both, edges_wave); done once per pair instead of
+ * once per listed contact they halve the launch's work.
  *
- * A wave takes its pairs from the queue in chunks by an atomic counter
- * (qcount[2]), guided: a chunk is about 1 / (2 x waves) of what is left, 4
- * to 32 pairs, so waves that drew expensive pairs (the edge-edge search)
- * do not hold up the launch.  The searches leave each pair's contact in
- * LDS, and the pair law then runs for the whole chunk, a lane per pair.
+ * A wave's first chunk is its own by its number: the first half of the
+ * queue (all of it while it has a pair per wave at most).  The rest is dealt
+ * in eight slices, each with its counter, in guided chunks of about
+ * 1 / (2 x waves) of what is left of the slice, 2 to 32 pairs, so waves that
+ * drew expensive pairs (the edge-edge search) do not hold up the launch; one
+ * counter for all would serve a chunk per 10 ns.  The searches leave each
+ * contact in LDS, and the pair law then runs for the whole chunk, a lane per
+ * contact.
  *
  * Staging is one round trip to memory per pair.  Each lane fetches one of
  * the chunk's queue entries and the shape rows of its two bodies ahead of
@@ -1553,42 +1583,55 @@ struct PairStage {
  * the record and never read) before the first LDS write.
  *
  * Five waves per SIMD: at most 96 VGPRs without spills, and five blocks of
- * 25 KiB of LDS (four stages and their chunk's pair records) per CU. */
+ * 29 KiB of LDS (four stages and their chunk's contacts) per CU. */
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_poly_narrow(const DevParams* __restrict__ Pp,
                                                      const bdem_poly_shape* __restrict__ shapes,
                                                      const ShapeHdr* __restrict__ hdr, int n, PolyLayout L,
                                                      const float4* __restrict__ rot,
                                                      const float4* __restrict__ pos, const float4* __restrict__ vel,
                                                      const float4* __restrict__ omg,
+                                                     const uint32_t* __restrict__ list32,
+                                                     const uint32_t* __restrict__ nn,
                                                      uint32_t* __restrict__ qcount,
-                                                     const uint2* __restrict__ equeue,
-                                                     float4* __restrict__ pf, float4* __restrict__ pt, int energy,
+                                                     const uint2* __restrict__ equeue, uint32_t subcap,
+                                                     float4* __restrict__ pf, float4* __restrict__ pt,
+                                                     uint8_t* __restrict__ hitf, int energy,
                                                      uint2* __restrict__ hint) {
   const DevParams& P = *Pp;
   float* const tally = energy ? P.tally : nullptr;   /* dissipation tallies (EnergyCalc) */
   __shared__ PairStage stage[4];
-  __shared__ PairHit hits[4][NARROW_CHUNK];
+  __shared__ PairHit hits[4][2][NARROW_CHUNK];
+  __shared__ uint32_t qpre[POLY_SUBQ + 1];   /* pairs before each part of the queue */
   PairStage& S = stage[threadIdx.x >> 6];
-  PairHit* const R = hits[threadIdx.x >> 6];
+  PairHit (*const R)[NARROW_CHUNK] = hits[threadIdx.x >> 6];
   const int lane = threadIdx.x & 63;
   const int h = lane >> 5, k = lane & 31;
   const int kv = k < L.pv ? k : L.pv - 1, kf = k < L.pf ? k : L.pf - 1;
+  static_assert(POLY_SUBQ == 64, "a lane per part of the queue");
+  if (threadIdx.x < 64) {
+    const uint32_t c = min(qcount[threadIdx.x * POLY_QSTRIDE], subcap);
+    uint32_t incl = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t v = (uint32_t)__shfl_up((int)incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    qpre[threadIdx.x + 1] = incl;
+    if (threadIdx.x == 0) qpre[0] = 0u;
+  }
+  __syncthreads();
+  const uint32_t cnt = qpre[POLY_SUBQ];
   const uint32_t cap = (uint32_t)n * LIST_STRIDE;
-  const uint32_t cnt = qcount[1] < cap ? qcount[1] : cap;
-  const uint32_t waves = gridDim.x * (blockDim.x / 64u);
-  uint32_t seen = 0u;   /* the counter's value at this wave's last grab */
-  for (;;) {
-    uint32_t size = (cnt > seen ? cnt - seen : 0u) / (2u * waves);
-    size = size < 4u ? 4u : (size > NARROW_CHUNK ? NARROW_CHUNK : size);
-    uint32_t base = 0u;
-    if (lane == 0) base = atomicAdd(&qcount[2], size);
-    base = __builtin_amdgcn_readfirstlane(base);
-    if (base >= cnt) break;
-    seen = base + size;
-    const uint32_t m = cnt - base < size ? cnt - base : size;
+
+  auto process = [&](uint32_t base, uint32_t m) {   /* pairs [base, base + m), m <= NARROW_CHUNK */
     uint32_t lslot = cap, lpart = 0u, lsa = 0u, lsb = 0u;
     if ((uint32_t)lane < m) {
-      const uint2 item = equeue[base + (uint32_t)lane];   /* (slot, partner) */
+      const uint32_t g = base + (uint32_t)lane;
+      uint32_t lo = 0u;   /* the last part starting at or before pair g */
+#pragma unroll
+      for (uint32_t o = POLY_SUBQ / 2; o > 0u; o >>= 1)
+        if (qpre[lo + o] <= g) lo += o;
+      const uint2 item = equeue[(size_t)lo * subcap + (g - qpre[lo])];   /* (slot, partner) */
       if (item.x < cap && item.y < (uint32_t)n) {
         lslot = item.x;
         lpart = item.y;
@@ -1598,7 +1641,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     }
     for (int j = 0; j < (int)m; ++j) {
       const uint32_t slot = __builtin_amdgcn_readlane(lslot, j);
-      if (slot >= cap) continue;
+      if (slot >= cap) {
+        if (k == 0) R[h][j].slot = NO_SLOT;
+        continue;
+      }
       const uint32_t partner = __builtin_amdgcn_readlane(lpart, j);
       const int sa = __builtin_amdgcn_readlane(lsa, j), sb = __builtin_amdgcn_readlane(lsb, j);
       const bdem_poly_shape& pa = shapes[sa];
@@ -1617,6 +1663,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
       }
       const float farea = F.area;
       const int fnv = F.num_vertex;
+      const uint32_t back = list32[(size_t)partner * LIST_STRIDE + k];
+      const uint32_t nback = nn[partner];
       const PairOps o = pair_ops_ab(P, slot, partner, pos, vel, omg);
       const float vbA = ha.vbound * P.vbound_scale, vbB = hb.vbound * P.vbound_scale;
       /* the previous pair's reads are done before the stage is overwritten */
@@ -1630,11 +1678,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
       S.area[h][k] = farea;
       S.fnv[h][k] = fnv;
       __builtin_amdgcn_wave_barrier();
+      /* A's place in B's list (absent when that list overflowed) */
+      const uint32_t at = (uint32_t)__ballot(!h && (uint32_t)k < nback && back == slot / LIST_STRIDE);
+      const uint32_t slot_b = at ? partner * LIST_STRIDE + (uint32_t)(__ffs(at) - 1) : NO_SLOT;
       const Shape A{S.v[0], S.fn[0], S.fc[0], ha.nv, ha.nf, S.vo[0], S.area[0], S.fnv[0]};
       const Shape B{S.v[1], S.fn[1], S.fc[1], hb.nv, hb.nf, S.vo[1], S.area[1], S.fnv[1]};
       const PairDirs D = pair_dirs(A, B, o.PosA, o.PosB);
       const uint32_t code = separated_wave(A, B, o.PosA, o.PosB, D);
-      PColl c{false, C_SP, 0.0f, mk3(0.f, 0.f, 0.f), mk3(0.f, 0.f, 0.f)};
+      PColl c{false, C_SP, 0.0f, mk3(0.f, 0.f, 0.f), mk3(0.f, 0.f, 0.f)};   /* lanes 0-31: A's, 32-63: B's */
       if (code != HINT_NONE) {
         if (lane == 0) {
           const int ida = packed_pid(omg[o.a].w);
@@ -1642,25 +1693,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
             hint[(size_t)ida * LIST_STRIDE + (slot % LIST_STRIDE)] = make_uint2((uint32_t)packed_pid(omg[o.b].w), code);
         }
       } else {
-        c = vertex_faces_pair(o.PosA, A, o.PosB, B, D);
-        if (!c.hit) {
-          const f3 RelPos = (o.PosA - o.PosB) / length(o.PosA - o.PosB);
-          c = edges_wave(A, S.e[0], ha.ne, B, S.e[1], hb.ne, RelPos, o.PosA, o.PosB, vbA, vbB,
+        PColl ab = c, ba = c;
+        if (vertex_faces_both(o.PosA, A, o.PosB, B, D, ab, ba)) {
+          c = h ? ba : ab;
+        } else {
+          c = edges_wave(A, S.e[0], ha.ne, B, S.e[1], hb.ne, o.PosA, o.PosB, vbA, vbB,
                          ha.plane_slack * P.vbound_scale, hb.plane_slack * P.vbound_scale, S.ia, S.ib, D.fA, D.fB);
-          if (c.hit) c.dis = fminf(0.025f * ha.radius, c.dis);
+          if (c.hit) c.dis = fminf(0.025f * (h ? hb : ha).radius, c.dis);
         }
       }
-      /* the pair law runs for the whole chunk at once below, a lane per pair */
-      if (lane == 0) R[j] = PairHit{c.hit ? 1u : 0u, c.dis, c.n.x, c.n.y, c.n.z, c.cp.x, c.cp.y, c.cp.z};
+      /* the pair law runs for the whole chunk at once below, a lane per contact */
+      if (k == 0)
+        R[h][j] = PairHit{c.hit ? (h ? slot_b : slot) : NO_SLOT, c.dis, c.n.x, c.n.y, c.n.z, c.cp.x, c.cp.y, c.cp.z};
     }
     __builtin_amdgcn_wave_barrier();
-    if ((uint32_t)lane < m && lslot < cap) {
-      const PairHit r = R[lane];
-      const PairOps o = pair_ops_ab(P, lslot, lpart, pos, vel, omg);
-      pair_store(P, shapes[lsa], o, PColl{r.hit != 0u, C_UNDEF, r.dis, mk3(r.nx, r.ny, r.nz), mk3(r.cx, r.cy, r.cz)},
-                 lslot, pf, pt, tally);
+    const uint32_t ps = (uint32_t)__shfl((int)lslot, k, 64), pp = (uint32_t)__shfl((int)lpart, k, 64);
+    const uint32_t sa = (uint32_t)__shfl((int)lsa, k, 64), sb = (uint32_t)__shfl((int)lsb, k, 64);
+    if ((uint32_t)k < m) {
+      const PairHit r = R[h][k];
+      if (r.slot != NO_SLOT) {
+        const PairOps o = pair_ops_ab(P, r.slot, h ? ps / LIST_STRIDE : pp, pos, vel, omg);
+        pair_store(P, shapes[h ? sb : sa], o, PColl{true, C_UNDEF, r.dis, mk3(r.nx, r.ny, r.nz), mk3(r.cx, r.cy, r.cz)},
+                   r.slot, pf, pt, hitf, tally);
+      }
     }
     __builtin_amdgcn_wave_barrier();   /* the records are read before the next chunk writes them */
+  };
+
+  const uint32_t waves = gridDim.x * (blockDim.x / 64u);
+  const uint32_t wid = blockIdx.x * (blockDim.x / 64u) + (threadIdx.x >> 6);
+  uint32_t own = cnt / (2u * waves);
+  own = own < 1u ? 1u : (own > NARROW_CHUNK ? NARROW_CHUNK : own);
+  if (wid * own < cnt) process(wid * own, min(own, cnt - wid * own));
+  const uint32_t dealt = waves * own;
+  if (dealt >= cnt) return;
+  const uint32_t slice = blockIdx.x % POLY_SLICES;
+  const uint32_t s0 = dealt + (uint32_t)((uint64_t)(cnt - dealt) * slice / POLY_SLICES);
+  const uint32_t len = dealt + (uint32_t)((uint64_t)(cnt - dealt) * (slice + 1u) / POLY_SLICES) - s0;
+  uint32_t seen = 0u;   /* the counter's value at this wave's last grab */
+  while (seen < len) {
+    uint32_t size = (len - seen) / (2u * (waves / POLY_SLICES));
+    size = size < 2u ? 2u : (size > NARROW_CHUNK ? NARROW_CHUNK : size);
+    uint32_t base = 0u;
+    if (lane == 0) base = atomicAdd(&qcount[(POLY_SUBQ + slice) * POLY_QSTRIDE], size);
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (base >= len) break;
+    seen = base + size;
+    process(s0 + base, min(size, len - base));
   }
 }
 
@@ -1670,7 +1749,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 template <bool FORCES_ONLY, bool LIFTERS>
 __global__ __launch_bounds__(256) void k_poly_finish(
     const DevParams* __restrict__ Pp, const bdem_poly_shape* __restrict__ shapes, int n, PolyLayout L,
-    const float4* __restrict__ rot, const uint32_t* __restrict__ nn, const float4* __restrict__ pf,
+    const float4* __restrict__ rot, const uint8_t* __restrict__ hitf, const float4* __restrict__ pf,
     const float4* __restrict__ pt, const float4* __restrict__ pos_in, const float4* __restrict__ vel_in,
     const float4* __restrict__ omg_in, const float4* __restrict__ quat_in, float4* __restrict__ pos_out,
     float4* __restrict__ vel_out, float4* __restrict__ omg_out, float4* __restrict__ quat_out,
@@ -1695,14 +1774,16 @@ __global__ __launch_bounds__(256) void k_poly_finish(
     if (pid >= 0) {
       const bdem_poly_shape& po = shapes[shape_index(P, ot.w)];
       f3 Fpp = cvt(P.gravity) * m, Tpp = mk3(0.f, 0.f, 0.f);
-      const uint32_t c = nn[i];
-      const int cnt = c < (uint32_t)LIST_STRIDE ? (int)c : LIST_STRIDE;
-      for (int k = 0; k < cnt; ++k) {
-        const float4 f = pf[(size_t)i * LIST_STRIDE + k];
-        if (f.w != 0.0f) {
-          Fpp = Fpp + xyz(f);
-          Tpp = Tpp + xyz(pt[(size_t)i * LIST_STRIDE + k]);
-        }
+      /* the marked contacts, in list order */
+      const uint4 h0 = reinterpret_cast<const uint4*>(hitf)[2 * (size_t)i], h1 = reinterpret_cast<const uint4*>(hitf)[2 * (size_t)i + 1];
+      auto nibble = [](uint32_t b) { return (b & 1u) | ((b >> 7) & 2u) | ((b >> 14) & 4u) | ((b >> 21) & 8u); };
+      uint32_t hit = nibble(h0.x) | nibble(h0.y) << 4 | nibble(h0.z) << 8 | nibble(h0.w) << 12 | nibble(h1.x) << 16 |
+                     nibble(h1.y) << 20 | nibble(h1.z) << 24 | nibble(h1.w) << 28;
+      while (hit) {
+        const int k = __ffs(hit) - 1;
+        hit &= hit - 1u;
+        Fpp = Fpp + xyz(pf[(size_t)i * LIST_STRIDE + k]);
+        Tpp = Tpp + xyz(pt[(size_t)i * LIST_STRIDE + k]);
       }
       if (!P.rotation) Tpp = mk3(0.f, 0.f, 0.f);
       const Shape A = shape_of(rot, L, i, po);
@@ -1768,22 +1849,22 @@ __global__ __launch_bounds__(256) void k_poly_finish(
 
 /* ------------------------------------------------------------------ launchers */
 /* Blocks of 256 threads of `kernel` that the device holds at once (every
- * CU full), a multiple of the 8 XCDs: the grid of the two pair kernels, so
- * that no partial second round of blocks starts late.  Queried once per
- * device (slot: which kernel). */
+ * CU full), a multiple of POLY_SLICES: the grid of the wave-per-pair kernel,
+ * so that no partial second round of blocks starts late.  Queried once per
+ * device. */
 template <class K>
-static unsigned resident_blocks(K kernel, int slot) {
-  static std::atomic<unsigned> cache[2][64];
+static unsigned resident_blocks(K kernel) {
+  static std::atomic<unsigned> cache[64];
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return (unsigned)POLY_PAIR_BLOCKS;
-  unsigned nb = cache[slot][dev].load(std::memory_order_relaxed);
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 1024u;
+  unsigned nb = cache[dev].load(std::memory_order_relaxed);
   if (nb == 0u) {
     int per = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, 256, 0) != hipSuccess || per <= 0) per = 8;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, 256, 0) != hipSuccess || per <= 0) per = 4;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    nb = (unsigned)(per * cus) / NUM_XCD * NUM_XCD;
-    if (nb < (unsigned)NUM_XCD) nb = NUM_XCD;
-    cache[slot][dev].store(nb, std::memory_order_relaxed);
+    nb = (unsigned)(per * cus) / POLY_SLICES * POLY_SLICES;
+    if (nb < (unsigned)POLY_SLICES) nb = POLY_SLICES;
+    cache[dev].store(nb, std::memory_order_relaxed);
   }
   return nb;
 }
@@ -1798,19 +1879,20 @@ static void launch_poly_forces_common(const DevParams* dP, const bdem_poly_shape
    * against 20 us at 50,000 */
   if (b.n <= LIST_TEAM_MAX)
     hipLaunchKernelGGL(k_poly_list, dim3((b.n + LIST_BLOCK - 1) / LIST_BLOCK), dim3(256), 0, s, dP, b.n, b.cells,
-                       b.pos_srt, b.omg_srt, pb.list, pb.nn, pb.queue, pb.qcount, b.status);
+                       b.pos_srt, b.omg_srt, pb.list, pb.nn, pb.hitf, b.status);
   else
     hipLaunchKernelGGL(k_poly_list2, dim3((b.n + LIST2_BLOCK - 1) / LIST2_BLOCK), dim3(64 * LIST2_WAVES), 0, s, dP,
-                       b.n, b.cells, b.pos_srt, b.omg_srt, sk, pb.list, pb.nn, pb.queue, pb.qcount, b.status);
-  /* both pair kernels loop over their queues with the resident grid; the
-   * first splits its queue by XCD (a grid of whole XCD multiples) */
-  static_assert(POLY_PAIR_BLOCKS % NUM_XCD == 0, "the pair kernel splits its queue by XCD");
-  hipLaunchKernelGGL(k_poly_pairs, dim3(resident_blocks(k_poly_pairs, 0)), dim3(256), 0, s, dP, dshape, pb.hdr, b.n,
-                     pb.L, pb.rot, b.pos_srt, b.vel_srt, b.omg_srt, pb.list, pb.queue, pb.qcount, pb.equeue, pb.pf,
-                     pb.pt, pb.hint);
-  hipLaunchKernelGGL(k_poly_narrow, dim3(resident_blocks(k_poly_narrow, 1)), dim3(256), 0, s, dP, dshape, pb.hdr, b.n,
-                     pb.L, pb.rot,
-                     b.pos_srt, b.vel_srt, b.omg_srt, pb.qcount, pb.equeue, pb.pf, pb.pt, energy ? 1 : 0, pb.hint);
+                       b.n, b.cells, b.pos_srt, b.omg_srt, sk, pb.list, pb.nn, pb.hitf, b.status);
+  const uint32_t subcap = poly_subqueue_capacity(b.n);
+  auto pairs = [&](auto kernel, int ppb) {
+    hipLaunchKernelGGL(kernel, dim3((b.n + ppb - 1) / ppb), dim3(256), 0, s, dP, pb.hdr, b.n, pb.L, pb.rot, b.pos_srt,
+                       b.omg_srt, pb.list, pb.nn, pb.qcount, pb.equeue, subcap, pb.hint);
+  };
+  if (b.n <= POLY_PAIRS_SMALL) pairs(k_poly_pairs<POLY_PPB_SMALL>, POLY_PPB_SMALL);
+  else pairs(k_poly_pairs<POLY_PPB>, POLY_PPB);
+  hipLaunchKernelGGL(k_poly_narrow, dim3(resident_blocks(k_poly_narrow)), dim3(256), 0, s, dP, dshape, pb.hdr, b.n,
+                     pb.L, pb.rot, b.pos_srt, b.vel_srt, b.omg_srt, pb.list, pb.nn, pb.qcount, pb.equeue, subcap,
+                     pb.pf, pb.pt, pb.hitf, energy ? 1 : 0, pb.hint);
 }
 
 /* World-frame shapes of the current (unsorted) state into pb.rot: the
@@ -1830,7 +1912,7 @@ void launch_poly_step(const DevParams* dP, const bdem_poly_shape* dshape, const 
   /* the lifter search needs private arrays (scratch): only its own instantiation carries it */
   auto k = lifters ? k_poly_finish<false, true> : k_poly_finish<false, false>;
   hipLaunchKernelGGL(k, dim3((b.n + 255) / 256), dim3(256), 0, s, dP, dshape, b.n, pb.L,
-                     pb.rot, pb.nn, pb.pf, pb.pt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, b.pos_cur,
+                     pb.rot, pb.hitf, pb.pf, pb.pt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, b.pos_cur,
                      b.vel_cur, b.omg_cur, b.quat_cur, b.keys_new, sk, b.changed, b.sbuf,
                      b.meta + META_APPEND + ap, b.hwc_srt, b.hwc_cur, want_wf ? b.wall_force : nullptr,
                      do_kill ? 1 : 0, b.status, b.kill_count, nullptr, nullptr, nullptr, nullptr, energy ? 1 : 0);
@@ -1840,7 +1922,7 @@ void launch_poly_forces(const DevParams* dP, const bdem_poly_shape* dshape, cons
                         const uint32_t* sk, float* fpp, float* tpp, float* fw, float* tw, hipStream_t s) {
   launch_poly_forces_common(dP, dshape, b, pb, sk, false, s);
   hipLaunchKernelGGL((k_poly_finish<true, false>), dim3((b.n + 255) / 256), dim3(256), 0, s, dP, dshape, b.n, pb.L,
-                     pb.rot, pb.nn, pb.pf, pb.pt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, nullptr, nullptr,
+                     pb.rot, pb.hitf, pb.pf, pb.pt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, nullptr, nullptr,
                      nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
                      b.status, b.kill_count, fpp, tpp, fw, tw, 0);
 }
