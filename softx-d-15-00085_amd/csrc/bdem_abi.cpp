@@ -793,6 +793,8 @@ int bdem_set_simulation_data(bdem_ctx* c, const bdem_WOBJ* wobj, const bdem_POBJ
     ALLOC(pb.hitf, (size_t)n * LIST_STRIDE);
     ALLOC(pb.pf, (size_t)n * LIST_STRIDE);
     ALLOC(pb.pt, (size_t)n * LIST_STRIDE);
+    ALLOC(pb.lf, (size_t)n);
+    ALLOC(pb.lt, (size_t)n);
     ALLOC(pb.hint, (size_t)n * LIST_STRIDE);
     launch_fill_u32(reinterpret_cast<uint32_t*>(pb.hint), (size_t)n * LIST_STRIDE * 2, 0xFFFFFFFFu, c->stream);
     launch_fill_u32(pb.nn, (size_t)n, 0u, c->stream);

@@ -82,6 +82,7 @@ struct PolyBuffers {
                                           the wave-per-pair kernel's slice counters */
   uint8_t* hitf;                       /* n * 32: 1 where the slot's pair is in contact */
   float4 *pf, *pt;                     /* n * 32: pair force, torque, where hitf is set */
+  float4 *lf, *lt;                     /* n: lifter force (w = 1 when in contact), torque */
   uint2* hint;                         /* n * 32 by P_ID and list slot: (partner P_ID, separating face code) */
 };
 constexpr int POLY_SUBQ = 64, POLY_SLICES = 8;

@@ -924,35 +924,36 @@ __device__ __forceinline__ void wall_forces_poly(const DevParams& P, int t, f3 p
 }
 
 /* ---- polyhedra against lifters (VolumeObject_InteractionParticle,
- * DEM_Kernels_Compute.cuh:100-224), one thread per particle: lifter contacts
- * are few, so the serial form of the restatement is kept. */
+ * DEM_Kernels_Compute.cuh:100-224), a wave per particle near a lifter.  A's
+ * turned vertices are in LDS. */
 
-/* is_SP_VolumeObject_Poly (Utilities.cuh:272-309) */
+/* is_SP_VolumeObject_Poly (Utilities.cuh:272-309): some face of D has P's
+ * centre and every vertex of A strictly in front; two faces a round, a lane
+ * per vertex. */
 __device__ __forceinline__ bool sp_dobj_poly(const bdem_DOBJ& D, f3 PosP, const Shape& A) {
-  for (int f = 0; f < D.num_faces; ++f) {
-    const f3 n = cvt(D.faces[f].normal), c = cvt(D.faces[f].centroid);
-    if (dot(n, PosP - c) > 0.0f) {
-      bool contact = false;
-      for (int v = 0; v < A.nv; ++v)
-        if (dot(n, ld3(A.V + v) - c) <= 0.00000f) { contact = true; break; }
-      if (!contact) return true;
-    }
+  const int lane = threadIdx.x & 63, v = lane & 31;
+  const bool vv = v < A.nv;
+  const f3 pv = ld3(A.V + (vv ? v : 0));
+  for (int f0 = 0; f0 < D.num_faces; f0 += 2) {
+    const int f = f0 + (lane >> 5);
+    const bool fv = f < D.num_faces;
+    const f3 n = cvt(D.faces[fv ? f : f0].normal), c = cvt(D.faces[fv ? f : f0].centroid);
+    const uint64_t front = __ballot(fv && dot(n, PosP - c) > 0.0f);
+    const uint64_t behind = __ballot(vv && dot(n, pv - c) <= 0.00000f);
+    if ((front & 1ull) && (uint32_t)behind == 0u) return true;
+    if ((front >> 32 & 1ull) && (uint32_t)(behind >> 32) == 0u) return true;
   }
   return false;
 }
 
-/* is_SP_Poly_VolumeObject (Utilities.cuh:212-247) */
+/* is_SP_Poly_VolumeObject (Utilities.cuh:212-247), a lane per face of A */
 __device__ __forceinline__ bool sp_poly_dobj(const Shape& A, f3 PosD, const bdem_DOBJ& D) {
-  for (int f = 0; f < A.nf; ++f) {
-    const f3 n = ld3(A.Fn + f), c = ld3(A.Fc + f);
-    if (dot(n, PosD - c) > 0.0f) {
-      bool contact = false;
-      for (int v = 0; v < D.num_vertex; ++v)
-        if (dot(n, cvt(D.vertex[v]) - c) <= 0.00000f) { contact = true; break; }
-      if (!contact) return true;
-    }
-  }
-  return false;
+  const int f = threadIdx.x & 63;
+  const bool fv = f < A.nf;
+  const f3 n = ld3(A.Fn + (fv ? f : 0)), c = ld3(A.Fc + (fv ? f : 0));
+  bool contact = false;
+  for (int v = 0; v < D.num_vertex; ++v) contact = contact || dot(n, cvt(D.vertex[v]) - c) <= 0.00000f;
+  return __ballot(fv && dot(n, PosD - c) > 0.0f && !contact) != 0ull;
 }
 
 /* Collision_Detection_Vertex_InDObject_3Faces (Collision_Detection_Polyhedra.cuh:383-476) */
@@ -1014,27 +1015,35 @@ __device__ __forceinline__ bool ray_hits_dface(f3 PosP, f3 through, const bdem_D
   return point_on_dface(D.faces[f], D.vertex, PosP + d * Ray, tol);
 }
 
-/* Collision_Detection_Polyhedara_VolumeObject_VertexFace (Collision_Detection_Polyhedra.cuh:1638-1990) */
+/* Lane l's InPoly, wave-uniform. */
+__device__ __forceinline__ InPoly in_poly_of(const InPoly& t, int l) {
+  return InPoly{__builtin_amdgcn_readlane(t.f0, l), __builtin_amdgcn_readlane(t.f1, l),
+                __builtin_amdgcn_readlane(t.f2, l), lane_f32(t.d0, l), lane_f32(t.d1, l), lane_f32(t.d2, l)};
+}
+
+/* Collision_Detection_Polyhedara_VolumeObject_VertexFace (Collision_Detection_Polyhedra.cuh:1638-1990):
+ * a lane per vertex; the first eight inside vertices are taken in ascending
+ * order, as the serial loop appends them. */
 __device__ __forceinline__ PColl vertex_faces_dobj(f3 PosP, const Shape& A, const bdem_DOBJ& D) {
   PColl res{false, C_UNDEF, 0.0f, mk3(0.f, 0.f, 0.f), mk3(0.f, 0.f, 0.f)};
-  int np = 0, valid[8];
-  InPoly sel[8];
-  for (int v = 0; v < A.nv; ++v) {
-    InPoly t;
-    if (vertex_in_dobj(PosP, ld3(A.V + v), D, t)) {
-      if (np < 8) { sel[np] = t; valid[np] = v; }
-      ++np;
-    }
-  }
+  const int lane = threadIdx.x & 63;
+  InPoly t;
+  const bool vv = lane < A.nv;
+  const bool in = vertex_in_dobj(PosP, ld3(A.V + (vv ? lane : 0)), D, t);
+  uint32_t mask = (uint32_t)__ballot(vv && in);
+  int np = __popc(mask);
   if (np == 0) return res;
   np = min(np, 8);
+  const int v0 = __ffs(mask) - 1;
+  const uint32_t after = mask & (mask - 1u);
+  const int v1 = after ? __ffs(after) - 1 : v0;
   res.hit = true;
-  const InPoly s0 = sel[0];
+  const InPoly s0 = in_poly_of(t, v0);
   if (np == 1) {
     res.cls = C_VF;
     res.dis = s0.d0;
     res.n = dnorm(D, s0.f0);
-    res.cp = ld3(A.V + valid[0]);
+    res.cp = ld3(A.V + v0);
     if (s0.f1 == -1) return res;
     if (ray_hits_dface(PosP, res.cp, D, s0.f0, 0.1f)) return res;
     for (int q = 1; q < 3; ++q) {
@@ -1049,10 +1058,10 @@ __device__ __forceinline__ PColl vertex_faces_dobj(f3 PosP, const Shape& A, cons
   }
   if (np == 2) {
     res.cls = C_EF;
-    res.cp = (ld3(A.V + valid[0]) + ld3(A.V + valid[1])) * 0.50f;
+    res.cp = (ld3(A.V + v0) + ld3(A.V + v1)) * 0.50f;
     res.n = dnorm(D, s0.f0);
     res.dis = fabsf(dot(dnorm(D, s0.f0), (res.cp - dcent(D, s0.f0))));
-    if (s0.f1 == -1 && sel[1].f1 == -1) return res;
+    if (s0.f1 == -1 && in_poly_of(t, v1).f1 == -1) return res;
     for (int q = 0; q < 3; ++q) {
       const int f = face_at(s0, q);
       if (q > 0 && !(f > -1)) continue;
@@ -1066,21 +1075,28 @@ __device__ __forceinline__ PColl vertex_faces_dobj(f3 PosP, const Shape& A, cons
   }
   res.cls = C_FF;
   f3 cp = mk3(0.0f, 0.0f, 0.0f);
-  for (int q = 0; q < np; ++q) cp = cp + ld3(A.V + valid[q]);
-  res.cp = cp / (float)np;
   int common[3] = {0, 0, 0};
   float cdis[3] = {10.0f, 10.0f, 10.0f};
-  for (int q = 0; q < np; ++q)
+  for (int q = 0; q < np; ++q) {
+    const int v = __ffs(mask) - 1;
+    mask &= mask - 1u;
+    cp = cp + ld3(A.V + v);
+    const InPoly sq = in_poly_of(t, v);
     for (int j = 0; j < 3; ++j) {
-      const int f = face_at(sel[q], j);
-      if (f > -1 && f < 3) {
-        common[f]++;
-        const float dj = dist_at(sel[q], j);
-        if (dj < cdis[f]) cdis[f] = dj;
-      }
+      const int f = face_at(sq, j);
+      const float dj = dist_at(sq, j);
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (f == k) {
+          common[k]++;
+          if (dj < cdis[k]) cdis[k] = dj;
+        }
     }
-  for (int f = 0; f < D.num_faces && f < 3; ++f)
-    if (common[f] == np) {
+  }
+  res.cp = cp / (float)np;
+#pragma unroll
+  for (int f = 0; f < 3; ++f)
+    if (f < D.num_faces && common[f] == np) {
       res.dis = cdis[f];
       res.n = dnorm(D, f);
       return res;
@@ -1090,55 +1106,64 @@ __device__ __forceinline__ PColl vertex_faces_dobj(f3 PosP, const Shape& A, cons
 
 /* Collision_Detection_DObject_Polyhedra_Edges (Collision_Detection_Polyhedra.cuh:716-890);
  * no crossing within 0.1 cm of the other point (the reference then reads an
- * unset normal) is no contact. */
+ * unset normal) is no contact.  Per edge of D a lane per edge of B; the
+ * crossings are summed in the serial order, and of equal least distances the
+ * last one counts, as the serial loop's <= leaves it. */
 __device__ __forceinline__ PColl edges_dobj(const bdem_DOBJ& D, const Shape& B, const bdem_poly_shape& pb, f3 PosB,
                                             f3 RelPos) {
   PColl res{false, C_SP, 0.0f, mk3(0.f, 0.f, 0.f), mk3(0.0f, 0.0f, 0.0f)};
-  float min_edgedis = 0.10f;
+  const int lane = threadIdx.x & 63;
+  const bool ev = lane < pb.num_edges;
+  const bdem_Edge_Def eb = pb.edge[ev ? lane : 0];
+  const f3 PB = ld3(B.V + eb.point_vindex[0]);
+  const f3 DB = ld3(B.V + eb.point_vindex[1]) - PB;
+  float best = 0.10f;
   f3 selA = mk3(0.f, 0.f, 0.f), selB = selA, nsel = selA, cpsum = selA;
-  int count = 0;
-  bool found = false, have_min = false;
+  int count = 0, bi = -1;   /* bi: the lane's best edge of D */
   for (int i = 0; i < D.num_edges; ++i) {
     const f3 PA = cvt(D.vertex[D.edge[i].point_vindex[0]]);
     const f3 DA = cvt(D.vertex[D.edge[i].point_vindex[1]]) - PA;
     const float DEAD = dot(DA, DA);
-    for (int j = 0; j < pb.num_edges; ++j) {
-      const f3 PB = ld3(B.V + pb.edge[j].point_vindex[0]);
-      const f3 DB = ld3(B.V + pb.edge[j].point_vindex[1]) - PB;
-      const f3 dir = cross(DA / length(DA), DB / length(DB));
-      const float mag = dot(dir, dir);
-      if (!(mag > 0.00000f)) continue;
-      f3 DV = PA - PB;
-      const float DEBD = dot(DB, DB);
-      const float DEABD = dot(DA, DB);
-      const float DEADAB = dot(DA, DV);
-      const float DEBDAB = dot(DB, DV);
-      const float detJinv = 1.00000f / (DEABD * DEABD - DEAD * DEBD);
-      const float dA = detJinv * (DEBD * DEADAB - DEABD * DEBDAB);
-      if (!(dA >= -0.010f && dA <= 1.0100f)) continue;
-      const float dB = detJinv * (DEABD * DEADAB - DEAD * DEBDAB);
-      if (!(dB >= -0.0100f && dB <= 1.010f)) continue;
-      const f3 pA = PA + DA * dA;
-      const f3 pB = PB + DB * dB;
-      DV = (pA - pB);
-      float dis = dot(DV, DV);
-      if (!(dis > 0.00000f)) continue;
-      dis = __builtin_sqrtf(dis);
-      if (length(PosB - pB) > length(PosB - pA)) {
-        ++count;
-        cpsum = cpsum + pA;
-        found = true;
-        if (dis <= min_edgedis) {
-          min_edgedis = dis;
-          nsel = cross(DA, DB);
-          selA = pA;
-          selB = pB;
-          have_min = true;
-        }
-      }
+    const f3 dir = cross(DA / length(DA), DB / length(DB));
+    const float mag = dot(dir, dir);
+    f3 DV = PA - PB;
+    const float DEBD = dot(DB, DB);
+    const float DEABD = dot(DA, DB);
+    const float DEADAB = dot(DA, DV);
+    const float DEBDAB = dot(DB, DV);
+    const float detJinv = 1.00000f / (DEABD * DEABD - DEAD * DEBD);
+    const float dA = detJinv * (DEBD * DEADAB - DEABD * DEBDAB);
+    const float dB = detJinv * (DEABD * DEADAB - DEAD * DEBDAB);
+    const f3 pA = PA + DA * dA;
+    const f3 pB = PB + DB * dB;
+    DV = (pA - pB);
+    float dis = dot(DV, DV);
+    const bool near = ev && mag > 0.00000f && dA >= -0.010f && dA <= 1.0100f && dB >= -0.0100f && dB <= 1.010f &&
+                      dis > 0.00000f && length(PosB - pB) > length(PosB - pA);
+    dis = __builtin_sqrtf(dis);
+    if (near && dis <= best) {
+      best = dis;
+      bi = i;
+      nsel = cross(DA, DB);
+      selA = pA;
+      selB = pB;
+    }
+    uint64_t m = __ballot(near);
+    count += __popcll(m);
+    while (m) {
+      const int l = __ffsll((unsigned long long)m) - 1;
+      m &= m - 1ull;
+      cpsum = cpsum + mk3(lane_f32(pA.x, l), lane_f32(pA.y, l), lane_f32(pA.z, l));
     }
   }
-  if (!found || !have_min) return res;
+  const float least = wave_min(bi >= 0 ? best : 3.0e38f);
+  const bool cand = bi >= 0 && best == least;
+  if (__ballot(cand) == 0ull) return res;
+  const int last = -wave_min_i32(cand ? -(bi * 64 + lane) : 1);
+  const int w = last & 63;
+  nsel = mk3(lane_f32(nsel.x, w), lane_f32(nsel.y, w), lane_f32(nsel.z, w));
+  selA = mk3(lane_f32(selA.x, w), lane_f32(selA.y, w), lane_f32(selA.z, w));
+  selB = mk3(lane_f32(selB.x, w), lane_f32(selB.y, w), lane_f32(selB.z, w));
   const f3 n = nsel * (1.0f / length(nsel));
   res.hit = true;
   res.cls = C_EE;
@@ -1153,45 +1178,6 @@ __device__ __forceinline__ PColl edges_dobj(const bdem_DOBJ& D, const Shape& B, 
     res.dis = fabsf(dot(res.n, (selB - selA))) + 0.000010f;
   }
   return res;
-}
-
-/* Lifter force and torque on a polyhedron: the first lifter in contact acts. */
-__device__ __forceinline__ void lifter_forces_poly(const DevParams& P, int t, f3 p, f3 v, f3 w, float m,
-                                                   const Shape& A, const bdem_poly_shape& pa, f3& F, f3& T,
-                                                   float* tally) {
-  F = mk3(0.f, 0.f, 0.f);
-  T = F;
-  const float r = pa.radius;
-  const bool check = P.dobj[0].is_translating || !P.mill_sim || P.rotating_wobj ||
-                     length(mk3(p.x, p.y, 0.0f) - cvt(P.mill_cent)) > (P.dobj_bound_r - 2.0f * r);
-  if (!check) return;
-  for (int d = 0; d < P.num_dobj; ++d) {
-    const bdem_DOBJ& D = P.dobj[d];
-    const f3 BV = (p - cvt(D.COM)) * cvt(D.Axis);
-    if (!(length(BV) < (D.boundR + r))) continue;
-    PColl res{false, C_SP, 0.0f, mk3(0.f, 0.f, 0.f), mk3(0.f, 0.f, 0.f)};
-    bool sp = sp_dobj_poly(D, p, A);
-    if (!sp) sp = sp_poly_dobj(A, cvt(D.COM), D);
-    if (!sp) {
-      f3 PosD = cvt(D.COM);
-      PosD.z = p.z;
-      res = vertex_faces_dobj(p, A, D);
-      if (!res.hit) {
-        const f3 RelPos = (PosD - p) / length(PosD - p);
-        res = edges_dobj(D, A, pa, p, RelPos);
-      }
-    }
-    if (!res.hit) continue;
-    f3 Vl = mk3(0.f, 0.f, 0.f);
-    if (D.is_attached_DWorld) Vl = drum_velocity(P, res.cp);
-    else if (D.is_translating) Vl = cvt(D.velocity);
-    const DColl c{true, 0, res.dis, res.n, res.cp};
-    f3 Ftr, Tq;
-    resp_dobject(P, t, p, v, w, m, c, Vl, Ftr, Tq, tally);
-    F = F + Ftr;
-    if (P.rotation) T = T + Tq;
-    break;
-  }
 }
 
 }  // namespace
@@ -1743,6 +1729,88 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
   }
 }
 
+/* Lifter force and torque of every particle (w = 1 in lf where there is a
+ * contact): the first lifter in contact acts.  A wave takes PPW particles;
+ * a lane each finds the lifters within reach, then the whole wave works on
+ * one particle and lifter at a time.  (A lane per particle inside
+ * k_poly_finish ran these searches serially with private arrays in scratch:
+ * 84 us of a step at 3,001 hulls, some 50 at 200,000.) */
+template <int PPW>
+__global__ __launch_bounds__(256) void k_poly_lift(const DevParams* __restrict__ Pp,
+                                                   const bdem_poly_shape* __restrict__ shapes,
+                                                   const ShapeHdr* __restrict__ hdr, int n, PolyLayout L,
+                                                   const float4* __restrict__ rot, const float4* __restrict__ pos,
+                                                   const float4* __restrict__ vel, const float4* __restrict__ omg,
+                                                   float4* __restrict__ lf, float4* __restrict__ lt, int energy) {
+  const DevParams& P = *Pp;
+  __shared__ float4 verts[4][BDEM_SHAPE_MAX_VERTEX];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int i0 = (xcd_block(blockIdx.x, gridDim.x) * 4 + wave) * PPW, i = i0 + lane;
+  const bool in = lane < PPW && i < n;
+  uint32_t reach = 0u;
+  if (in) {
+    const float w = omg[i].w;
+    if (packed_pid(w) >= 0) {
+      const f3 p = xyz(pos[i]);
+      const float r = hdr[shape_index(P, w)].radius;
+      const bool check = P.dobj[0].is_translating || !P.mill_sim || P.rotating_wobj ||
+                         length(mk3(p.x, p.y, 0.0f) - cvt(P.mill_cent)) > (P.dobj_bound_r - 2.0f * r);
+      if (check)
+        for (int d = 0; d < P.num_dobj; ++d) {
+          const bdem_DOBJ& D = P.dobj[d];
+          const f3 BV = (p - cvt(D.COM)) * cvt(D.Axis);
+          if (length(BV) < (D.boundR + r)) reach |= 1u << d;
+        }
+    }
+  }
+  float4 F4 = make_float4(0.f, 0.f, 0.f, 0.f), T4 = F4;
+  uint64_t todo = __ballot(reach != 0u);
+  while (todo) {
+    const int s = __ffsll((unsigned long long)todo) - 1;
+    todo &= todo - 1ull;
+    const int a = i0 + s;
+    uint32_t ds = (uint32_t)__builtin_amdgcn_readlane((int)reach, s);
+    const float4 pr = pos[a], vm = vel[a], ot = omg[a];
+    const int row = shape_index(P, ot.w), t = packed_type(ot.w);
+    const ShapeHdr hd = hdr[row];
+    const f3 p = xyz(pr), v = xyz(vm), w = xyz(ot);
+    const float4* const ra = rot + (size_t)a * L.stride;
+    __builtin_amdgcn_wave_barrier();   /* the previous particle's reads are done */
+    if (lane < BDEM_SHAPE_MAX_VERTEX) verts[wave][lane] = ra[lane < L.pv ? lane : 0];
+    __builtin_amdgcn_wave_barrier();
+    const Shape A{verts[wave], ra + L.pv, ra + L.pv + L.pf, hd.nv, hd.nf};
+    while (ds) {
+      const int d = __ffs(ds) - 1;
+      ds &= ds - 1u;
+      const bdem_DOBJ& D = P.dobj[d];
+      if (sp_dobj_poly(D, p, A) || sp_poly_dobj(A, cvt(D.COM), D)) continue;
+      f3 PosD = cvt(D.COM);
+      PosD.z = p.z;
+      PColl res = vertex_faces_dobj(p, A, D);
+      if (!res.hit) {
+        const f3 RelPos = (PosD - p) / length(PosD - p);
+        res = edges_dobj(D, A, shapes[row], p, RelPos);
+      }
+      if (!res.hit) continue;
+      f3 Vl = mk3(0.f, 0.f, 0.f);
+      if (D.is_attached_DWorld) Vl = drum_velocity(P, res.cp);
+      else if (D.is_translating) Vl = cvt(D.velocity);
+      const DColl c{true, 0, res.dis, res.n, res.cp};
+      f3 Ftr, Tq;
+      resp_dobject(P, t, p, v, w, vm.w, c, Vl, Ftr, Tq, energy && lane == 0 ? P.tally : nullptr);
+      if (lane == s) {
+        F4 = make_float4(Ftr.x, Ftr.y, Ftr.z, 1.0f);
+        T4 = make_float4(Tq.x, Tq.y, Tq.z, 0.0f);
+      }
+      break;
+    }
+  }
+  if (in) {
+    lf[i] = F4;
+    if (F4.w != 0.0f) lt[i] = T4;
+  }
+}
+
 /* Per particle: gravity, the pair slots in list order, walls, integration,
  * discharge, next key, changed flag and changed-list append (as k_step).
  * FORCES_ONLY stops after the forces and writes them (debug stage). */
@@ -1750,8 +1818,9 @@ template <bool FORCES_ONLY, bool LIFTERS>
 __global__ __launch_bounds__(256) void k_poly_finish(
     const DevParams* __restrict__ Pp, const bdem_poly_shape* __restrict__ shapes, int n, PolyLayout L,
     const float4* __restrict__ rot, const uint8_t* __restrict__ hitf, const float4* __restrict__ pf,
-    const float4* __restrict__ pt, const float4* __restrict__ pos_in, const float4* __restrict__ vel_in,
-    const float4* __restrict__ omg_in, const float4* __restrict__ quat_in, float4* __restrict__ pos_out,
+    const float4* __restrict__ pt, const float4* __restrict__ lf, const float4* __restrict__ lt,
+    const float4* __restrict__ pos_in, const float4* __restrict__ vel_in, const float4* __restrict__ omg_in,
+    const float4* __restrict__ quat_in, float4* __restrict__ pos_out,
     float4* __restrict__ vel_out, float4* __restrict__ omg_out, float4* __restrict__ quat_out,
     uint32_t* __restrict__ keys_out, const uint32_t* __restrict__ sorted_keys, uint8_t* __restrict__ changed,
     unsigned long long* __restrict__ sbuf, uint32_t* __restrict__ append, const uint32_t* __restrict__ hwc_in,
@@ -1790,7 +1859,13 @@ __global__ __launch_bounds__(256) void k_poly_finish(
       f3 Fw, Tw;
       wall_forces_poly(P, ta, p, r, v, w, m, A, po.vbound * P.vbound_scale, Fw, Tw, tally);
       f3 Fl = mk3(0.f, 0.f, 0.f), Tl = Fl;
-      if (LIFTERS && P.num_dobj > 0) lifter_forces_poly(P, ta, p, v, w, m, A, po, Fl, Tl, tally);
+      if (LIFTERS && P.num_dobj > 0) {
+        const float4 f = lf[i];
+        if (f.w != 0.0f) {
+          Fl = Fl + xyz(f);
+          if (P.rotation) Tl = Tl + xyz(lt[i]);
+        }
+      }
       if (FORCES_ONLY) {
         fpp[3 * i] = Fpp.x; fpp[3 * i + 1] = Fpp.y; fpp[3 * i + 2] = Fpp.z;
         tpp[3 * i] = Tpp.x; tpp[3 * i + 1] = Tpp.y; tpp[3 * i + 2] = Tpp.z;
@@ -1909,10 +1984,18 @@ void launch_poly_step(const DevParams* dP, const bdem_poly_shape* dshape, const 
                       const uint32_t* sk, int ap, bool do_kill, bool want_wf, bool lifters, bool energy,
                       hipStream_t s) {
   launch_poly_forces_common(dP, dshape, b, pb, sk, energy, s);
-  /* the lifter search needs private arrays (scratch): only its own instantiation carries it */
+  if (lifters) {
+    auto lift = [&](auto kernel, int ppw) {
+      hipLaunchKernelGGL(kernel, dim3((b.n + 4 * ppw - 1) / (4 * ppw)), dim3(256), 0, s, dP, dshape, pb.hdr, b.n, pb.L,
+                         pb.rot, b.pos_srt, b.vel_srt, b.omg_srt, pb.lf, pb.lt, energy ? 1 : 0);
+    };
+    /* few particles: few per wave, so that the searches spread over the chip */
+    if (b.n <= POLY_PAIRS_SMALL) lift(k_poly_lift<2>, 2);
+    else lift(k_poly_lift<8>, 8);
+  }
   auto k = lifters ? k_poly_finish<false, true> : k_poly_finish<false, false>;
   hipLaunchKernelGGL(k, dim3((b.n + 255) / 256), dim3(256), 0, s, dP, dshape, b.n, pb.L,
-                     pb.rot, pb.hitf, pb.pf, pb.pt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, b.pos_cur,
+                     pb.rot, pb.hitf, pb.pf, pb.pt, pb.lf, pb.lt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, b.pos_cur,
                      b.vel_cur, b.omg_cur, b.quat_cur, b.keys_new, sk, b.changed, b.sbuf,
                      b.meta + META_APPEND + ap, b.hwc_srt, b.hwc_cur, want_wf ? b.wall_force : nullptr,
                      do_kill ? 1 : 0, b.status, b.kill_count, nullptr, nullptr, nullptr, nullptr, energy ? 1 : 0);
@@ -1922,7 +2005,7 @@ void launch_poly_forces(const DevParams* dP, const bdem_poly_shape* dshape, cons
                         const uint32_t* sk, float* fpp, float* tpp, float* fw, float* tw, hipStream_t s) {
   launch_poly_forces_common(dP, dshape, b, pb, sk, false, s);
   hipLaunchKernelGGL((k_poly_finish<true, false>), dim3((b.n + 255) / 256), dim3(256), 0, s, dP, dshape, b.n, pb.L,
-                     pb.rot, pb.hitf, pb.pf, pb.pt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, nullptr, nullptr,
+                     pb.rot, pb.hitf, pb.pf, pb.pt, pb.lf, pb.lt, b.pos_srt, b.vel_srt, b.omg_srt, b.quat_srt, nullptr, nullptr,
                      nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
                      b.status, b.kill_count, fpp, tpp, fw, tw, 0);
 }
