@@ -218,7 +218,8 @@ int upload_params(bdem_ctx* c) {
     HIPCHK(c, hipMemcpyAsync(c->dshape, c->shapes.data(), c->shapes.size() * sizeof(bdem_poly_shape),
                              hipMemcpyHostToDevice, c->stream));
     for (const bdem_poly_shape& s : c->shapes)
-      hdr.push_back(ShapeHdr{s.num_vertex, s.num_faces, s.num_edges, 0, s.vbound, s.plane_slack, s.radius, 0.0f});
+      hdr.push_back(ShapeHdr{(uint32_t)(s.num_vertex | s.num_faces << 8 | s.num_edges << 16), s.vbound, s.plane_slack,
+                             s.radius});
     HIPCHK(c, hipMemcpyAsync(c->pb.hdr, hdr.data(), hdr.size() * sizeof(ShapeHdr), hipMemcpyHostToDevice,
                              c->stream));
     const PolyLayout& L = c->pb.L;

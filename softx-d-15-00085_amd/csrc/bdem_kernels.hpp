@@ -63,11 +63,14 @@ struct SkinArgs {
  * contact list, its pair queue and one force/torque slot per listed pair. */
 struct PolyLayout { int pv, pf, stride; };
 /* The fields of a shape-table row that the pair tests read for every pair,
- * one 32-byte record per row (in the 3,148-byte row they lie at its start,
- * middle and end, three cache lines apart). */
-struct ShapeHdr {
-  int nv, nf, ne, pad0;
-  float vbound, plane_slack, radius, pad1;
+ * one 16-byte load (in the 3,148-byte row they lie at its start, middle and
+ * end, three cache lines apart). */
+struct alignas(16) ShapeHdr {
+  uint32_t counts;                     /* vertices | faces << 8 | edges << 16 */
+  float vbound, plane_slack, radius;
+  __host__ __device__ int nv() const { return (int)(counts & 0xFFu); }
+  __host__ __device__ int nf() const { return (int)(counts >> 8 & 0xFFu); }
+  __host__ __device__ int ne() const { return (int)(counts >> 16 & 0xFFu); }
 };
 struct PolyBuffers {
   PolyLayout L;
@@ -78,15 +81,16 @@ struct PolyBuffers {
   uint32_t* list;                      /* n * 32 partner slots */
   uint32_t* nn;                        /* full contact count per particle */
   uint2* equeue;                       /* (slot, partner) of the pairs for the wave-per-pair kernel, POLY_SUBQ parts */
-  uint32_t* qcount;                    /* POLY_QCOUNTS counters, POLY_QSTRIDE words apart: the parts' lengths, then
-                                          the wave-per-pair kernel's slice counters */
+  uint32_t* qcount;                    /* POLY_QCOUNTS counters, POLY_QSTRIDE words apart: the parts' lengths, the
+                                          wave-per-pair kernel's slice counters, the overflow word */
   uint8_t* hitf;                       /* n * 32: 1 where the slot's pair is in contact */
   float4 *pf, *pt;                     /* n * 32: pair force, torque, where hitf is set */
   float4 *lf, *lt;                     /* n: lifter force (w = 1 when in contact), torque */
   uint2* hint;                         /* n * 32 by P_ID and list slot: (partner P_ID, separating face code) */
 };
 constexpr int POLY_SUBQ = 64, POLY_SLICES = 8;
-constexpr int POLY_QCOUNTS = POLY_SUBQ + POLY_SLICES, POLY_QSTRIDE = 32;   /* a counter per 128-byte line */
+constexpr int POLY_OVERFLOW = POLY_SUBQ + POLY_SLICES;   /* word: some list of this step overflowed */
+constexpr int POLY_QCOUNTS = POLY_OVERFLOW + 1, POLY_QSTRIDE = 32;   /* a counter per 128-byte line */
 /* Particles per block of the separating-plane kernel.  Up to
  * POLY_PAIRS_SMALL particles the smaller blocks spread them over the CUs. */
 constexpr int POLY_PPB = 128, POLY_PPB_SMALL = 16, POLY_PAIRS_SMALL = 16384;

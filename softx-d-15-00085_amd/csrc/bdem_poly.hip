@@ -79,7 +79,7 @@ __device__ __forceinline__ Shape shape_of(const float4* __restrict__ rot, const 
 __device__ __forceinline__ Shape shape_of(const float4* __restrict__ rot, const PolyLayout& L, int i,
                                           const ShapeHdr& h) {
   const float4* base = rot + (size_t)i * L.stride;
-  return Shape{base, base + L.pv, base + L.pv + L.pf, h.nv, h.nf};
+  return Shape{base, base + L.pv, base + L.pv + L.pf, h.nv(), h.nf()};
 }
 
 /* Face f; f = -1 (no face of B had A's centre in front) is a zero plane. */
@@ -1214,12 +1214,16 @@ __global__ __launch_bounds__(256) void k_poly_rotate(const DevParams* __restrict
  * its slots' contact marks cleared. */
 template <int G>
 __device__ __forceinline__ void list_store(int i, bool in, int c, const uint32_t* mine, uint32_t* __restrict__ list32,
-                                           uint32_t* __restrict__ nn, uint8_t* __restrict__ hitf, uint32_t* status) {
+                                           uint32_t* __restrict__ nn, uint8_t* __restrict__ hitf, uint32_t* qcount,
+                                           uint32_t* status) {
   if (!in) return;
   const int sub = threadIdx.x & (G - 1);
   if (sub == 0) {
     nn[i] = (uint32_t)c;
-    if (c > LIST_STRIDE) atomicOr(status, ST_LIST_OVERFLOW);
+    if (c > LIST_STRIDE) {
+      atomicOr(status, ST_LIST_OVERFLOW);
+      qcount[POLY_OVERFLOW * POLY_QSTRIDE] = 1u;
+    }
   }
   const int m = min(c, LIST_STRIDE);
   for (int k = sub; k < m; k += G) list32[(size_t)i * LIST_STRIDE + k] = mine[k];
@@ -1244,7 +1248,8 @@ __global__ __launch_bounds__(256) void k_poly_list(const DevParams* __restrict__
                                                    const float4* __restrict__ pos_r,
                                                    const float4* __restrict__ omg,
                                                    uint32_t* __restrict__ list32, uint32_t* __restrict__ nn,
-                                                   uint8_t* __restrict__ hitf, uint32_t* status) {
+                                                   uint8_t* __restrict__ hitf, uint32_t* qcount,
+                                                   uint32_t* status) {
   const DevParams& P = *Pp;
   __shared__ uint32_t cand[4][LIST_NP][LIST_CAND];
   __shared__ uint32_t list[4][LIST_NP][LIST_STRIDE];
@@ -1260,20 +1265,21 @@ __global__ __launch_bounds__(256) void k_poly_list(const DevParams* __restrict__
                                                    if (k < LIST_STRIDE) mine[k] = (uint32_t)j;
                                                  });
   __builtin_amdgcn_wave_barrier();
-  list_store<LIST_G>(i, in, c, mine, list32, nn, hitf, status);
+  list_store<LIST_G>(i, in, c, mine, list32, nn, hitf, qcount, status);
 }
 
 /* The same list for larger counts, two lanes per particle and 32 particles
  * per wave: the gathers of k_poly_list are bound by their addresses there.
- * The wave stages the three rows of one y layer (cells, then candidates) by
- * coalesced loads into LDS; a particle's two lanes test one half each of a
+ * The wave loads the three rows of one y layer (cells, then candidates) by
+ * coalesced loads and stages a row at a time in LDS; a particle's two lanes test one half each of a
  * row's candidates into a bit mask, and the masks' set bits, the first
- * half's before the second's, are the contacts in order. */
+ * half's before the second's, are the contacts in order.  75 us at 200,000
+ * hulls (137 for one lane per particle); 111 while a row's stage held only 80
+ * candidates and the dense rows read global memory. */
 constexpr int LIST_TEAM_MAX = 24576;
-constexpr int LIST2_POS = 80;
 struct ListStage {
-  float4 pos[3][LIST2_POS];
-  uint2 cell[3][64];
+  float4 pos[STAGE_POS];
+  uint2 cell[64];
   uint32_t list[32][LIST_STRIDE + 1];   /* odd stride: both lanes of 32 particles write it */
 };
 constexpr int LIST2_WAVES = 4, LIST2_BLOCK = 32 * LIST2_WAVES;
@@ -1284,7 +1290,8 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
                                                                  const uint32_t* __restrict__ sorted_keys,
                                                                  uint32_t* __restrict__ list32,
                                                                  uint32_t* __restrict__ nn,
-                                                                 uint8_t* __restrict__ hitf, uint32_t* status) {
+                                                                 uint8_t* __restrict__ hitf, uint32_t* qcount,
+                                                   uint32_t* status) {
   const DevParams& P = *Pp;
   __shared__ ListStage stage[LIST2_WAVES];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1323,23 +1330,20 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
     for (int z = 0; z < 3; ++z) {
       const RowStage rs = row_stage(ce[z], none, (uint32_t)n);
       pmin[z] = rs.pmin;
-      pcnt[z] = rs.any && rs.pmax - rs.pmin <= (uint32_t)LIST2_POS ? rs.pmax - rs.pmin : 0u;
+      pcnt[z] = rs.staged ? rs.pmax - rs.pmin : 0u;
       q0[z] = make_float4(0.f, 0.f, 0.f, 0.f);
       q1[z] = q0[z];
       if ((uint32_t)lane < pcnt[z]) q0[z] = pos_r[pmin[z] + lane];
       if ((uint32_t)lane + 64u < pcnt[z]) q1[z] = pos_r[pmin[z] + 64u + lane];
     }
-    __builtin_amdgcn_wave_barrier();   /* the previous layer's reads are done */
-#pragma unroll
-    for (int z = 0; z < 3; ++z) {
-      st.cell[z][lane] = ce[z];
-      st.pos[z][lane] = q0[z];
-      if (lane + 64 < LIST2_POS) st.pos[z][lane + 64] = q1[z];
-    }
-    __builtin_amdgcn_wave_barrier();
     const uint32_t y = (uint32_t)g[1] + (uint32_t)dy - 1u;
 #pragma unroll
     for (int z = 0; z < 3; ++z) {
+      __builtin_amdgcn_wave_barrier();   /* the previous row's reads are done */
+      st.cell[lane] = ce[z];
+      st.pos[lane] = q0[z];
+      st.pos[lane + 64] = q1[z];
+      __builtin_amdgcn_wave_barrier();
       const uint32_t zz = (uint32_t)g[2] + (uint32_t)z - 1u;
       uint32_t lo = 0u, cnt = 0u;
       if (live && xs <= xe && y < (uint32_t)P.ny && zz < (uint32_t)P.nz) {
@@ -1347,7 +1351,7 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
         if (h1 < P.C) {   /* at most three cells, first and last occupied entry */
           uint2 c0 = none, c1 = none, c2 = none;
           if (narrow && h0 >= w[z].w0 && h1 < w[z].w0 + w[z].wn) {
-            const uint2* const row = st.cell[z] - w[z].w0;
+            const uint2* const row = st.cell - w[z].w0;
             c0 = row[h0];
             if (h0 + 1u <= h1) c1 = row[h0 + 1u];
             if (h0 + 2u <= h1) c2 = row[h0 + 2u];
@@ -1374,7 +1378,7 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
         if (__all((int)(staged || len == 0u))) {
           /* four reads in flight; past the end the last entry is read again */
           const uint32_t at = j0 - pmin[z], last = len ? len - 1u : 0u;
-          const float4* const src = st.pos[z] + (len ? at : 0u);
+          const float4* const src = st.pos + (len ? at : 0u);
           for (uint32_t t = 0u; t < len; t += 4u) {
             float4 pb[4];
 #pragma unroll
@@ -1403,7 +1407,7 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
     }
   }
   __builtin_amdgcn_wave_barrier();
-  list_store<2>(i, in, count, mine, list32, nn, hitf, status);
+  list_store<2>(i, in, count, mine, list32, nn, hitf, qcount, status);
 }
 
 /* Whether particle i is among the listed contacts of j. */
@@ -1425,7 +1429,8 @@ __device__ __forceinline__ bool is_listed(const uint32_t* __restrict__ list32, i
  * (1,172 more of them added 12 us to a launch): 35,700 per launch held an
  * earlier form of this kernel at 457 us for 200,000 hulls.  Here a block
  * makes one, in one of POLY_SUBQ counters, each with its own part of the
- * queue. */
+ * queue.  Now 132 us, bound by the address rate of its per-lane loads (a
+ * pair's face, vertices and headers lie in lines of their own). */
 template <int PPB>
 __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict__ Pp,
                                                     const ShapeHdr* __restrict__ hdr, int n, PolyLayout L,
@@ -1472,14 +1477,42 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
   };
   if (threadIdx.x == 0) { nitems = 0u; nleft = 0u; nout = 0u; }
   __syncthreads();
-  for (uint32_t e = threadIdx.x; e < (uint32_t)(PPB * LIST_STRIDE); e += 256u) {
-    const int i = base + (int)(e / LIST_STRIDE), k = (int)(e % LIST_STRIDE);
-    bool want = false;
-    if (i < n && (uint32_t)k < min(nn[i], (uint32_t)LIST_STRIDE)) {
-      const int j = (int)list32[(size_t)i * LIST_STRIDE + k];
-      want = j > i || (nn[j] > (uint32_t)LIST_STRIDE && !is_listed(list32, j, (uint32_t)i));
+  /* two threads a particle, 16 list entries each in four loads; nn of the
+   * partners is needed only in a step where some list overflowed */
+  const bool over = qcount[POLY_OVERFLOW * POLY_QSTRIDE] != 0u;
+  for (int t0 = 0; t0 < 2 * PPB; t0 += 256) {
+    const int t = t0 + (int)threadIdx.x, i = base + (t >> 1), k0 = (t & 1) * (LIST_STRIDE / 2);
+    int m = 0;
+    if (t < 2 * PPB && i < n) m = (int)min(nn[i], (uint32_t)LIST_STRIDE) - k0;
+    uint32_t js[LIST_STRIDE / 2];
+#pragma unroll
+    for (int q = 0; q < LIST_STRIDE / 8; ++q) {
+      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+      if (4 * q < m) v = *reinterpret_cast<const uint4*>(list32 + (size_t)i * LIST_STRIDE + k0 + 4 * q);
+      js[4 * q] = v.x; js[4 * q + 1] = v.y; js[4 * q + 2] = v.z; js[4 * q + 3] = v.w;
     }
-    push(items, &nitems, want, e);
+    uint32_t want = 0u;
+#pragma unroll
+    for (int q = 0; q < LIST_STRIDE / 2; ++q) {
+      bool w = q < m && js[q] > (uint32_t)i;
+      if (over && q < m && !w) w = nn[js[q]] > (uint32_t)LIST_STRIDE && !is_listed(list32, (int)js[q], (uint32_t)i);
+      want |= (w ? 1u : 0u) << q;
+    }
+    const int own = __popc(want);
+    int incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    uint32_t at = 0u;
+    if (lane == 63) at = atomicAdd(&nitems, (uint32_t)incl);
+    at = (uint32_t)__builtin_amdgcn_readlane((int)at, 63) + (uint32_t)(incl - own);
+    while (want) {
+      const int q = __ffs(want) - 1;
+      want &= want - 1u;
+      items[at++] = (uint16_t)((t >> 1) * LIST_STRIDE + k0 + q);
+    }
   }
   __syncthreads();
   const uint32_t cnt = nitems;
@@ -1549,7 +1582,8 @@ struct PairStage {
  * searches read LDS instead of chains of dependent global loads.  The inside
  * tests and the edge search are the same for the contact of A with B and of
  * B with A (vertex_faces_both, edges_wave); done once per pair instead of
- * once per listed contact they halve the launch's work.
+ * once per listed contact they halve the launch's work (517 -> 240 us at
+ * 200,000 hulls, VALU issue bound).
  *
  * A wave's first chunk is its own by its number: the first half of the
  * queue (all of it while it has a pair per wave at most).  The rest is dealt
@@ -1667,8 +1701,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
       /* A's place in B's list (absent when that list overflowed) */
       const uint32_t at = (uint32_t)__ballot(!h && (uint32_t)k < nback && back == slot / LIST_STRIDE);
       const uint32_t slot_b = at ? partner * LIST_STRIDE + (uint32_t)(__ffs(at) - 1) : NO_SLOT;
-      const Shape A{S.v[0], S.fn[0], S.fc[0], ha.nv, ha.nf, S.vo[0], S.area[0], S.fnv[0]};
-      const Shape B{S.v[1], S.fn[1], S.fc[1], hb.nv, hb.nf, S.vo[1], S.area[1], S.fnv[1]};
+      const Shape A{S.v[0], S.fn[0], S.fc[0], ha.nv(), ha.nf(), S.vo[0], S.area[0], S.fnv[0]};
+      const Shape B{S.v[1], S.fn[1], S.fc[1], hb.nv(), hb.nf(), S.vo[1], S.area[1], S.fnv[1]};
       const PairDirs D = pair_dirs(A, B, o.PosA, o.PosB);
       const uint32_t code = separated_wave(A, B, o.PosA, o.PosB, D);
       PColl c{false, C_SP, 0.0f, mk3(0.f, 0.f, 0.f), mk3(0.f, 0.f, 0.f)};   /* lanes 0-31: A's, 32-63: B's */
@@ -1683,7 +1717,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
         if (vertex_faces_both(o.PosA, A, o.PosB, B, D, ab, ba)) {
           c = h ? ba : ab;
         } else {
-          c = edges_wave(A, S.e[0], ha.ne, B, S.e[1], hb.ne, o.PosA, o.PosB, vbA, vbB,
+          c = edges_wave(A, S.e[0], ha.ne(), B, S.e[1], hb.ne(), o.PosA, o.PosB, vbA, vbB,
                          ha.plane_slack * P.vbound_scale, hb.plane_slack * P.vbound_scale, S.ia, S.ib, D.fA, D.fB);
           if (c.hit) c.dis = fminf(0.025f * (h ? hb : ha).radius, c.dis);
         }
@@ -1778,7 +1812,7 @@ __global__ __launch_bounds__(256) void k_poly_lift(const DevParams* __restrict__
     __builtin_amdgcn_wave_barrier();   /* the previous particle's reads are done */
     if (lane < BDEM_SHAPE_MAX_VERTEX) verts[wave][lane] = ra[lane < L.pv ? lane : 0];
     __builtin_amdgcn_wave_barrier();
-    const Shape A{verts[wave], ra + L.pv, ra + L.pv + L.pf, hd.nv, hd.nf};
+    const Shape A{verts[wave], ra + L.pv, ra + L.pv + L.pf, hd.nv(), hd.nf()};
     while (ds) {
       const int d = __ffs(ds) - 1;
       ds &= ds - 1u;
@@ -1954,10 +1988,10 @@ static void launch_poly_forces_common(const DevParams* dP, const bdem_poly_shape
    * against 20 us at 50,000 */
   if (b.n <= LIST_TEAM_MAX)
     hipLaunchKernelGGL(k_poly_list, dim3((b.n + LIST_BLOCK - 1) / LIST_BLOCK), dim3(256), 0, s, dP, b.n, b.cells,
-                       b.pos_srt, b.omg_srt, pb.list, pb.nn, pb.hitf, b.status);
+                       b.pos_srt, b.omg_srt, pb.list, pb.nn, pb.hitf, pb.qcount, b.status);
   else
     hipLaunchKernelGGL(k_poly_list2, dim3((b.n + LIST2_BLOCK - 1) / LIST2_BLOCK), dim3(64 * LIST2_WAVES), 0, s, dP,
-                       b.n, b.cells, b.pos_srt, b.omg_srt, sk, pb.list, pb.nn, pb.hitf, b.status);
+                       b.n, b.cells, b.pos_srt, b.omg_srt, sk, pb.list, pb.nn, pb.hitf, pb.qcount, b.status);
   const uint32_t subcap = poly_subqueue_capacity(b.n);
   auto pairs = [&](auto kernel, int ppb) {
     hipLaunchKernelGGL(kernel, dim3((b.n + ppb - 1) / ppb), dim3(256), 0, s, dP, pb.hdr, b.n, pb.L, pb.rot, b.pos_srt,
