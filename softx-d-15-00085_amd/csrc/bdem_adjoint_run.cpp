@@ -9,9 +9,10 @@
  * writes per-block moments of the state, summed on the host in block order.
  *
  * Backward: for each segment, last first, the checkpoint is restored and
- * the segment re-run with the step kernel writing its contact lists; after
- * each step its sorted input state and sort permutation are copied into the
- * segment's store.  Then the adjoint kernels run over the segment's steps
+ * the segment re-run with the step kernel writing its contact lists, and
+ * with the sort writing each step's sorted input state and permutation
+ * straight into the segment's store (copying them out after every step took
+ * four copies of about 4 us each, and more on the host).  Then the adjoint kernels run over the segment's steps
  * in reverse, carrying the state cotangent (three float4 per slot) from
  * each step's output order to its input order.
  */
@@ -321,27 +322,36 @@ int bdem_adj_backward(bdem_adjoint* A, const double* cot, double* dtheta) {
   float4* lam_cur = A->lam_a;
   float4* lam_nxt = A->lam_b;
   int rc = BDEM_OK;
-  /* the step kernel writes its contact lists only while these are set */
-  struct Unrecord {
+  /* the step kernel writes its contact lists, and the sort into the segment's
+   * store, only while these are set */
+  struct Record {
     bdem_ctx* c;
-    ~Unrecord() { c->dbg_list = nullptr; c->dbg_nn = nullptr; }
-  } unrecord{c};
+    float4 *pos, *vel, *omg;
+    int* idx;
+    explicit Record(bdem_ctx* x)
+        : c(x), pos(x->b.pos_srt), vel(x->b.vel_srt), omg(x->b.omg_srt), idx(x->b.idx_sorted) {}
+    void off() {
+      c->dbg_list = nullptr;
+      c->dbg_nn = nullptr;
+      c->b.pos_srt = pos;
+      c->b.vel_srt = vel;
+      c->b.omg_srt = omg;
+      c->b.idx_sorted = idx;
+    }
+    ~Record() { off(); }
+  } record{c};
   for (int seg = A->nseg - 1; seg >= 0 && rc == BDEM_OK; --seg) {
     rc = restore(A, A->ckpt + (size_t)seg * 3 * n);
     for (int t = 0; t < A->every && rc == BDEM_OK; ++t) {
       c->dbg_list = A->slist + (size_t)t * n * LIST_STRIDE;
       c->dbg_nn = A->snn + (size_t)t * n;
+      c->b.pos_srt = A->spos + (size_t)t * n;
+      c->b.vel_srt = A->svel + (size_t)t * n;
+      c->b.omg_srt = A->somg + (size_t)t * n;
+      c->b.idx_sorted = A->sidx + (size_t)t * n;
       rc = step_ctx(A);
-      if (rc != BDEM_OK) break;
-      const size_t bytes = n * sizeof(float4);
-      AHIP(A, hipMemcpyAsync(A->spos + (size_t)t * n, c->b.pos_srt, bytes, hipMemcpyDeviceToDevice, c->stream));
-      AHIP(A, hipMemcpyAsync(A->svel + (size_t)t * n, c->b.vel_srt, bytes, hipMemcpyDeviceToDevice, c->stream));
-      AHIP(A, hipMemcpyAsync(A->somg + (size_t)t * n, c->b.omg_srt, bytes, hipMemcpyDeviceToDevice, c->stream));
-      AHIP(A, hipMemcpyAsync(A->sidx + (size_t)t * n, c->b.idx_sorted, n * sizeof(int), hipMemcpyDeviceToDevice,
-                             c->stream));
     }
-    c->dbg_list = nullptr;
-    c->dbg_nn = nullptr;
+    record.off();
     for (int t = A->every - 1; t >= 0 && rc == BDEM_OK; --t) {
       const int s = seg * A->every + t;
       AdjStep st{A->n, A->spos + (size_t)t * n, A->svel + (size_t)t * n, A->somg + (size_t)t * n,
