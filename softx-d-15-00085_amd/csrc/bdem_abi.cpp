@@ -567,13 +567,14 @@ hipEvent_t* timing_slot(bdem_ctx* c) {
 
 /* hash (if needed) + sort + gather + cells: the sorted scratch state.
  * On return b.keys_sorted[c->sorted_par] and b.idx_sorted hold the order. */
-int prepare_sorted(bdem_ctx* c, hipEvent_t* ev = nullptr) {
+int prepare_sorted(bdem_ctx* c, hipEvent_t* ev = nullptr, const TurnArgs& turn = TurnArgs{}) {
   if (ev) (void)hipEventRecord(ev[0], c->stream);
   const bool incremental = c->keys_valid && c->flags_valid && !c->full_next;
   if (!c->keys_valid) launch_hash(c->dp, c->b, c->stream);
   const int prev = c->sorted_par;
   const int next = incremental ? prev ^ 1 : prev;
   SortArgs a{};
+  a.turn = turn;
   const StepBuffers& b = c->b;
   a.n = b.n;
   a.C = c->hp.C;
@@ -1387,13 +1388,13 @@ int bdem_update_sim(bdem_ctx* c) {
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
   hipEvent_t* ev = timing_slot(c);
+  TurnArgs turn{};
   if (c->lift_on && !c->dobj.empty()) {
     /* UpdateSim turns the lifters before the step (main.cpp:114-121) */
-    launch_turn_lifters(c->dp, c->lift_c, c->lift_s, c->lift_about[0], c->lift_about[1], c->lift_about[2],
-                        c->stream);
+    turn = TurnArgs{c->dp, c->lift_c, c->lift_s, {c->lift_about[0], c->lift_about[1], c->lift_about[2]}};
     c->dobj_dirty = true;
   }
-  if ((rc = prepare_sorted(c, ev)) != BDEM_OK) return rc;
+  if ((rc = prepare_sorted(c, ev, turn)) != BDEM_OK) return rc;
   bool do_kill = false;
   if (c->sim.Kill_Particles) {
     const int interval = (c->has_ext && c->ext.kill_check_interval > 0) ? c->ext.kill_check_interval : 1000;

@@ -117,8 +117,18 @@ inline __host__ __device__ int sort_blocks(int n) { return (n + SORT_TILE - 1) /
 int key_bits(uint32_t max_key);
 int sort_passes(uint32_t max_key);
 
+/* Rotate_VolObject_Inc on the device: every lifter attached to the drum in
+ * the parameter block (null: no turn) turned by the angle whose cosine and
+ * sine are c, s about `about`, its faces re-derived. */
+struct TurnArgs {
+  DevParams* params;
+  double c, s;
+  float about[3];
+};
+
 /* Everything the sort kernels touch for one step. */
 struct SortArgs {
+  TurnArgs turn;                       /* the lifters' turn before this step, made beside the sort */
   int n;
   uint32_t C;
   int passes;
@@ -192,10 +202,8 @@ void launch_step_team_batch(const BatchLaunch& L, const StepBuffers& b, const ui
                             int append_par, hipStream_t s);
 void launch_step_batch(const BatchLaunch& L, const StepBuffers& b, const uint32_t* sorted_keys, int hist_par,
                        int append_par, hipStream_t s);
-/* Rotate_VolObject_Inc on the device: every lifter attached to the drum in
- * the parameter block turned by the angle whose cosine and sine are c, s
- * about (ax, ay, az), its faces re-derived.  One small launch. */
-void launch_turn_lifters(DevParams* dP, double c, double s, float ax, float ay, float az, hipStream_t st);
+/* The turn as a launch of its own (launch_sort makes it beside a full sort). */
+void launch_turn_lifters(const TurnArgs& t, hipStream_t st);
 /* Skin masks before a step: decide a new epoch (every row tested in full)
  * from the displacement bound, else flag the stencil rows whose cells a
  * particle entered or left.  Uses this step's cell table; par alternates. */

@@ -39,7 +39,7 @@
  * host runs it on the first step after an upload and after a discharge
  * check, when many particles change key at once.
  */
-#include "bdem_kernels.hpp"
+#include "bdem_turn.hpp"
 
 
 namespace bdem {
@@ -188,6 +188,11 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
   __shared__ unsigned long long s_wlo, s_whi, s_upred, s_maxb, s_mina;
   __shared__ uint32_t s_below, s_chgb, s_nl, s_n2, s_ncand;
 
+  static_assert(T >= TURN_THREADS && sizeof(Ls) >= TURN_THREADS * sizeof(bdem_float3), "room for the lifters' turn");
+  if (a.turn.params && blockIdx.x == gridDim.x - 1) {   /* the block past the tiles */
+    turn_lifters_block(a.turn.params, a.turn, reinterpret_cast<bdem_float3*>(Ls));
+    return;
+  }
   const int n = a.n;
   const uint32_t C = a.C;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -616,10 +621,12 @@ static hipError_t launch_full_sort(const SortArgs& a, int par, hipStream_t s) {
 
 hipError_t launch_sort(const SortArgs& a, bool incremental, int par, hipStream_t s) {
   if (incremental) {
-    if (a.n <= RS_SMALL) hipLaunchKernelGGL(k_resort<256>, dim3((a.n + 255) / 256), dim3(256), 0, s, a, par);
-    else hipLaunchKernelGGL(k_resort<512>, dim3((a.n + 511) / 512), dim3(512), 0, s, a, par);
+    const int extra = a.turn.params ? 1 : 0;
+    if (a.n <= RS_SMALL) hipLaunchKernelGGL(k_resort<256>, dim3((a.n + 255) / 256 + extra), dim3(256), 0, s, a, par);
+    else hipLaunchKernelGGL(k_resort<512>, dim3((a.n + 511) / 512 + extra), dim3(512), 0, s, a, par);
     return hipGetLastError();
   }
+  if (a.turn.params) launch_turn_lifters(a.turn, s);
   return launch_full_sort(a, par, s);
 }
 
