@@ -450,11 +450,26 @@ int require(bdem_ctx* c) {
   return BDEM_OK;
 }
 
+/* The sorted scratch streams as the caller's arrays: they hold nothing
+ * between steps (the next sort writes them). */
+StateArrays scratch_arrays(bdem_ctx* c) {
+  const StepBuffers& b = c->b;
+  const size_t n = (size_t)b.n;
+  StateArrays a{};
+  a.pos = reinterpret_cast<bdem_float3*>(b.pos_srt);
+  a.ptype = reinterpret_cast<unsigned*>(a.pos + n);
+  a.vel = reinterpret_cast<bdem_float3*>(b.vel_srt);
+  a.pid = reinterpret_cast<int*>(a.vel + n);
+  a.avel = reinterpret_cast<bdem_float3*>(b.omg_srt);
+  a.quat = reinterpret_cast<bdem_Quaterion*>(b.quat_srt);
+  return a;
+}
+
 /* Host AoS -> device float4 streams.  Radius and mass come from the type
  * table (the reference's only source) unless per-particle values exist. */
 int upload_state(bdem_ctx* c, const bdem_float3* pos, const bdem_Quaterion* ornt,
                  const bdem_float3* vel, const bdem_float3* avel, const unsigned int* ptype,
-                 const int* pid, bool keep_vel) {
+                 const int* pid) {
   const int n = c->b.n;
   /* every check before the first copy: a rejected upload leaves the state,
    * keys and flags of the previous one untouched */
@@ -491,45 +506,24 @@ int upload_state(bdem_ctx* c, const bdem_float3* pos, const bdem_Quaterion* ornt
                           double(ornt[i].y) * ornt[i].y + double(ornt[i].z) * ornt[i].z;
         qscale = std::max(qscale, s2 * (1.0 + 1e-6));
       }
-  std::vector<float4> P(n), V(n), O(n), Q;
-  std::vector<float4> oldP, oldV, oldO;
-  if (keep_vel || c->hp.per_particle) {
-    oldP.resize(n); oldV.resize(n); oldO.resize(n);
-    HIPCHK(c, hipMemcpy(oldP.data(), c->b.pos_cur, n * sizeof(float4), hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(oldV.data(), c->b.vel_cur, n * sizeof(float4), hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(oldO.data(), c->b.omg_cur, n * sizeof(float4), hipMemcpyDeviceToHost));
-  }
-  for (int i = 0; i < n; ++i) {
-    const unsigned t = ptype[i];
-    float r = c->hp.per_particle ? oldP[i].w : c->pobj[t].radius;
-    float m = c->hp.per_particle ? oldV[i].w : c->pobj[t].mass;
-    if (c->shape_by_pid) {   /* per-particle shapes carry their own radius and mass */
-      const bdem_poly_shape& sh = c->shapes[pid[i] > 0 ? pid[i] : 0];
-      r = sh.radius;
-      m = sh.mass;
-    }
-    P[i] = make_float4(pos[i].x, pos[i].y, pos[i].z, r);
-    if (vel) V[i] = make_float4(vel[i].x, vel[i].y, vel[i].z, m);
-    else V[i] = make_float4(oldV[i].x, oldV[i].y, oldV[i].z, m);
-    if (avel) O[i] = make_float4(avel[i].x, avel[i].y, avel[i].z, bits_f(pack_id_type(pid[i], t)));
-    else O[i] = make_float4(oldO[i].x, oldO[i].y, oldO[i].z, bits_f(pack_id_type(pid[i], t)));
-  }
   /* from here on the device state changes: whatever happens, the next step
    * re-hashes and fully re-sorts */
   c->keys_valid = false;
   c->flags_valid = false;
   c->lists_full = true;
-  HIPCHK(c, hipMemcpy(c->b.pos_cur, P.data(), n * sizeof(float4), hipMemcpyHostToDevice));
-  HIPCHK(c, hipMemcpy(c->b.vel_cur, V.data(), n * sizeof(float4), hipMemcpyHostToDevice));
-  HIPCHK(c, hipMemcpy(c->b.omg_cur, O.data(), n * sizeof(float4), hipMemcpyHostToDevice));
-  if (c->orient) {
-    Q.resize(n);
-    for (int i = 0; i < n; ++i) {
-      if (ornt && !c->sim.sphere_orient) Q[i] = make_float4(ornt[i].w, ornt[i].x, ornt[i].y, ornt[i].z);
-      else Q[i] = make_float4(1.f, 0.f, 0.f, 0.f);  /* Set_Pos: identity for sphere_orient */
-    }
-    HIPCHK(c, hipMemcpy(c->b.quat_cur, Q.data(), n * sizeof(float4), hipMemcpyHostToDevice));
-  }
+  const StateArrays d = scratch_arrays(c);
+  const bool quat = c->orient && ornt && !c->sim.sphere_orient;
+  const size_t v3 = (size_t)n * sizeof(bdem_float3), w1 = (size_t)n * sizeof(int);
+  using Region = HostStage::Region;
+  auto in = [](const void* p) { return const_cast<void*>(p); };
+  std::vector<Region> r{Region{(char*)d.pos, in(pos), v3, in(ptype), w1}, Region{(char*)d.vel, in(vel), v3, in(pid), w1}};
+  if (avel) r.push_back(Region{(char*)d.avel, in(avel), v3, nullptr, 0});
+  if (quat) r.push_back(Region{(char*)d.quat, in(ornt), (size_t)n * sizeof(bdem_Quaterion), nullptr, 0});
+  HIPCHK(c, c->stage.to_device(r, c->stream));
+  const UnpackMode m{vel ? 1 : 0, avel ? 1 : 0, quat ? 1 : 0, c->hp.per_particle, c->shape_by_pid ? 1 : 0};
+  launch_unpack_state(c->dp, c->b, d, m, c->dshape, c->orient, c->stream);
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   if (c->b.hwc_cur) {   /* spring counts and lifter contact types restart */
     launch_fill_u32(c->b.hwc_cur, c->b.n, 0u, c->stream);
     launch_fill_u32(c->b.hwc_srt, c->b.n, 0u, c->stream);
@@ -891,7 +885,7 @@ int bdem_set_pos(bdem_ctx* c, const bdem_float3* pos, const bdem_Quaterion* ornt
   if (!pos || !ptype || !pid) return fail(c, BDEM_EINVAL, "null argument");
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  return upload_state(c, pos, ornt, nullptr, nullptr, ptype, pid, true);
+  return upload_state(c, pos, ornt, nullptr, nullptr, ptype, pid);
 }
 
 int bdem_set_pos_velocity(bdem_ctx* c, const bdem_float3* pos, const bdem_Quaterion* ornt,
@@ -902,7 +896,7 @@ int bdem_set_pos_velocity(bdem_ctx* c, const bdem_float3* pos, const bdem_Quater
   if (!pos || !vel || !avel || !ptype || !pid) return fail(c, BDEM_EINVAL, "null argument");
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  return upload_state(c, pos, ornt, vel, avel, ptype, pid, false);
+  return upload_state(c, pos, ornt, vel, avel, ptype, pid);
 }
 
 int bdem_set_system_state(bdem_ctx* c, const bdem_float3* pos, const bdem_Quaterion* ornt,
@@ -920,16 +914,17 @@ int bdem_set_radii(bdem_ctx* c, const float* radius, const float* mass) {
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   const int n = c->b.n;
-  std::vector<float4> P(n), V(n);
-  HIPCHK(c, hipMemcpy(P.data(), c->b.pos_cur, n * sizeof(float4), hipMemcpyDeviceToHost));
-  HIPCHK(c, hipMemcpy(V.data(), c->b.vel_cur, n * sizeof(float4), hipMemcpyDeviceToHost));
-  for (int i = 0; i < n; ++i) {
+  for (int i = 0; i < n; ++i)
     if (!(radius[i] > 0.f) || !(mass[i] > 0.f)) return fail(c, BDEM_EINVAL, "radius and mass must be positive");
-    P[i].w = radius[i];
-    V[i].w = mass[i];
-  }
-  HIPCHK(c, hipMemcpy(c->b.pos_cur, P.data(), n * sizeof(float4), hipMemcpyHostToDevice));
-  HIPCHK(c, hipMemcpy(c->b.vel_cur, V.data(), n * sizeof(float4), hipMemcpyHostToDevice));
+  using Region = HostStage::Region;
+  float *dr = reinterpret_cast<float*>(c->b.pos_srt), *dm = reinterpret_cast<float*>(c->b.vel_srt);
+  const size_t w1 = (size_t)n * sizeof(float);
+  const std::vector<Region> r{Region{(char*)dr, const_cast<float*>(radius), w1, nullptr, 0},
+                              Region{(char*)dm, const_cast<float*>(mass), w1, nullptr, 0}};
+  HIPCHK(c, c->stage.to_device(r, c->stream));
+  launch_set_radii(c->b, dr, dm, c->stream);
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   c->lists_full = true;   /* list membership depends on the radii */
   return BDEM_OK;
 }
@@ -950,27 +945,17 @@ int bdem_get_system_state(bdem_ctx* c, bdem_float3* pos, bdem_Quaterion* ornt, b
   int rc = require(c);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  std::vector<float4> P, V, O, Q;
-  if ((rc = download(c, P, V, O, Q)) != BDEM_OK) return rc;
-  for (int i = 0; i < c->b.n; ++i) {
-    if (pos) {
-      pos[i] = bdem_float3{P[i].x, P[i].y, P[i].z};
-      const int row = shape_row(c, f_bits(O[i].w));
-      if (c->poly && row >= 0) {
-        /* Get_SystemState / Get_Particle_PosArray return position - COM for
-         * polyhedra (GPU_Memory_Transfer.cuh:461, 504) */
-        const bdem_float3 cm = c->shapes[row].COM;
-        pos[i] = bdem_float3{P[i].x - cm.x, P[i].y - cm.y, P[i].z - cm.z};
-      }
-    }
-    if (vel) vel[i] = bdem_float3{V[i].x, V[i].y, V[i].z};
-    if (avel) avel[i] = bdem_float3{O[i].x, O[i].y, O[i].z};
-    if (acc) acc[i] = bdem_float3{0.f, 0.f, 0.f};
-    const int packed = f_bits(O[i].w);
-    if (ptype) ptype[i] = (unsigned)(packed & 7);
-    if (pid) pid[i] = packed >> 3;
-    if (ornt && c->orient) ornt[i] = bdem_Quaterion{Q[i].x, Q[i].y, Q[i].z, Q[i].w};
-  }
+  const size_t n = (size_t)c->b.n, v3 = n * sizeof(bdem_float3), w1 = n * sizeof(int);
+  const StateArrays d = scratch_arrays(c);
+  launch_pack_state(c->b, c->poly ? c->dshape : nullptr, (int)c->shapes.size(), c->shape_by_pid, c->orient, d,
+                    c->stream);
+  HIPCHK(c, hipGetLastError());
+  using Region = HostStage::Region;
+  std::vector<Region> r{Region{(char*)d.pos, pos, v3, ptype, w1}, Region{(char*)d.vel, vel, v3, pid, w1},
+                        Region{(char*)d.avel, avel, v3, nullptr, 0}};
+  if (c->orient) r.push_back(Region{(char*)d.quat, ornt, n * sizeof(bdem_Quaterion), nullptr, 0});
+  HIPCHK(c, c->stage.to_host(r, c->stream));
+  if (acc) std::memset(acc, 0, v3);
   return BDEM_OK;
 }
 

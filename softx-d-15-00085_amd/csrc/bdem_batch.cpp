@@ -67,6 +67,8 @@ struct bdem_batch {
 
   bool keys_valid = false;        /* false: the next step hashes and fully sorts */
   int hist_par = 0, sorted_par = 0, append_par = 0, qpar = 0;
+  HostStage stage;
+  std::vector<float4> host;       /* one simulation's streams (bdem_batch_get_state) */
   /* graphs of 2 and of GRAPH_STEPS steps, per parity */
   struct StepGraph {
     hipGraphExec_t exec = nullptr;
@@ -553,10 +555,14 @@ int bdem_batch_get_state(bdem_batch* B, int index, bdem_float3* pos, bdem_float3
   const Instance& I = B->inst[(size_t)index];
   BHIP(B, hipSetDevice(B->device));
   BHIP(B, hipStreamSynchronize(B->stream));
-  std::vector<float4> P(I.cap), V(I.cap), O(I.cap);
-  BHIP(B, hipMemcpy(P.data(), B->b.pos_cur + I.off, I.cap * sizeof(float4), hipMemcpyDeviceToHost));
-  BHIP(B, hipMemcpy(V.data(), B->b.vel_cur + I.off, I.cap * sizeof(float4), hipMemcpyDeviceToHost));
-  BHIP(B, hipMemcpy(O.data(), B->b.omg_cur + I.off, I.cap * sizeof(float4), hipMemcpyDeviceToHost));
+  /* the three streams into memory kept between calls */
+  const size_t cap = (size_t)I.cap;
+  if (B->host.size() < 3 * cap) B->host.resize(3 * cap);
+  float4 *P = B->host.data(), *V = P + cap, *O = V + cap;
+  using Region = HostStage::Region;
+  BHIP(B, B->stage.to_host({Region{(char*)(B->b.pos_cur + I.off), P, cap * sizeof(float4), nullptr, 0},
+                            Region{(char*)(B->b.vel_cur + I.off), V, cap * sizeof(float4), nullptr, 0},
+                            Region{(char*)(B->b.omg_cur + I.off), O, cap * sizeof(float4), nullptr, 0}}, B->stream));
   int k = 0;
   for (int s = 0; s < I.cap; ++s) {
     const int g = f_bits(O[s].w) >> 3;

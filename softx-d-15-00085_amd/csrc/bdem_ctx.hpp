@@ -9,6 +9,7 @@
 #include <vector>
 #include "bdem_abi.h"
 #include "bdem_kernels.hpp"
+#include "bdem_stage.hpp"
 
 using bdem::DevParams;
 using bdem::PolyBuffers;
@@ -70,6 +71,7 @@ struct bdem_ctx {
   uint32_t* dbg_list = nullptr;  /* debug: the contacts the step kernel used */
   uint32_t* dbg_nn = nullptr;
   int stepc = 0;
+  bdem::HostStage stage;     /* the state's way to and from the caller */
   /* runs of steady-state steps captured as HIP graphs, by length (2 or
    * GRAPH_STEPS) and parity of the per-step alternations (see bdem_step) */
   struct StepGraph {

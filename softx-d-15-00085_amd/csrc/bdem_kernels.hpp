@@ -248,6 +248,24 @@ hipError_t noalloc_scratch(int device, uint32_t** out);
 void launch_profile_noalloc(const StepBuffers& b, int axis, float lo, float inv_w, int bins, uint32_t* scr,
                             hipStream_t s);
 
+/* The caller's layout of the state (bdem_state.hip), device pointers. */
+struct StateArrays {
+  bdem_float3* pos;
+  unsigned* ptype;
+  bdem_float3* vel;
+  int* pid;
+  bdem_float3* avel;
+  bdem_Quaterion* quat;
+};
+struct UnpackMode { int has_vel, has_avel, has_quat, per_particle, shape_by_pid; };
+/* Current state -> out (shapes: position - COM of the row); in -> current
+ * state; radius and mass of every slot. */
+void launch_pack_state(const StepBuffers& b, const bdem_poly_shape* shapes, int num_shapes, bool by_pid, bool orient,
+                       const StateArrays& out, hipStream_t s);
+void launch_unpack_state(const DevParams* dP, const StepBuffers& b, const StateArrays& in, const UnpackMode& m,
+                         const bdem_poly_shape* shapes, bool orient, hipStream_t s);
+void launch_set_radii(const StepBuffers& b, const float* radius, const float* mass, hipStream_t s);
+
 /* Debug stages on the sorted scratch state. */
 void launch_contact_list(const DevParams* dP, const StepBuffers& b, uint32_t* list32, uint32_t* nn,
                          hipStream_t s);

@@ -1254,7 +1254,7 @@ __global__ __launch_bounds__(256) void k_poly_list(const DevParams* __restrict__
   __shared__ uint32_t cand[4][LIST_NP][LIST_CAND];
   __shared__ uint32_t list[4][LIST_NP][LIST_STRIDE];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int ps = lane / LIST_G, sub = lane & (LIST_G - 1);
+  const int ps = lane / LIST_G;
   const int i = xcd_block(blockIdx.x, gridDim.x) * LIST_BLOCK + wave * LIST_NP + ps;
   const bool in = i < n;
   const bool live = in && packed_pid(omg[i].w) >= 0;
