@@ -180,6 +180,21 @@ __device__ __forceinline__ bool overlaps(f3 pa, float ra, float4 pb) {
   return hit;
 }
 
+/* The same decision as one integer, for loops over many candidates.  The bits
+ * of a non-negative float order as the float, so with
+ *   key = bits(|d2|) - bits(s2) + 32
+ * a key below 0 says that d2 lies more than 32 floats below s2, that is below
+ * s2 (1 - 2^-19.1), a sure overlap by the argument above; a key above 64 that
+ * d2 lies as far above it (or is infinite or not a number), a sure miss; and
+ * only keys in 0 .. 64 need overlaps() itself. */
+constexpr uint32_t OVERLAP_BAND = 32u;
+__device__ __forceinline__ uint32_t overlap_key(f3 pa, float ra, float4 pb) {
+  const f3 d = pa - xyz(pb);
+  const float d2 = dot(d, d);
+  const float s = ra + pb.w;
+  return (__float_as_uint(d2) & 0x7FFFFFFFu) - (__float_as_uint(s * s) - OVERLAP_BAND);
+}
+
 /* The contact predicate of the reference (exact, above) and the membership
  * predicate of the skin lists: |pa - pb| < ra + rb + skin, decided on the
  * safe side (every pair that close is included, a few slightly farther may
@@ -252,7 +267,7 @@ __device__ __forceinline__ int for_each_contact(const DevParams& P, const uint2*
 constexpr int STAGE_POS = 128;
 constexpr int STAGE_CELL = 128;
 struct WaveStage {
-  float4 pos[STAGE_POS];
+  float4 pos[STAGE_POS + 1];   /* one more: scan_stage reads in pairs */
   uint2 cell[STAGE_CELL];
 };
 
@@ -302,51 +317,74 @@ __device__ __forceinline__ RowStage row_stage(uint2 e0, uint2 e1, uint32_t n) {
   return s;
 }
 
-/* Candidates [lo, hi) of one lane, read from `src` (LDS stage or global): a
- * bit per candidate, two reads in flight (past the end the last one is read
- * again), then the set bits are visited in order.  Visiting inside the loop
- * ran the visit's stores for nearly every candidate, since some lane hits:
- * 157.8 -> 151.6 us a step at 1,048,576 spheres (one read in flight 158.0,
- * four 163.5). */
-constexpr uint32_t SCAN_U = 2;
-template <class Visit, class Pred>
-__device__ __forceinline__ void scan_candidates(const float4* src, uint32_t lo, uint32_t hi, uint32_t shift,
-                                                int i, f3 pa, float ra, int& count, Visit& visit,
-                                                const Pred& pred) {
+/* Candidates [lo, hi) of one lane from the LDS stage: a bit per candidate,
+ * two reads in flight (one entry past the end may be read and is dropped),
+ * then the set bits are visited in order.  Per candidate the loop only takes
+ * overlap_key, shifts its sign into the mask and keeps the smallest key: a
+ * run with a key in the undecided band (about one candidate in 10^5) is tested
+ * again exactly.  The scan is half of k_step's instructions, 25 a candidate
+ * with the two-threshold test and 15 now; visiting inside the loop also ran
+ * the visit's stores for nearly every candidate, since some lane hits.
+ * Steps before and after (visits inside the loop / this): 1,048,576 spheres
+ * 157.8 / 142.6 us, 262,143 56.6 / 52.3, 64 batched boxes 109 / 100. */
+template <class Visit>
+__device__ __forceinline__ void scan_stage(const float4* src, uint32_t lo, uint32_t hi, uint32_t shift, int i, f3 pa,
+                                           float ra, int& count, Visit& visit) {
   for (uint32_t base = lo; base < hi; base += 32u) {
-    const uint32_t len = min(hi - base, 32u);
+    const uint32_t len = min(hi - base, 32u), even = (len + 1u) & ~1u;
     const float4* const at = src + (base - shift);
-    uint32_t mask = 0u;
-    for (uint32_t t = 0u; t < len; t += SCAN_U) {
-      float4 pb[SCAN_U];
-#pragma unroll
-      for (uint32_t u = 0u; u < SCAN_U; ++u) pb[u] = at[min(t + u, len - 1u)];
-#pragma unroll
-      for (uint32_t u = 0u; u < SCAN_U; ++u) mask |= (pred(pa, ra, pb[u]) ? 1u : 0u) << (t + u);
+    uint32_t mask = 0u, least = 0xFFFFFFFFu;   /* candidate t: bit even - 1 - t */
+    for (uint32_t t = 0u; t < len; t += 2u) {
+      const float4 p0 = at[t], p1 = at[t + 1u];
+      const uint32_t k0 = overlap_key(pa, ra, p0), k1 = overlap_key(pa, ra, p1);
+      mask = __builtin_amdgcn_alignbit(mask, k0, 31);   /* mask << 1 | sign */
+      mask = __builtin_amdgcn_alignbit(mask, k1, 31);
+      least = min(least, min(k0, k1));
     }
-    if (len < 32u) mask &= (1u << len) - 1u;
+    if (__builtin_expect(least <= 2u * OVERLAP_BAND, 0)) {
+      mask = 0u;
+      for (uint32_t t = 0u; t < len; ++t) mask = mask << 1 | (overlaps(pa, ra, at[t]) ? 1u : 0u);
+      mask <<= even - len;
+    }
+    mask &= ~(even - len);   /* an entry past the end */
     const uint32_t self = (uint32_t)i - base;
-    if (self < len) mask &= ~(1u << self);
+    if (self < len) mask &= ~(1u << (even - 1u - self));
     while (mask) {
-      const uint32_t t = (uint32_t)__builtin_ctz(mask);
-      mask &= mask - 1u;
-      visit((int)(base + t), at[t], count);
+      const uint32_t b = 31u - (uint32_t)__clz((int)mask);
+      mask &= ~(1u << b);
+      visit((int)(base + (even - 1u - b)), float4{}, count);
+      ++count;
+    }
+  }
+}
+
+/* The same from global memory (rows past the stage): exact, one by one. */
+template <class Visit>
+__device__ __forceinline__ void scan_global(const float4* __restrict__ pos_r, uint32_t lo, uint32_t hi, int i, f3 pa,
+                                            float ra, int& count, Visit& visit) {
+  for (uint32_t j = lo; j < hi; ++j) {
+    const float4 pb = pos_r[j];
+    if ((int)j != i && overlaps(pa, ra, pb)) {
+      visit((int)j, pb, count);
       ++count;
     }
   }
 }
 
 /* How one lane scans the candidate run [lo, hi) of stencil row r
- * (r = 3 (dy + 1) + (dz + 1)): every candidate with a predicate. */
-template <class Pred>
+ * (r = 3 (dy + 1) + (dz + 1)): every candidate with the contact predicate. */
 struct PlainRows {
-  Pred pred;
   template <class Visit>
-  __device__ __forceinline__ void row(const float4* src, uint32_t lo, uint32_t hi, uint32_t shift, int, int i,
-                                      f3 pa, float ra, int& count, Visit& visit) {
-    scan_candidates(src, lo, hi, shift, i, pa, ra, count, visit, pred);
+  __device__ __forceinline__ void staged(const float4* src, uint32_t lo, uint32_t hi, uint32_t shift, int, int i,
+                                         f3 pa, float ra, int& count, Visit& visit) {
+    scan_stage(src, lo, hi, shift, i, pa, ra, count, visit);
   }
-  __device__ __forceinline__ Pred lane_pred() { return pred; }
+  template <class Visit>
+  __device__ __forceinline__ void global(const float4* pos_r, uint32_t lo, uint32_t hi, int, int i, f3 pa, float ra,
+                                         int& count, Visit& visit) {
+    scan_global(pos_r, lo, hi, i, pa, ra, count, visit);
+  }
+  __device__ __forceinline__ OverlapTest lane_pred() { return OverlapTest(); }
 };
 
 /* Skin masks.  Bits 7r .. 7r+6 of `mask` mark which of the first seven
@@ -400,6 +438,16 @@ struct MaskedRows {
         }
       }
     }
+  }
+  template <class Visit>
+  __device__ __forceinline__ void staged(const float4* src, uint32_t lo, uint32_t hi, uint32_t shift, int r, int i,
+                                         f3 pa, float ra, int& count, Visit& visit) {
+    row(src, lo, hi, shift, r, i, pa, ra, count, visit);
+  }
+  template <class Visit>
+  __device__ __forceinline__ void global(const float4* pos_r, uint32_t lo, uint32_t hi, int r, int i, f3 pa, float ra,
+                                         int& count, Visit& visit) {
+    row(pos_r, lo, hi, 0u, r, i, pa, ra, count, visit);
   }
   /* a lane scanned on its own (outside the grid): no mask */
   __device__ __forceinline__ OverlapTest lane_pred() {
@@ -486,9 +534,9 @@ __device__ __forceinline__ int for_each_contact_wave_rows(const DevParams& P, co
           /* a consistent cell table puts every lane's run inside the stage;
            * checked, so LDS is never indexed outside it whatever the table holds */
           if (sc.staged && lo >= sc.pmin && hi <= sc.pmax)
-            rows.row(st.pos, lo, hi, sc.pmin, r, i, pa, ra, count, visit);
+            rows.staged(st.pos, lo, hi, sc.pmin, r, i, pa, ra, count, visit);
           else
-            rows.row(pos_r, lo, hi, 0u, r, i, pa, ra, count, visit);
+            rows.global(pos_r, lo, hi, r, i, pa, ra, count, visit);
         }
         __builtin_amdgcn_wave_barrier();
         ce0 = ne0; ce1 = ne1; ne0 = nn0; ne1 = nn1;
@@ -523,10 +571,10 @@ __device__ __forceinline__ int for_each_contact_wave_rows(const DevParams& P, co
           if (pmax - pmin <= (uint32_t)STAGE_POS) {
             for (uint32_t c = lane; c < pmax - pmin; c += 64) st.pos[c] = pos_r[pmin + c];
             __builtin_amdgcn_wave_barrier();
-            if (lo >= pmin && hi <= pmax) rows.row(st.pos, lo, hi, pmin, (dy + 1) * 3 + (dz + 1), i, pa, ra, count, visit);
-            else rows.row(pos_r, lo, hi, 0u, (dy + 1) * 3 + (dz + 1), i, pa, ra, count, visit);
+            if (lo >= pmin && hi <= pmax) rows.staged(st.pos, lo, hi, pmin, (dy + 1) * 3 + (dz + 1), i, pa, ra, count, visit);
+            else rows.global(pos_r, lo, hi, (dy + 1) * 3 + (dz + 1), i, pa, ra, count, visit);
           } else {
-            rows.row(pos_r, lo, hi, 0u, (dy + 1) * 3 + (dz + 1), i, pa, ra, count, visit);
+            rows.global(pos_r, lo, hi, (dy + 1) * 3 + (dz + 1), i, pa, ra, count, visit);
           }
           __builtin_amdgcn_wave_barrier();
         }
@@ -538,12 +586,12 @@ __device__ __forceinline__ int for_each_contact_wave_rows(const DevParams& P, co
   return count;
 }
 
-template <class Visit, class Pred = OverlapTest>
+template <class Visit>
 __device__ __forceinline__ int for_each_contact_wave(const DevParams& P, const uint2* __restrict__ cells,
                                                      const float4* __restrict__ pos_r, uint32_t n, int i,
                                                      f3 pa, float ra, bool active, WaveStage& st,
-                                                     Visit&& visit, Pred pred = Pred()) {
-  PlainRows<Pred> rows{pred};
+                                                     Visit&& visit) {
+  PlainRows rows;
   return for_each_contact_wave_rows(P, cells, pos_r, n, i, pa, ra, active, st, visit, rows);
 }
 

@@ -1379,13 +1379,23 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
           /* four reads in flight; past the end the last entry is read again */
           const uint32_t at = j0 - pmin[z], last = len ? len - 1u : 0u;
           const float4* const src = st.pos + (len ? at : 0u);
+          uint32_t least = 0xFFFFFFFFu;
           for (uint32_t t = 0u; t < len; t += 4u) {
             float4 pb[4];
 #pragma unroll
             for (uint32_t u = 0u; u < 4u; ++u) pb[u] = src[min(t + u, last)];
 #pragma unroll
-            for (uint32_t u = 0u; u < 4u; ++u) mask |= (overlaps(pa, ra, pb[u]) && t + u < len ? 1u : 0u) << (t + u);
+            for (uint32_t u = 0u; u < 4u; ++u) {
+              const uint32_t key = overlap_key(pa, ra, pb[u]);
+              mask |= (key >> 31) << (t + u);
+              least = min(least, key);
+            }
           }
+          if (__builtin_expect(least <= 2u * OVERLAP_BAND, 0)) {   /* a key in the undecided band */
+            mask = 0u;
+            for (uint32_t t = 0u; t < len; ++t) mask |= (overlaps(pa, ra, src[t]) ? 1u : 0u) << t;
+          }
+          if (len < 32u) mask &= (1u << len) - 1u;
         } else {
           for (uint32_t t = 0u; t < len; ++t) {
             const bool hit = overlaps(pa, ra, pos_r[j0 + t]);
