@@ -473,6 +473,11 @@ __device__ __forceinline__ int for_each_contact_wave_rows(const DevParams& P, co
   int count = 0;
   if (hmin <= hmax) {   /* some lane is in the grid (wave-uniform) */
     if (hmax - hmin + 3u <= (uint32_t)STAGE_CELL) {
+      /* a lane's row r is cells hx + off(r) .. + dx, where bit r of rowok is
+       * set (the hash is linear in the cell's coordinates) */
+      const uint32_t hx = H - (uint32_t)(g[0] - xs), dx = (uint32_t)(xe - xs);
+      const uint32_t zok = (g[2] > 0 ? 1u : 0u) | 2u | (g[2] + 1 < P.nz ? 4u : 0u);
+      const uint32_t rowok = ingrid ? (g[1] > 0 ? zok : 0u) | zok << 3 | (g[1] + 1 < P.ny ? zok << 6 : 0u) : 0u;
       /* Software pipeline over the nine rows r = 3 (dy + 1) + (dz + 1): while
        * row r is scanned from LDS, the candidates of row r + 1 and the cell
        * entries of row r + 2 are already in flight. */
@@ -515,21 +520,19 @@ __device__ __forceinline__ int for_each_contact_wave_rows(const DevParams& P, co
         }
         /* 3. scan row r: each lane's cells, then its candidates */
         if (wc.ok && sc.any) {
-          const int y = g[1] + (r / 3 - 1), z = g[2] + (r % 3 - 1);
-          const bool rv0 = ingrid && y >= 0 && y < P.ny && z >= 0 && z < P.nz && xs <= xe;
-          const uint32_t h0 = rv0 ? hash_of(P, xs, y, z) : 0u;
-          const uint32_t h1 = rv0 ? hash_of(P, xe, y, z) : 0u;
+          const long long off = (long long)(r % 3 - 1) * P.nz + (long long)(r / 3 - 1) * P.nx * P.nz;
+          const uint32_t h0 = hx + (uint32_t)off, h1 = h0 + dx;
           uint32_t lo = sc.pmin, hi = sc.pmin;
-          if (rv0 && h1 < P.C) {
-            uint32_t l2 = 0xFFFFFFFFu, h2 = 0u;
-            for (uint32_t h = h0; h <= h1; ++h) {
-              const uint2 c = st.cell[h - wc.w0];
-              if (c.x != 0xFFFFFFFFu) {
-                l2 = min(l2, c.x);
-                h2 = c.y;
-              }
+          if ((rowok >> r) & 1u && h1 < P.C) {
+            /* first and last occupied of the row's one to three cells; an
+             * empty entry's bounds are all ones */
+            const uint2* const cell = st.cell - wc.w0;
+            const uint2 c0 = cell[h0], c1 = cell[min(h0 + 1u, h1)], c2 = cell[h1];
+            const uint32_t l2 = min(min(c0.x, c1.x), c2.x);
+            if (l2 != 0xFFFFFFFFu) {
+              lo = l2;
+              hi = min((uint32_t)max(max((int)c0.y, (int)c1.y), (int)c2.y), n);
             }
-            if (l2 != 0xFFFFFFFFu) { lo = l2; hi = min(h2, n); }
           }
           /* a consistent cell table puts every lane's run inside the stage;
            * checked, so LDS is never indexed outside it whatever the table holds */
