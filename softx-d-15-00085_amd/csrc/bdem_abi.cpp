@@ -213,7 +213,7 @@ int upload_params(bdem_ctx* c) {
   build_params(c);
   HIPCHK(c, hipMemcpyAsync(c->dp, &c->hp, sizeof(DevParams), hipMemcpyHostToDevice, c->stream));
   std::vector<ShapeHdr> hdr;
-  std::vector<float4> local;
+  std::vector<float> local;
   if (c->dshape) {
     HIPCHK(c, hipMemcpyAsync(c->dshape, c->shapes.data(), c->shapes.size() * sizeof(bdem_poly_shape),
                              hipMemcpyHostToDevice, c->stream));
@@ -223,21 +223,24 @@ int upload_params(bdem_ctx* c) {
     HIPCHK(c, hipMemcpyAsync(c->pb.hdr, hdr.data(), hdr.size() * sizeof(ShapeHdr), hipMemcpyHostToDevice,
                              c->stream));
     const PolyLayout& L = c->pb.L;
-    local.assign(c->shapes.size() * (size_t)L.stride, float4{0.f, 0.f, 0.f, 0.f});
+    local.assign(c->shapes.size() * (size_t)L.stride * 3, 0.0f);
     for (size_t r = 0; r < c->shapes.size(); ++r) {
       const bdem_poly_shape& s = c->shapes[r];
-      float4* row = local.data() + r * (size_t)L.stride;
-      for (int v = 0; v < s.num_vertex; ++v)
-        row[v] = float4{s.Local_Vertex[v].x, s.Local_Vertex[v].y, s.Local_Vertex[v].z, 1.0f};
+      float* row = local.data() + r * (size_t)L.stride * 3;
+      auto put = [&](int slot, float x, float y, float z) {
+        row[3 * slot] = x;
+        row[3 * slot + 1] = y;
+        row[3 * slot + 2] = z;
+      };
+      for (int v = 0; v < s.num_vertex; ++v) put(v, s.Local_Vertex[v].x, s.Local_Vertex[v].y, s.Local_Vertex[v].z);
       for (int f = 0; f < s.num_faces; ++f) {
         const bdem_Surface& F = s.face[f];
-        row[L.pv + f] = float4{F.normal.x, F.normal.y, F.normal.z, 1.0f};
+        put(L.pv + f, F.normal.x, F.normal.y, F.normal.z);
         /* the float differences the turned centroid is made from */
-        const float dx = F.centroid.x - s.COM.x, dy = F.centroid.y - s.COM.y, dz = F.centroid.z - s.COM.z;
-        row[L.pv + L.pf + f] = float4{dx, dy, dz, 1.0f};
+        put(L.pv + L.pf + f, F.centroid.x - s.COM.x, F.centroid.y - s.COM.y, F.centroid.z - s.COM.z);
       }
     }
-    HIPCHK(c, hipMemcpyAsync(c->pb.local, local.data(), local.size() * sizeof(float4), hipMemcpyHostToDevice,
+    HIPCHK(c, hipMemcpyAsync(c->pb.local, local.data(), local.size() * sizeof(float), hipMemcpyHostToDevice,
                              c->stream));
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -780,7 +783,7 @@ int bdem_set_simulation_data(bdem_ctx* c, const bdem_WOBJ* wobj, const bdem_POBJ
     pb.L = poly_layout(c->shapes);
     ALLOC(c->dshape, c->shapes.size());
     ALLOC(pb.hdr, c->shapes.size());
-    ALLOC(pb.local, c->shapes.size() * (size_t)pb.L.stride);
+    ALLOC(pb.local, c->shapes.size() * (size_t)pb.L.stride * 3);
     ALLOC(pb.rot, (size_t)n * pb.L.stride);
     ALLOC(pb.list, (size_t)n * LIST_STRIDE);
     ALLOC(pb.nn, (size_t)n);
@@ -1069,9 +1072,9 @@ int bdem_set_poly_shapes(bdem_ctx* c, const bdem_poly_shape* shapes, int count) 
   drop_graphs(c);
   bdem_poly_shape* d = nullptr;
   ShapeHdr* dh = nullptr;
-  float4* dl = nullptr;
+  float* dl = nullptr;
   if ((rc = dalloc(c, &d, t.size())) != BDEM_OK) return rc;
-  if ((rc = dalloc(c, &dh, t.size())) != BDEM_OK || (rc = dalloc(c, &dl, t.size() * (size_t)L.stride)) != BDEM_OK) {
+  if ((rc = dalloc(c, &dh, t.size())) != BDEM_OK || (rc = dalloc(c, &dl, t.size() * (size_t)L.stride * 3)) != BDEM_OK) {
     dfree(c, d);
     dfree(c, dh);
     return rc;

@@ -5,8 +5,8 @@
  * 736-992) rotates both shapes for every listed pair and tests one pair per
  * particle thread in a serial loop.  Here a step is five launches:
  *
- *   k_poly_rotate   one thread per (particle, vertex / face-normal /
- *                   face-centroid slot): world-frame shapes into `rot`,
+ *   k_poly_rotate   a thread per four slots (vertex, face normal or face
+ *                   centroid) of a particle: world-frame shapes into `rot`,
  *                   written coalesced (RotatePolyhedra, Utilities.cuh:420-479)
  *   k_poly_list     bounding-sphere contact list in the reference order (the
  *   k_poly_list2    sphere broad phase; the second form for larger counts),
@@ -1183,31 +1183,54 @@ __device__ __forceinline__ PColl edges_dobj(const bdem_DOBJ& D, const Shape& B, 
 }  // namespace
 
 /* ------------------------------------------------------------------ kernels */
+/* World-frame shapes: a thread takes four slots of one particle, a quarter of
+ * the row apart, so that the particle's own loads (ID,
+ * shape header, position, quaternion) and its index serve several slots.
+ * Slots past a shape's counts are skipped: nothing reads them.  With a thread
+ * per slot its five loads, not the bytes, were the bound: 92 us at 200,000
+ * hulls, 88 with the skipped slots and 12-byte local rows, 63 now. */
+constexpr int ROT_SLOTS = 4;
 __global__ __launch_bounds__(256) void k_poly_rotate(const DevParams* __restrict__ Pp,
-                                                     const float4* __restrict__ local, int n,
-                                                     PolyLayout L, const float4* __restrict__ pos,
+                                                     const float* __restrict__ local,
+                                                     const ShapeHdr* __restrict__ hdr, int n, PolyLayout L,
+                                                     const float4* __restrict__ pos,
                                                      const float4* __restrict__ omg,
                                                      const float4* __restrict__ quat,
                                                      float4* __restrict__ rot, uint32_t* __restrict__ qcount) {
   const DevParams& P = *Pp;
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < POLY_QCOUNTS) qcount[t * POLY_QSTRIDE] = 0u;   /* this step's queues start empty */
-  const size_t i = t / (size_t)L.stride;
-  const int e = (int)(t - i * (size_t)L.stride);
+  const int part = (L.stride + ROT_SLOTS - 1) / ROT_SLOTS;
+  const size_t i = t / (size_t)part;
+  const int e0 = (int)(t - i * (size_t)part);
   if (i >= (size_t)n) return;
-  /* the shape row's slot e in the same layout, local frame (w = 1: used) */
-  const float4 l4 = local[(size_t)shape_index(P, omg[i].w) * L.stride + e];
-  const f3 l = xyz(l4);
+  const int row = shape_index(P, omg[i].w);
+  const ShapeHdr hd = hdr[row];
   const f3 c = xyz(pos[i]);
   const float4 q4 = quat[i];
   const QuatF Q{q4.x, q4.y, q4.z, q4.w};
   const QuatF QT{Q.w, -Q.x, -Q.y, -Q.z};
-  f3 out = mk3(0.f, 0.f, 0.f);
-  if (l4.w != 0.0f) {
-    out = P.rotation ? qrot(Q, QT, l) : l;
-    if (e < L.pv || e >= L.pv + L.pf) out = out + c;   /* vertices and centroids; normals turn only */
+  f3 l[ROT_SLOTS];
+  bool used[ROT_SLOTS];
+#pragma unroll
+  for (int k = 0; k < ROT_SLOTS; ++k) {
+    const int e = e0 + k * part;
+    const bool vertex = e < L.pv, normal = !vertex && e < L.pv + L.pf;
+    used[k] = e < L.stride && (vertex ? e < hd.nv() : (normal ? e - L.pv : e - L.pv - L.pf) < hd.nf());
+    l[k] = mk3(0.f, 0.f, 0.f);
+    if (used[k]) {   /* the row's slot e, local frame */
+      const float* const l3 = local + ((size_t)row * L.stride + e) * 3;
+      l[k] = mk3(l3[0], l3[1], l3[2]);
+    }
   }
-  rot[t] = make_float4(out.x, out.y, out.z, 0.0f);
+#pragma unroll
+  for (int k = 0; k < ROT_SLOTS; ++k) {
+    if (!used[k]) continue;
+    const int e = e0 + k * part;
+    f3 out = P.rotation ? qrot(Q, QT, l[k]) : l[k];
+    if (e < L.pv || e >= L.pv + L.pf) out = out + c;   /* vertices and centroids; normals turn only */
+    rot[i * (size_t)L.stride + e] = make_float4(out.x, out.y, out.z, 0.0f);
+  }
 }
 
 /* A particle's list (its c contacts, in LDS) to memory by its G lanes, and
@@ -1990,9 +2013,9 @@ static unsigned resident_blocks(K kernel) {
 
 static void launch_poly_forces_common(const DevParams* dP, const bdem_poly_shape* dshape, const StepBuffers& b,
                                       const PolyBuffers& pb, const uint32_t* sk, bool energy, hipStream_t s) {
-  const size_t rot_threads = (size_t)b.n * pb.L.stride;
+  const size_t rot_threads = (size_t)b.n * ((pb.L.stride + ROT_SLOTS - 1) / ROT_SLOTS);
   hipLaunchKernelGGL(k_poly_rotate, dim3((unsigned)((rot_threads + 255) / 256)), dim3(256), 0, s, dP, pb.local,
-                     b.n, pb.L, b.pos_srt, b.omg_srt, b.quat_srt, pb.rot, pb.qcount);
+                     pb.hdr, b.n, pb.L, b.pos_srt, b.omg_srt, b.quat_srt, pb.rot, pb.qcount);
   /* sixteen lanes a particle while the chip holds their waves (8,192) a few
    * times over: 11 against 36 us at 3,001 hulls, level near 30,000, 41
    * against 20 us at 50,000 */
@@ -2018,10 +2041,10 @@ static void launch_poly_forces_common(const DevParams* dP, const bdem_poly_shape
  * point-cloud output, between steps (the next step rewrites pb.rot). */
 void launch_poly_world_shapes(const DevParams* dP, const bdem_poly_shape* dshape, const StepBuffers& b,
                               const PolyBuffers& pb, hipStream_t s) {
-  const size_t rot_threads = (size_t)b.n * pb.L.stride;
+  const size_t rot_threads = (size_t)b.n * ((pb.L.stride + ROT_SLOTS - 1) / ROT_SLOTS);
   if (rot_threads == 0) return;
   hipLaunchKernelGGL(k_poly_rotate, dim3((unsigned)((rot_threads + 255) / 256)), dim3(256), 0, s, dP, pb.local,
-                     b.n, pb.L, b.pos_cur, b.omg_cur, b.quat_cur, pb.rot, pb.qcount);
+                     pb.hdr, b.n, pb.L, b.pos_cur, b.omg_cur, b.quat_cur, pb.rot, pb.qcount);
 }
 
 void launch_poly_step(const DevParams* dP, const bdem_poly_shape* dshape, const StepBuffers& b, const PolyBuffers& pb,
