@@ -3,28 +3,30 @@
  *
  * Kernel_ParticleInteraction_Polyhedra_NonSymmetry (DEM_Kernels_Compute.cuh:
  * 736-992) rotates both shapes for every listed pair and tests one pair per
- * particle thread in a serial loop.  Here a step is five launches:
+ * particle thread in a serial loop.  Here a step is five launches, six with
+ * lifters:
  *
  *   k_poly_rotate   a thread per four slots (vertex, face normal or face
  *                   centroid) of a particle: world-frame shapes into `rot`,
  *                   written coalesced (RotatePolyhedra, Utilities.cuh:420-479)
  *   k_poly_list     bounding-sphere contact list in the reference order (the
- *   k_poly_list2    sphere broad phase; the second form for larger counts),
- *                   plus a queue of (particle, slot) work items appended one
- *                   atomic per block
- *   k_poly_pairs    one thread per queued pair, grid-stride over the queue:
- *                   the separating-plane test of the two facing faces; the
- *                   pairs it does not separate go to a second queue
+ *   k_poly_list2    sphere broad phase; the second form for larger counts)
+ *   k_poly_pairs    the separating-plane test of each listed pair, once for
+ *                   both bodies: last step's face, then the two facing faces;
+ *                   the pairs these do not separate go to a queue
  *   k_poly_narrow   one wave per pair of that queue, both bodies staged in
  *                   LDS: the full separating-plane test (a lane per face),
  *                   vertex-face both ways (a lane per vertex), edge-edge
  *                   (lanes over the edge pairs a distance bound keeps),
- *                   depth clamps, pair law.  Results go to the pair's own
- *                   slot, so the queue orders do not matter
- *   k_poly_finish   one thread per particle: gravity, then the slots in list
- *                   order (the reference's summation order), walls, the
- *                   tensor integrator and quaternion, discharge, next key,
- *                   changed flag and changed-list append
+ *                   depth clamps, pair law, for both bodies' contacts.
+ *                   Results go to the contacts' own slots, so the queue
+ *                   order does not matter
+ *   k_poly_lift     with lifters: a wave per hull in reach of one
+ *   k_poly_finish   one thread per particle: gravity, then the slots in
+ *                   contact in list order (the reference's summation order),
+ *                   lifter force, walls, the tensor integrator and
+ *                   quaternion, discharge, next key, changed flag and
+ *                   changed-list append
  *
  * Every float expression follows the restatement's operation order, so the
  * results equal the oracle's bit for bit away from sin/cos in the quaternion.
@@ -615,7 +617,7 @@ __device__ __forceinline__ int facing_face(const Shape& A, f3 dirAB) {
  * starts with the separating-plane test both ways (is_SP_Poly_Poly): true
  * when some face of one body separates them.  Which face is found does not
  * matter, only whether one exists, so each body's face turned most towards
- * the other is tried first (quick_separated, one thread per pair): it
+ * the other is tried first (quick_separated, a lane per pair): it
  * separates most separated pairs.  The rest go to the wave-per-pair kernel,
  * where separated_wave tests every face at once. */
 /* A separating face is named by a code: f for face f of A, 0x100 | f for
