@@ -17,6 +17,7 @@
 #include <vector>
 #include "bdem_abi.h"
 #include "bdem_ctx.hpp"
+#include "bdem_grid.hpp"
 #include "bdem_kernels.hpp"
 
 using namespace bdem;
@@ -158,6 +159,11 @@ void build_params(bdem_ctx* c) {
   P.one_type = c->pobj.size() == 1 ? 1 : 0;   /* uploads reject types >= num_pobj */
   P.vbound_scale = float(c->vbound_scale);
   P.shape_by_pid = c->shape_by_pid ? 1 : 0;
+  if (c->poly) {
+    float rmax = 0.0f;
+    for (const bdem_poly_shape& sh : c->shapes) rmax = std::max(rmax, sh.radius);
+    P.hash_local = hash_is_local(P.nx, P.ny, P.nz, contact_reach(rmax, P.cell.x, P.cell.y, P.cell.z)) ? 1 : 0;
+  }
   for (size_t t = 0; t < c->pobj.size() && t < size_t(MAX_TYPES); ++t) {
     const bdem_POBJ& po = c->pobj[t];
     P.t_radius[t] = po.radius;
@@ -1611,12 +1617,25 @@ int bdem_debug_poly_queues(bdem_ctx* c, unsigned int* counts) {
   if (!c->poly) return fail(c, BDEM_EINVAL, "not a polyhedra context (particle_type 1)");
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  std::vector<uint32_t> nn((size_t)c->b.n), q(POLY_QCOUNTS * POLY_QSTRIDE);
+  const size_t n = (size_t)c->b.n, subcap = poly_subqueue_capacity(c->b.n);
+  std::vector<uint32_t> nn(n), list(n * LIST_STRIDE), q(POLY_QCOUNTS * POLY_QSTRIDE);
   HIPCHK(c, hipMemcpy(nn.data(), c->pb.nn, nn.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
+  HIPCHK(c, hipMemcpy(list.data(), c->pb.list, list.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
   HIPCHK(c, hipMemcpy(q.data(), c->pb.qcount, q.size() * sizeof(uint32_t), hipMemcpyDeviceToHost));
   counts[0] = counts[1] = 0u;
   for (uint32_t v : nn) counts[0] += std::min(v, (uint32_t)LIST_STRIDE);
-  for (int s = 0; s < POLY_SUBQ; ++s) counts[1] += 2u * q[(size_t)s * POLY_QSTRIDE];   /* a pair is listed from both sides */
+  for (int s = 0; s < POLY_SUBQ; ++s) {
+    std::vector<uint2> e(std::min((size_t)q[(size_t)s * POLY_QSTRIDE], subcap));
+    if (e.empty()) continue;
+    HIPCHK(c, hipMemcpy(e.data(), c->pb.equeue + s * subcap, e.size() * sizeof(uint2), hipMemcpyDeviceToHost));
+    for (const uint2& w : e) {   /* an entry stands for both bodies' contacts where both list it */
+      const uint32_t a = w.x / LIST_STRIDE;
+      const uint32_t *A = &list[(size_t)a * LIST_STRIDE], *B = &list[(size_t)w.y * LIST_STRIDE];
+      const auto ours = std::count(A, A + w.x % LIST_STRIDE, w.y);
+      const auto theirs = std::count(B, B + std::min(nn[w.y], (uint32_t)LIST_STRIDE), a);
+      counts[1] += ours < theirs ? 2u : 1u;
+    }
+  }
   return BDEM_OK;
 }
 

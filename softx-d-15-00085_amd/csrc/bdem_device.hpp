@@ -110,6 +110,7 @@ struct DevParams {
   int one_type;               /* one particle type: every pair uses law_pp[0][0] */
   float vbound_scale;         /* polyhedra: largest |q|^2 (>= 1) of the last orientation upload */
   int shape_by_pid;           /* polyhedra: shape-table rows are P_IDs (else types) */
+  int hash_local;             /* polyhedra: no two nearby cells share a hash (hash_is_local) */
   LawPair law_w[MAX_TYPES];
   bdem_cone cone[BDEM_MAX_CONES];
   bdem_WOBJ wobj[MAX_WOBJ];

@@ -1445,20 +1445,32 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
   list_store<2>(i, in, count, mine, list32, nn, hitf, qcount, status);
 }
 
-/* Whether particle i is among the listed contacts of j. */
-__device__ __forceinline__ bool is_listed(const uint32_t* __restrict__ list32, int j, uint32_t i) {
-  bool found = false;
-  for (int k = 0; k < LIST_STRIDE; ++k) found = found || list32[(size_t)j * LIST_STRIDE + k] == i;
-  return found;
+/* Whether the list of j holds the contact that entry k of particle i's list
+ * names (partner j).  A partner may be listed several times where cells share
+ * a hash; the entries of the two lists then belong together in list order,
+ * the first to the first.  False when j's list has no such entry: i's key is
+ * past the table, its row was cut off there, or j's list overflowed. */
+__device__ __forceinline__ bool listed_back(const uint32_t* __restrict__ list32, const uint32_t* __restrict__ nn, int i,
+                                            int k, int j) {
+  int ours = 0, theirs = 0;
+  for (int q = 0; q < k; ++q) ours += list32[(size_t)i * LIST_STRIDE + q] == (uint32_t)j ? 1 : 0;
+  const int m = (int)min(nn[j], (uint32_t)LIST_STRIDE);
+  for (int q = 0; q < m; ++q) theirs += list32[(size_t)j * LIST_STRIDE + q] == (uint32_t)i ? 1 : 0;
+  return ours < theirs;
 }
 
 /* The separating-plane test of the pairs listed by PPB consecutive
  * particles.  Whether a face separates two bodies is the same question from
- * both sides, so a pair is tested once, by the particle with the lower
- * sorted slot (the other only when the first one's list overflowed without
- * it).  First every pair takes the face that separated it at the last step;
- * those it does not separate are gathered in LDS and take the two facing
- * faces with full waves; the rest go to a queue for k_poly_narrow.
+ * both sides, so a contact that both bodies list is tested once, by the
+ * particle with the lower sorted slot; what only one of them lists is tested
+ * by that one (listed_back).  The higher body looks into its partners' lists
+ * only where they may lack it: in a step in which some list overflowed, for
+ * keys in the table's last two cells and past it (in other cells every row
+ * that holds the particle is inside the table), and everywhere in grids whose
+ * nearby cells share hashes (DevParams::hash_local).  First every pair takes
+ * the face that separated it at the last step; those it does not separate are
+ * gathered in LDS and take the two facing faces with full waves; the rest go
+ * to a queue for k_poly_narrow.
  *
  * A reservation in one shared counter costs about 10 ns, one after another
  * (1,172 more of them added 12 us to a launch): 35,700 per launch held an
@@ -1471,6 +1483,7 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
                                                     const ShapeHdr* __restrict__ hdr, int n, PolyLayout L,
                                                     const float4* __restrict__ rot,
                                                     const float4* __restrict__ pos, const float4* __restrict__ omg,
+                                                    const uint32_t* __restrict__ sorted_keys,
                                                     const uint32_t* __restrict__ list32,
                                                     const uint32_t* __restrict__ nn, uint32_t* __restrict__ qcount,
                                                     uint2* __restrict__ equeue, uint32_t subcap,
@@ -1512,13 +1525,16 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
   };
   if (threadIdx.x == 0) { nitems = 0u; nleft = 0u; nout = 0u; }
   __syncthreads();
-  /* two threads a particle, 16 list entries each in four loads; nn of the
-   * partners is needed only in a step where some list overflowed */
+  /* two threads a particle, 16 list entries each in four loads */
   const bool over = qcount[POLY_OVERFLOW * POLY_QSTRIDE] != 0u;
   for (int t0 = 0; t0 < 2 * PPB; t0 += 256) {
     const int t = t0 + (int)threadIdx.x, i = base + (t >> 1), k0 = (t & 1) * (LIST_STRIDE / 2);
     int m = 0;
-    if (t < 2 * PPB && i < n) m = (int)min(nn[i], (uint32_t)LIST_STRIDE) - k0;
+    bool look = !P.hash_local;
+    if (t < 2 * PPB && i < n) {
+      m = (int)min(nn[i], (uint32_t)LIST_STRIDE) - k0;
+      look = look || sorted_keys[i] + 2u >= P.C;
+    }
     uint32_t js[LIST_STRIDE / 2];
 #pragma unroll
     for (int q = 0; q < LIST_STRIDE / 8; ++q) {
@@ -1530,7 +1546,8 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
 #pragma unroll
     for (int q = 0; q < LIST_STRIDE / 2; ++q) {
       bool w = q < m && js[q] > (uint32_t)i;
-      if (over && q < m && !w) w = nn[js[q]] > (uint32_t)LIST_STRIDE && !is_listed(list32, (int)js[q], (uint32_t)i);
+      if ((look || over) && q < m && !w)
+        w = (look || nn[js[q]] > (uint32_t)LIST_STRIDE) && !listed_back(list32, nn, i, k0 + q, (int)js[q]);
       want |= (w ? 1u : 0u) << q;
     }
     const int own = __popc(want);
@@ -1592,13 +1609,13 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
   }
 }
 
-/* One pair's bodies staged in LDS by its wave: turned vertices, face
- * normals and centroids, and edge lists of A (row 0) and B (row 1). */
 /* A pair's contact, kept until the chunk's pair law runs. */
 struct PairHit { uint32_t slot; float dis, nx, ny, nz, cx, cy, cz; };   /* slot NO_SLOT: no contact */
 constexpr uint32_t NO_SLOT = 0xFFFFFFFFu;
 constexpr uint32_t NARROW_CHUNK = 32;   /* largest chunk of the narrow kernel's queue */
 
+/* One pair's bodies staged in LDS by its wave: turned vertices, face
+ * normals and centroids, and edge lists of A (row 0) and B (row 1). */
 struct PairStage {
   float4 v[2][BDEM_SHAPE_MAX_VERTEX];
   float4 fn[2][BDEM_SHAPE_MAX_FACE];
@@ -1637,7 +1654,7 @@ struct PairStage {
  * counts (lanes 0-31 body A, 32-63 body B; rows past the counts are inside
  * the record and never read) before the first LDS write.
  *
- * Five waves per SIMD: at most 96 VGPRs without spills, and five blocks of
+ * Five waves per SIMD: at most 96 VGPRs (26 values spill), and five blocks of
  * 29 KiB of LDS (four stages and their chunk's contacts) per CU. */
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_poly_narrow(const DevParams* __restrict__ Pp,
                                                      const bdem_poly_shape* __restrict__ shapes,
@@ -1718,7 +1735,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
       }
       const float farea = F.area;
       const int fnv = F.num_vertex;
-      const uint32_t back = list32[(size_t)partner * LIST_STRIDE + k];
+      /* both bodies' lists: lanes 0-31 the partner's, 32-63 the particle's own */
+      const uint32_t self = slot / LIST_STRIDE;
+      const uint32_t entry = list32[(size_t)(h ? self : partner) * LIST_STRIDE + k];
       const uint32_t nback = nn[partner];
       const PairOps o = pair_ops_ab(P, slot, partner, pos, vel, omg);
       const float vbA = ha.vbound * P.vbound_scale, vbB = hb.vbound * P.vbound_scale;
@@ -1733,8 +1752,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
       S.area[h][k] = farea;
       S.fnv[h][k] = fnv;
       __builtin_amdgcn_wave_barrier();
-      /* A's place in B's list (absent when that list overflowed) */
-      const uint32_t at = (uint32_t)__ballot(!h && (uint32_t)k < nback && back == slot / LIST_STRIDE);
+      /* this contact's place in B's list: of the entries that name A the one
+       * with as many before it as this slot has in A's list (listed_back);
+       * none when B's list has no such entry */
+      const uint64_t same = __ballot(h ? entry == partner : (uint32_t)k < nback && entry == self);
+      uint32_t at = (uint32_t)same;
+      for (uint32_t before = (uint32_t)(same >> 32) & ((1u << (slot % LIST_STRIDE)) - 1u); before; before &= before - 1u)
+        at &= at - 1u;
       const uint32_t slot_b = at ? partner * LIST_STRIDE + (uint32_t)(__ffs(at) - 1) : NO_SLOT;
       const Shape A{S.v[0], S.fn[0], S.fc[0], ha.nv(), ha.nf(), S.vo[0], S.area[0], S.fnv[0]};
       const Shape B{S.v[1], S.fn[1], S.fc[1], hb.nv(), hb.nf(), S.vo[1], S.area[1], S.fnv[1]};
@@ -2030,7 +2054,7 @@ static void launch_poly_forces_common(const DevParams* dP, const bdem_poly_shape
   const uint32_t subcap = poly_subqueue_capacity(b.n);
   auto pairs = [&](auto kernel, int ppb) {
     hipLaunchKernelGGL(kernel, dim3((b.n + ppb - 1) / ppb), dim3(256), 0, s, dP, pb.hdr, b.n, pb.L, pb.rot, b.pos_srt,
-                       b.omg_srt, pb.list, pb.nn, pb.qcount, pb.equeue, subcap, pb.hint);
+                       b.omg_srt, sk, pb.list, pb.nn, pb.qcount, pb.equeue, subcap, pb.hint);
   };
   if (b.n <= POLY_PAIRS_SMALL) pairs(k_poly_pairs<POLY_PPB_SMALL>, POLY_PPB_SMALL);
   else pairs(k_poly_pairs<POLY_PPB>, POLY_PPB);
