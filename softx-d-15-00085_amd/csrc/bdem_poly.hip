@@ -913,12 +913,18 @@ __device__ __forceinline__ void wall_forces_poly(const DevParams& P, int t, f3 p
         F = ft;
         if (P.rotation && res.cls != C_FF) T = T + tq;
       }
-      if (cyl.has_top_cap && !clear_of_plane(cvt(cyl.normal_top_cap), cvt(cyl.center_top_cap), p, vb)) {
-        res = vertices_plane(A, cvt(cyl.normal_top_cap), cvt(cyl.center_top_cap));
+      /* a body clear of a cap has no contact with it, and that is the result
+       * an infinite plane after the cylinder finds */
+      if (cyl.has_top_cap) {
+        res.hit = false;
+        if (!clear_of_plane(cvt(cyl.normal_top_cap), cvt(cyl.center_top_cap), p, vb))
+          res = vertices_plane(A, cvt(cyl.normal_top_cap), cvt(cyl.center_top_cap));
         if (res.hit) F = resp_endplate(P, t, v, Coll{true, res.dis, res.cp, res.n});
       }
-      if (cyl.has_bot_cap && !clear_of_plane(cvt(cyl.normal_bot_cap), cvt(cyl.center_bot_cap), p, vb)) {
-        res = vertices_plane(A, cvt(cyl.normal_bot_cap), cvt(cyl.center_bot_cap));
+      if (cyl.has_bot_cap) {
+        res.hit = false;
+        if (!clear_of_plane(cvt(cyl.normal_bot_cap), cvt(cyl.center_bot_cap), p, vb))
+          res = vertices_plane(A, cvt(cyl.normal_bot_cap), cvt(cyl.center_bot_cap));
         if (res.hit) F = resp_endplate(P, t, v, Coll{true, res.dis, res.cp, res.n});
       }
     }
