@@ -1396,13 +1396,13 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
             uint32_t b = c2.x != 0xFFFFFFFFu ? c2.y : (c1.x != 0xFFFFFFFFu ? c1.y : c0.y);
             b = min(b, (uint32_t)n);   /* table entries never exceed n; kept in range regardless */
             lo = a;
-            cnt = b > a ? b - a : 0u;
+            cnt = b - min(a, b);
           }
         }
       }
       const bool staged = lo >= pmin[z] && lo + cnt <= pmin[z] + pcnt[z];
       for (uint32_t base = 0u; __any((int)(base < cnt)); base += 64u) {
-        const uint32_t rem = base < cnt ? min(cnt - base, 64u) : 0u;
+        const uint32_t rem = min(cnt - min(base, cnt), 64u);
         const uint32_t half = (rem + 1u) >> 1;
         const uint32_t j0 = lo + base + (sub ? half : 0u), len = sub ? rem - half : half;
         uint32_t mask = 0u;

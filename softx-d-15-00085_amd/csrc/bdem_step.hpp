@@ -284,7 +284,7 @@ __device__ __forceinline__ int team_contacts(const DevParams& P, const uint2* __
           uint32_t b = c2.x != 0xFFFFFFFFu ? c2.y : (c1.x != 0xFFFFFFFFu ? c1.y : c0.y);
           b = min(b, n);   /* table entries never exceed n; kept in range regardless */
           lo[q] = a;
-          cnt[q] = b > a ? b - a : 0u;
+          cnt[q] = b - min(a, b);
         }
       }
     }
@@ -346,7 +346,7 @@ __device__ __forceinline__ int team_contacts(const DevParams& P, const uint2* __
       for (int k = max(-at, 0); k < end; ++k) cand[at + k] = lo[q] + (uint32_t)k;
     }
     __builtin_amdgcn_wave_barrier();
-    const uint32_t m = total > c0 ? min(total - c0, (uint32_t)CAND) : 0u;
+    const uint32_t m = min(total - min(c0, total), (uint32_t)CAND);
     for (uint32_t t0 = 0u; __any((int)(t0 < m)); t0 += 4u * G) {
       uint32_t j[4];
 #pragma unroll
