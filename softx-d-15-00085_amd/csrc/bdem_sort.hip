@@ -163,28 +163,31 @@ __device__ __forceinline__ int wave_find_unchanged(const uint8_t* __restrict__ c
   return -1;
 }
 
-/* A block owns T slots, one per thread.  What bounds it: at a million slots
- * the bytes (state read and written, about 130 B a slot); below some 300,000
- * the chain of round trips and barriers in a block and what one CU can move.
- * So the tile is small (4,096 slots a block left 8,192 particles to two of
- * 256 CUs), every load of a thread's slot is issued at the start, before
- * anything waits, and stored when the position is known (loading and storing
- * stream by stream, each load behind the previous store, took 5-7 us of a
- * 13-15 us block), and the output's keys are kept in LDS for the cell bounds.
- * Steps with 1,024 threads on 4,096 slots / this one: 8,192 LSD 28.2 / 17.1
- * us, 60,013 Hertz-Mindlin 41.5 / 31.6, 262,143 66.3 / 58.6, 1,048,576
- * 159.7 / 159.4. */
-template <int T>
+/* A block owns T x ITEMS slots.  What bounds it: at a million slots the bytes
+ * (state read and written, about 130 B a slot) and the changed list, which
+ * every block reads; below some 300,000 the chain of round trips and barriers
+ * in a block and what one CU can move.  So few slots take small tiles of one
+ * slot a thread (4,096 slots a block left 8,192 particles to two of 256 CUs):
+ * every load of a thread's slot is issued at the start, before anything
+ * waits, and stored when the position is known (loading and storing stream
+ * by stream, each load behind the previous store, took 5-7 us of a 13-15 us
+ * block).  Larger tiles read stream by stream, since holding several slots'
+ * state spills.  The output's keys are kept in LDS for the cell bounds.
+ * Steps with 1,024 threads on 4,096 slots / one slot a thread: 8,192 LSD
+ * 28.2 / 17.1 us, 60,013 Hertz-Mindlin 41.5 / 31.6; the tiles' own times
+ * stand beside their rule (RS_T256). */
+template <int T, int ITEMS>
 __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
-  static_assert(T >= 256, "the fourth wave scans the per-wave counts");
+  constexpr int TILE = T * ITEMS, ROWS = ITEMS * (T / 64);   /* slots, (item, wave) counts of a block */
+  static_assert(T >= 256 && ROWS <= 64, "the fourth wave scans the per-(item, wave) counts");
   constexpr uint32_t LCAP = RS_LCAP / 1024 * T;   /* changed composites sorted in LDS */
-  __shared__ uint32_t okey_l[T];           /* old keys of the block's slots */
-  __shared__ uint32_t nkey[T + RS_KEYS];   /* keys of the block's output, when it fits */
-  __shared__ uint16_t ucnt[T + 1];         /* exclusive prefix of unchanged slots */
-  __shared__ uint8_t cand[T];              /* 1: candidate cell to clear, 2: refilled */
+  __shared__ uint32_t okey_l[TILE];          /* old keys of the block's slots */
+  __shared__ uint32_t nkey[TILE + RS_KEYS];  /* keys of the block's output, when it fits */
+  __shared__ uint16_t ucnt[TILE + 1];      /* exclusive prefix of unchanged slots */
+  __shared__ uint8_t cand[TILE];           /* 1: candidate cell to clear, 2: refilled */
   __shared__ unsigned long long Ls[LCAP];  /* L_b */
-  __shared__ uint32_t wcnt[T / 64];        /* unchanged per wave */
-  __shared__ uint32_t wpre[T / 64];
+  __shared__ uint32_t wcnt[ROWS];          /* unchanged per (item, wave) */
+  __shared__ uint32_t wpre[ROWS];
   __shared__ unsigned long long s_wlo, s_whi, s_upred, s_maxb, s_mina;
   __shared__ uint32_t s_below, s_chgb, s_nl, s_n2, s_ncand;
 
@@ -196,8 +199,8 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
   const int n = a.n;
   const uint32_t C = a.C;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int s0 = blockIdx.x * T;
-  const int cnt = min(T, n - s0);
+  const int s0 = blockIdx.x * TILE;
+  const int cnt = min(TILE, n - s0);
   uint32_t ns = a.meta[META_APPEND + par];
   if (ns > (uint32_t)n) {   /* each slot appends at most once: never read past the list */
     if (tid == 0) atomicOr(a.status, ST_SORT_ERROR);
@@ -208,21 +211,35 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
     a.meta[META_COUNT] = ns;
   }
 
-  /* 1. the block's slots, one per thread: old keys, changed flags, unchanged
-   * prefix.  The state is read now and stored in step 4. */
+  /* 1. the block's slots: old keys, changed flags, unchanged prefix.  Item it
+   * of thread tid is slot it * T + tid.  With one item the state is read now
+   * and stored in step 4. */
   const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  const bool mine = tid < cnt;
-  const int s = s0 + (mine ? tid : cnt - 1);
-  uint32_t ok = a.okeys[s];
-  const uint8_t cf = a.changed[s];
-  const float4 ps = a.pos_cur[s], vs = a.vel_cur[s], os = a.omg_cur[s];
-  const uint32_t hw = a.hwc_cur ? a.hwc_cur[s] : 0u;
-  if (!mine) ok = 0xFFFFFFFFu;
-  const bool ch = !mine || cf != 0;
-  if (mine) okey_l[tid] = ok;
-  cand[tid] = 0;
-  const uint64_t bal = __ballot(!ch);
-  if (lane == 0) wcnt[wave] = (uint32_t)__popcll(bal);
+  uint32_t ok[ITEMS];
+  bool ch[ITEMS];
+  uint64_t bal[ITEMS];
+  float4 ps, vs, os;
+  uint32_t hw;
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int t = it * T + tid;
+    const bool mine = t < cnt;
+    const int s = s0 + (mine ? t : cnt - 1);
+    ok[it] = a.okeys[s];
+    const uint8_t cf = a.changed[s];
+    if constexpr (ITEMS == 1) {
+      ps = a.pos_cur[s];
+      vs = a.vel_cur[s];
+      os = a.omg_cur[s];
+      hw = a.hwc_cur ? a.hwc_cur[s] : 0u;
+    }
+    if (!mine) ok[it] = 0xFFFFFFFFu;
+    ch[it] = !mine || cf != 0;
+    if (mine) okey_l[t] = ok[it];
+    cand[t] = 0;
+    bal[it] = __ballot(!ch[it]);
+    if (lane == 0) wcnt[it * (T / 64) + wave] = (uint32_t)__popcll(bal[it]);
+  }
   if (tid == 0) {
     s_below = 0u; s_chgb = 0u; s_nl = 0u; s_n2 = 0u; s_ncand = 0u;
     s_maxb = 0ull; s_mina = COMP_INF;
@@ -230,16 +247,16 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
   __syncthreads();
 
   if (wave == 3) {
-    /* exclusive scan of the waves' counts, in slot order */
-    const uint32_t v = lane < T / 64 ? wcnt[lane] : 0u;
+    /* exclusive scan of the (item, wave) counts, in slot order */
+    const uint32_t v = lane < ROWS ? wcnt[lane] : 0u;
     uint32_t incl = v;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const uint32_t u = (uint32_t)__shfl_up((int)incl, o, 64);
       if (lane >= o) incl += u;
     }
-    if (lane < T / 64) wpre[lane] = incl - v;
-    if (lane == T / 64 - 1) ucnt[T] = (uint16_t)incl;
+    if (lane < ROWS) wpre[lane] = incl - v;
+    if (lane == ROWS - 1) ucnt[TILE] = (uint16_t)incl;
   } else if (wave == 0) {
     /* window ends and the last unchanged element before the block */
     unsigned long long wlo = COMP_INF;
@@ -259,16 +276,23 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
   }
   /* cells the changed particles may leave empty: first slot of an old run,
    * every slot of the run changed (the run may continue past the block) */
-  if (mine && ch && ok < C && !(s > 0 && (tid > 0 ? okey_l[tid - 1] : a.okeys[s - 1]) == ok)) {
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int t = it * T + tid, s = s0 + t;
+    if (t >= cnt || !ch[it] || ok[it] >= C) continue;
+    if (s > 0 && (t > 0 ? okey_l[t - 1] : a.okeys[s - 1]) == ok[it]) continue;
     bool all = true;
-    for (int j = s + 1; j < n && a.okeys[j] == ok; ++j)
+    for (int j = s + 1; j < n && a.okeys[j] == ok[it]; ++j)
       if (a.changed[j] == 0) { all = false; break; }
-    if (all) { cand[tid] = 1; atomicAdd(&s_ncand, 1u); }
+    if (all) { cand[t] = 1; atomicAdd(&s_ncand, 1u); }
   }
   __syncthreads();
-  /* unchanged slots of the block before mine */
-  const uint32_t myc = wpre[wave] + (uint32_t)__popcll(bal & lt);
-  ucnt[tid] = (uint16_t)myc;
+  uint32_t myc[ITEMS];   /* unchanged slots of the block before mine */
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    myc[it] = wpre[it * (T / 64) + wave] + (uint32_t)__popcll(bal[it] & lt);
+    ucnt[it * T + tid] = (uint16_t)myc[it];
+  }
 
   /* 2. one pass over S */
   const unsigned long long wlo = s_wlo, whi = s_whi;
@@ -338,27 +362,33 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
 
   /* 4. positions, keys, slots and the gather */
   const uint32_t base = (uint32_t)s0 - s_chgb + below;
-  const uint32_t nu_b = ucnt[T];
+  const uint32_t nu_b = ucnt[TILE];
   const uint32_t total = nu_b + nl;
-  const bool keyed = total <= (uint32_t)(T + RS_KEYS);   /* the output's keys fit in LDS */
-  if (!ch) {
-    const unsigned long long c = comp(ok, (uint32_t)s);
+  const bool keyed = total <= (uint32_t)(TILE + RS_KEYS);   /* the output's keys fit in LDS */
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    if (ch[it]) continue;
+    const int s = s0 + it * T + tid;
+    const unsigned long long c = comp(ok[it], (uint32_t)s);
     const uint32_t r = nl == 0u ? 0u : (big ? lower_bound_u64(gl, nl, c) : lower_bound_u64(Ls, nl, c));
-    const uint32_t pos = base + myc + r;
-    if (pos >= (uint32_t)n) {
-      atomicOr(a.status, ST_SORT_ERROR);
-    } else {
-      if (keyed) nkey[myc + r] = ok;
-      a.keys_sorted[pos] = ok;
-      a.idx_sorted[pos] = s;
-      if (a.inv_map) a.inv_map[s] = pos;
-      a.pos_srt[pos] = ps;
-      a.vel_srt[pos] = vs;
-      a.omg_srt[pos] = os;
-      if (a.hwc_cur) a.hwc_srt[pos] = hw;
-      if (a.quat_cur) a.quat_srt[pos] = a.quat_cur[s];
-      if (a.mask_cur) a.mask_srt[pos] = a.mask_cur[s];
+    const uint32_t pos = base + myc[it] + r;
+    if (pos >= (uint32_t)n) { atomicOr(a.status, ST_SORT_ERROR); continue; }
+    if constexpr (ITEMS > 1) {
+      ps = a.pos_cur[s];
+      vs = a.vel_cur[s];
+      os = a.omg_cur[s];
+      hw = a.hwc_cur ? a.hwc_cur[s] : 0u;
     }
+    if (keyed) nkey[myc[it] + r] = ok[it];
+    a.keys_sorted[pos] = ok[it];
+    a.idx_sorted[pos] = s;
+    if (a.inv_map) a.inv_map[s] = pos;
+    a.pos_srt[pos] = ps;
+    a.vel_srt[pos] = vs;
+    a.omg_srt[pos] = os;
+    if (a.hwc_cur) a.hwc_srt[pos] = hw;
+    if (a.quat_cur) a.quat_srt[pos] = a.quat_cur[s];
+    if (a.mask_cur) a.mask_srt[pos] = a.mask_cur[s];
   }
   for (uint32_t r = tid; r < nl; r += T) {
     const unsigned long long c = big ? gl[r] : Ls[r];
@@ -409,7 +439,11 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
     else bounds([&](uint32_t q) { return a.keys_sorted[base + q]; });
   }
   /* 6. cells left empty */
-  if (mine && cand[tid] == 1) a.cells[ok] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int t = it * T + tid;
+    if (t < cnt && cand[t] == 1) a.cells[ok[it]] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
+  }
 }
 
 /* Kernel_SpatialDecomp_BinData (Collision_Detection_BroadPhase.cuh:279-325):
@@ -589,12 +623,19 @@ __global__ __launch_bounds__(SORT_THREADS) void k_fs_bin(SortArgs a) {
   if (i < a.n) bin_one(a.n, i, a.keys_sorted, a.cells, a.C);
 }
 
-/* Tile of the incremental path: 256, 512 and 1,024 slots a block measured the
- * same within 2 % up to 262,143 slots and 157.9, 159.4 and 163.9 us a step at
- * 1,048,576 with few changed keys.  Every block reads the whole changed list,
- * so larger arrays take the larger of the two fast tiles, which halves that
- * work when many keys change. */
-constexpr int RS_SMALL = 65536;
+/* Tile of the incremental path, by the number of slots.  Every block reads
+ * the whole changed list, so a step costs blocks x changed keys beside its
+ * bytes; a small tile shortens a block's chain.  Sort stage in us (events
+ * included) for 256 / 512 slots a block, one a thread, and 2,048 / 4,096 by
+ * 1,024 threads, with 0.3 %, 7 % and 27 % of the keys changed:
+ *     8,000   11.2 16.3 23.3 / 12.0 16.7 22.8
+ *    30,000   11.9 19.5 29.8 / 12.6 19.3 28.3 / 15.8 24.0 38.0 / 19.4 31.3 54.5
+ *   131,072                    15.5 26.2 43.5 / 18.6 30.4 51.2 / 22.8 39.4 71.4
+ *   262,144                    19.2 33.6 61.5 / 19.1 33.2 57.7 / 22.9 43.6 81.2
+ *   524,288                    26.0 71.5  173 / 21.1 43.7 82.2 / 25.5 52.9  102
+ *   750,000                    30.8  103  276 / 31.8 79.9  173 / 28.6 62.3  125
+ * 1,000,000                    40.4  160  459 / 35.2 93.5  213 / 31.7 71.3  149 */
+constexpr int RS_T256 = 32768, RS_T512 = 196608, RS_T2048 = 655360;
 
 static hipError_t launch_full_sort(const SortArgs& a, int par, hipStream_t s) {
   const int ntiles = sort_blocks(a.n);
@@ -622,8 +663,13 @@ static hipError_t launch_full_sort(const SortArgs& a, int par, hipStream_t s) {
 hipError_t launch_sort(const SortArgs& a, bool incremental, int par, hipStream_t s) {
   if (incremental) {
     const int extra = a.turn.params ? 1 : 0;
-    if (a.n <= RS_SMALL) hipLaunchKernelGGL(k_resort<256>, dim3((a.n + 255) / 256 + extra), dim3(256), 0, s, a, par);
-    else hipLaunchKernelGGL(k_resort<512>, dim3((a.n + 511) / 512 + extra), dim3(512), 0, s, a, par);
+    auto go = [&](auto kernel, int threads, int tile) {
+      hipLaunchKernelGGL(kernel, dim3((a.n + tile - 1) / tile + extra), dim3(threads), 0, s, a, par);
+    };
+    if (a.n <= RS_T256) go(k_resort<256, 1>, 256, 256);
+    else if (a.n <= RS_T512) go(k_resort<512, 1>, 512, 512);
+    else if (a.n <= RS_T2048) go(k_resort<1024, 2>, 1024, 2048);
+    else go(k_resort<1024, 4>, 1024, 4096);
     return hipGetLastError();
   }
   if (a.turn.params) launch_turn_lifters(a.turn, s);
