@@ -112,7 +112,8 @@ int bdem_set_tallys(bdem_ctx* ctx, const float* tallys);
 
 /* ---- state out (synchronous) -------------------------------------------- */
 /* Device_Get_System_State, Device/DeviceInterface.h:42-47: all
- * Num_Particles slots in device order; acc (may be NULL) is zero. */
+ * Num_Particles slots in device order; acc (may be NULL) is zero.  Threads
+ * may read one context at the same time. */
 int bdem_get_system_state(bdem_ctx* ctx, bdem_float3* pos, bdem_Quaterion* ornt, bdem_float3* vel,
                           bdem_float3* avel, bdem_float3* acc, unsigned int* ptype, int* pid);
 /* Device_Get_P_Positions, Device/DeviceInterface.h:50-51 */

@@ -87,6 +87,7 @@ void free_all(bdem_ctx* c) {
   c->shapes.clear();
   c->shape_by_pid = false;
   c->dp = nullptr;
+  c->io = nullptr;
   c->configured = false;
 }
 
@@ -459,19 +460,21 @@ int require(bdem_ctx* c) {
   return BDEM_OK;
 }
 
-/* The sorted scratch streams as the caller's arrays: they hold nothing
- * between steps (the next sort writes them). */
-StateArrays scratch_arrays(bdem_ctx* c) {
-  const StepBuffers& b = c->b;
-  const size_t n = (size_t)b.n;
+/* The caller's arrays on the device, in the context's own buffer for them:
+ * a read leaves the step's buffers alone, whatever is queued. */
+StateArrays state_arrays(bdem_ctx* c) {
+  const size_t n = (size_t)c->b.n;
   StateArrays a{};
-  a.pos = reinterpret_cast<bdem_float3*>(b.pos_srt);
+  a.pos = reinterpret_cast<bdem_float3*>(c->io);
   a.ptype = reinterpret_cast<unsigned*>(a.pos + n);
-  a.vel = reinterpret_cast<bdem_float3*>(b.vel_srt);
+  a.vel = reinterpret_cast<bdem_float3*>(a.ptype + n);
   a.pid = reinterpret_cast<int*>(a.vel + n);
-  a.avel = reinterpret_cast<bdem_float3*>(b.omg_srt);
-  a.quat = reinterpret_cast<bdem_Quaterion*>(b.quat_srt);
+  a.avel = reinterpret_cast<bdem_float3*>(a.pid + n);
+  if (c->orient) a.quat = reinterpret_cast<bdem_Quaterion*>(a.avel + n);
   return a;
+}
+size_t state_bytes(size_t n, bool orient) {
+  return n * (3 * sizeof(bdem_float3) + sizeof(unsigned) + sizeof(int) + (orient ? sizeof(bdem_Quaterion) : 0));
 }
 
 /* Host AoS -> device float4 streams.  Radius and mass come from the type
@@ -520,7 +523,8 @@ int upload_state(bdem_ctx* c, const bdem_float3* pos, const bdem_Quaterion* ornt
   c->keys_valid = false;
   c->flags_valid = false;
   c->lists_full = true;
-  const StateArrays d = scratch_arrays(c);
+  const std::lock_guard<std::mutex> one(c->io_lock);
+  const StateArrays d = state_arrays(c);
   const bool quat = c->orient && ornt && !c->sim.sphere_orient;
   const size_t v3 = (size_t)n * sizeof(bdem_float3), w1 = (size_t)n * sizeof(int);
   using Region = HostStage::Region;
@@ -769,6 +773,7 @@ int bdem_set_simulation_data(bdem_ctx* c, const bdem_WOBJ* wobj, const bdem_POBJ
   ALLOC(b.pos_cur, n); ALLOC(b.vel_cur, n); ALLOC(b.omg_cur, n);
   ALLOC(b.pos_srt, n); ALLOC(b.vel_srt, n); ALLOC(b.omg_srt, n);
   if (c->orient) { ALLOC(b.quat_cur, n); ALLOC(b.quat_srt, n); }
+  ALLOC(c->io, state_bytes((size_t)n, c->orient));
   ALLOC(b.keys_new, n); ALLOC(b.keys_sorted[0], n); ALLOC(b.keys_sorted[1], n);
   ALLOC(b.idx_sorted, n);
   ALLOC(b.changed, n);
@@ -922,11 +927,12 @@ int bdem_set_radii(bdem_ctx* c, const float* radius, const float* mass) {
   if (!radius || !mass) return fail(c, BDEM_EINVAL, "null argument");
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  const std::lock_guard<std::mutex> one(c->io_lock);
   const int n = c->b.n;
   for (int i = 0; i < n; ++i)
     if (!(radius[i] > 0.f) || !(mass[i] > 0.f)) return fail(c, BDEM_EINVAL, "radius and mass must be positive");
   using Region = HostStage::Region;
-  float *dr = reinterpret_cast<float*>(c->b.pos_srt), *dm = reinterpret_cast<float*>(c->b.vel_srt);
+  float *dr = reinterpret_cast<float*>(c->io), *dm = dr + n;
   const size_t w1 = (size_t)n * sizeof(float);
   const std::vector<Region> r{Region{(char*)dr, const_cast<float*>(radius), w1, nullptr, 0},
                               Region{(char*)dm, const_cast<float*>(mass), w1, nullptr, 0}};
@@ -954,8 +960,9 @@ int bdem_get_system_state(bdem_ctx* c, bdem_float3* pos, bdem_Quaterion* ornt, b
   int rc = require(c);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
+  const std::lock_guard<std::mutex> one(c->io_lock);   /* threads that read one context take turns */
   const size_t n = (size_t)c->b.n, v3 = n * sizeof(bdem_float3), w1 = n * sizeof(int);
-  const StateArrays d = scratch_arrays(c);
+  const StateArrays d = state_arrays(c);
   launch_pack_state(c->b, c->poly ? c->dshape : nullptr, (int)c->shapes.size(), c->shape_by_pid, c->orient, d,
                     c->stream);
   HIPCHK(c, hipGetLastError());

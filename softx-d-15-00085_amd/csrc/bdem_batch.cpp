@@ -24,6 +24,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 #include "bdem_batch.h"
@@ -67,8 +68,11 @@ struct bdem_batch {
 
   bool keys_valid = false;        /* false: the next step hashes and fully sorts */
   int hist_par = 0, sorted_par = 0, append_par = 0, qpar = 0;
+  /* one simulation's streams on their way out (bdem_batch_get_state) and the
+   * lock that a transfer holds */
   HostStage stage;
-  std::vector<float4> host;       /* one simulation's streams (bdem_batch_get_state) */
+  std::vector<float4> host;
+  std::mutex io_lock;
   /* graphs of 2 and of GRAPH_STEPS steps, per parity */
   struct StepGraph {
     hipGraphExec_t exec = nullptr;
@@ -555,6 +559,7 @@ int bdem_batch_get_state(bdem_batch* B, int index, bdem_float3* pos, bdem_float3
   const Instance& I = B->inst[(size_t)index];
   BHIP(B, hipSetDevice(B->device));
   BHIP(B, hipStreamSynchronize(B->stream));
+  const std::lock_guard<std::mutex> one(B->io_lock);   /* threads that read one batch take turns */
   /* the three streams into memory kept between calls */
   const size_t cap = (size_t)I.cap;
   if (B->host.size() < 3 * cap) B->host.resize(3 * cap);

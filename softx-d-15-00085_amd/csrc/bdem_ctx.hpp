@@ -5,6 +5,7 @@
  */
 #pragma once
 #include <hip/hip_runtime.h>
+#include <mutex>
 #include <string>
 #include <vector>
 #include "bdem_abi.h"
@@ -71,7 +72,11 @@ struct bdem_ctx {
   uint32_t* dbg_list = nullptr;  /* debug: the contacts the step kernel used */
   uint32_t* dbg_nn = nullptr;
   int stepc = 0;
-  bdem::HostStage stage;     /* the state's way to and from the caller */
+  /* the state's way to and from the caller: the caller's arrays on the
+   * device, the pinned stage, and the lock that a transfer holds */
+  char* io = nullptr;
+  bdem::HostStage stage;
+  std::mutex io_lock;
   /* runs of steady-state steps captured as HIP graphs, by length (2 or
    * GRAPH_STEPS) and parity of the per-step alternations (see bdem_step) */
   struct StepGraph {

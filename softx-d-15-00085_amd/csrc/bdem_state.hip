@@ -5,10 +5,10 @@
  *
  * The streams were copied whole through pageable vectors (allocated, faulted
  * in and converted particle by particle on each call): 8 of the 10 ms of a
- * 100,003-sphere restart.  Now a kernel packs what the caller asked for into
- * the sorted scratch streams, which hold nothing between steps, and the
- * bytes cross through two pinned halves of a small staging buffer, one in
- * flight while the other is copied from or to the caller's memory.
+ * 100,003-sphere restart.  Now a kernel packs the state into a buffer of the
+ * caller's layout, and the bytes asked for cross through two pinned halves of
+ * a small staging buffer, one in flight while the other is copied from or to
+ * the caller's memory.
  */
 #include "bdem_kernels.hpp"
 
