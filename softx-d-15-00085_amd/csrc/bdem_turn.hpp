@@ -38,15 +38,17 @@ __device__ __forceinline__ void turn_point(bdem_float3& v, double c, double s, f
 constexpr int TURN_THREADS = 256;
 static_assert(TURN_THREADS == 8 * MAX_DOBJ, "a thread per lifter vertex");
 /* By the first TURN_THREADS threads of a block, all of whose threads call;
- * tv: 8 x MAX_DOBJ turned vertices in LDS. */
+ * tv: 8 x MAX_DOBJ vertices in LDS, as they are after the turn. */
 __device__ __forceinline__ void turn_lifters_block(DevParams* __restrict__ P, const TurnArgs& t, bdem_float3* tv) {
   const int k = (int)threadIdx.x >> 3, q = (int)threadIdx.x & 7;
   const bool on = threadIdx.x < TURN_THREADS && k < P->num_dobj && P->dobj[k].is_attached_DWorld;
-  if (on && q < P->dobj[k].num_vertex) {
+  if (on) {
     bdem_float3 v = P->dobj[k].vertex[q];
-    turn_point(v, t.c, t.s, t.about[0], t.about[1], t.about[2]);
-    P->dobj[k].vertex[q] = v;
-    tv[threadIdx.x] = v;
+    if (q < P->dobj[k].num_vertex) {
+      turn_point(v, t.c, t.s, t.about[0], t.about[1], t.about[2]);
+      P->dobj[k].vertex[q] = v;
+    }
+    tv[threadIdx.x] = v;   /* a face of fewer than four vertices may name any of the eight */
   }
   __syncthreads();
   if (!on) return;
