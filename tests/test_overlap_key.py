@@ -1,7 +1,9 @@
 """The contact scan's one-integer test against the reference's own expression
 sqrt(d2) - s < 0 in float32: a key below 0 is a sure overlap, one above 64 a
 sure miss, over all magnitudes, the floats around equality, denormals,
-infinities and NaN of both signs."""
+infinities and NaN of both signs.  This proves the arithmetic, restated here
+in numpy; the device's own scans are held to the restatement's contact lists
+with pairs inside the undecided band in test_gpu_step_forms.py."""
 import numpy as np
 
 
