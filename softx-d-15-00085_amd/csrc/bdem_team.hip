@@ -25,11 +25,14 @@
  * resident round of waves the address rate of its 16-byte gathers, which
  * k_step avoids by staging whole rows in LDS.  Hence the shapes below: the
  * most lanes per particle whose waves the chip still holds at once.
- * Measured per step (resort and launch gaps included, about 21 us of each;
- * k_step beside it): 8,192 LSD 27.8 us (47.7), 20,000 reference law 29.5
- * (46.4), 32,000 LSD 31.4 (54.6), 60,013 Hertz-Mindlin 41.0 (61.8), 100,003
- * reference law 49.8 (54.0), 130,003 Hertz-Mindlin 65.5 (66.2), 262,143
- * 115 (66).
+ * Measured per step with the re-sort and the launch gaps (k_step beside it),
+ * random packs of r 0.5 cm at 1.5 to the cm3, about six contacts each: 8,192
+ * LSD 29.5 us (62), 20,000 reference law 29.1 (50), 32,000 LSD 37 (64),
+ * 60,013 Hertz-Mindlin 51.5 (71), 100,003 reference law 57 (65), 131,000
+ * reference law 66.6 (71.4), LSD 77 (87), Hertz-Mindlin 79 (89), 160,000
+ * Hertz-Mindlin 85 (92), 262,143 116 (108).  The gathers grow with the
+ * candidates: at 3 to the cm3, 12 contacts, 131,000 of the reference law take
+ * 153 (132).  TEAM_STEP_MAX lies between the two crossings.
  */
 #include "bdem_step.hpp"
 
@@ -171,8 +174,7 @@ __global__ __launch_bounds__(PB* G + 64) __attribute__((amdgpu_waves_per_eu(6)))
 
 /* Six waves per SIMD on 1,024 SIMDs hold 6,144 waves at once: five for 16
  * particles at 16 lanes each, five for 32 at 8, three for 32 at 4.  The last
- * shape is kept for two such rounds: at 100,003 it is still 8 % faster than
- * k_step, at 130,003 level with it. */
+ * shape is kept for two such rounds, up to TEAM_STEP_MAX (the figures above). */
 constexpr int TEAM16_MAX = 6144 / 5 * 16, TEAM8_MAX = 6144 / 5 * 32;
 static_assert(TEAM_STEP_MAX >= TEAM8_MAX, "team shapes in order");
 
