@@ -167,16 +167,20 @@ __device__ __forceinline__ int wave_find_unchanged(const uint8_t* __restrict__ c
  * (state read and written, about 130 B a slot) and the changed list, which
  * every block reads; below some 300,000 the chain of round trips and barriers
  * in a block and what one CU can move.  So few slots take small tiles of one
- * slot a thread (4,096 slots a block left 8,192 particles to two of 256 CUs):
- * every load of a thread's slot is issued at the start, before anything
- * waits, and stored when the position is known (loading and storing stream
- * by stream, each load behind the previous store, took 5-7 us of a 13-15 us
- * block).  Larger tiles read stream by stream, since holding several slots'
- * state spills.  The output's keys are kept in LDS for the cell bounds.
+ * slot a thread (4,096 slots a block left 8,192 particles to two of 256 CUs).
+ * The state of a thread's first EARLY slots is read at the start, before
+ * anything waits, and stored when the position is known; a further slot's is
+ * read while the one EARLY before it is stored.  (Stream by stream, each load
+ * behind the previous store, took 5-7 us of a 13-15 us block.)  The largest
+ * tile leaves one block a CU at a million slots, so all four of a thread's
+ * slots are read at the start, at 92 VGPRs: 28.6 us for the settled silo's
+ * sort against 33.7 with one early and 32.1 with 512 slots a block.  Two
+ * blocks a CU hide each other's waits, and one early slot is the better
+ * choice for 2,048.  The output's keys are kept in LDS for the cell bounds.
  * Steps with 1,024 threads on 4,096 slots / one slot a thread: 8,192 LSD
  * 28.2 / 17.1 us, 60,013 Hertz-Mindlin 41.5 / 31.6; the tiles' own times
  * stand beside their rule (RS_T256). */
-template <int T, int ITEMS>
+template <int T, int ITEMS, int EARLY>
 __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
   constexpr int TILE = T * ITEMS, ROWS = ITEMS * (T / 64);   /* slots, (item, wave) counts of a block */
   static_assert(T >= 256 && ROWS <= 64, "the fourth wave scans the per-(item, wave) counts");
@@ -212,14 +216,19 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
   }
 
   /* 1. the block's slots: old keys, changed flags, unchanged prefix.  Item it
-   * of thread tid is slot it * T + tid.  With one item the state is read now
-   * and stored in step 4. */
+   * of thread tid is slot it * T + tid. */
   const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
   uint32_t ok[ITEMS];
   bool ch[ITEMS];
   uint64_t bal[ITEMS];
-  float4 ps, vs, os;
-  uint32_t hw;
+  struct State { float4 p, v, o; uint32_t hw; };
+  auto state_of = [&](int it) {   /* past the end: the last slot's */
+    const int s = s0 + min(it * T + tid, cnt - 1);
+    return State{a.pos_cur[s], a.vel_cur[s], a.omg_cur[s], a.hwc_cur ? a.hwc_cur[s] : 0u};
+  };
+  State st[EARLY];   /* items it .. it + EARLY - 1 */
+#pragma unroll
+  for (int e = 0; e < EARLY; ++e) st[e] = state_of(e);
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
     const int t = it * T + tid;
@@ -227,12 +236,6 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
     const int s = s0 + (mine ? t : cnt - 1);
     ok[it] = a.okeys[s];
     const uint8_t cf = a.changed[s];
-    if constexpr (ITEMS == 1) {
-      ps = a.pos_cur[s];
-      vs = a.vel_cur[s];
-      os = a.omg_cur[s];
-      hw = a.hwc_cur ? a.hwc_cur[s] : 0u;
-    }
     if (!mine) ok[it] = 0xFFFFFFFFu;
     ch[it] = !mine || cf != 0;
     if (mine) okey_l[t] = ok[it];
@@ -367,28 +370,26 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
   const bool keyed = total <= (uint32_t)(TILE + RS_KEYS);   /* the output's keys fit in LDS */
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
-    if (ch[it]) continue;
+    const State cur = st[it % EARLY];
+    if (it + EARLY < ITEMS) st[it % EARLY] = state_of(it + EARLY);
     const int s = s0 + it * T + tid;
     const unsigned long long c = comp(ok[it], (uint32_t)s);
-    const uint32_t r = nl == 0u ? 0u : (big ? lower_bound_u64(gl, nl, c) : lower_bound_u64(Ls, nl, c));
+    const uint32_t r = ch[it] || nl == 0u ? 0u : (big ? lower_bound_u64(gl, nl, c) : lower_bound_u64(Ls, nl, c));
     const uint32_t pos = base + myc[it] + r;
-    if (pos >= (uint32_t)n) { atomicOr(a.status, ST_SORT_ERROR); continue; }
-    if constexpr (ITEMS > 1) {
-      ps = a.pos_cur[s];
-      vs = a.vel_cur[s];
-      os = a.omg_cur[s];
-      hw = a.hwc_cur ? a.hwc_cur[s] : 0u;
+    if (!ch[it] && pos >= (uint32_t)n) {
+      atomicOr(a.status, ST_SORT_ERROR);
+    } else if (!ch[it]) {
+      if (keyed) nkey[myc[it] + r] = ok[it];
+      a.keys_sorted[pos] = ok[it];
+      a.idx_sorted[pos] = s;
+      if (a.inv_map) a.inv_map[s] = pos;
+      a.pos_srt[pos] = cur.p;
+      a.vel_srt[pos] = cur.v;
+      a.omg_srt[pos] = cur.o;
+      if (a.hwc_cur) a.hwc_srt[pos] = cur.hw;
+      if (a.quat_cur) a.quat_srt[pos] = a.quat_cur[s];
+      if (a.mask_cur) a.mask_srt[pos] = a.mask_cur[s];
     }
-    if (keyed) nkey[myc[it] + r] = ok[it];
-    a.keys_sorted[pos] = ok[it];
-    a.idx_sorted[pos] = s;
-    if (a.inv_map) a.inv_map[s] = pos;
-    a.pos_srt[pos] = ps;
-    a.vel_srt[pos] = vs;
-    a.omg_srt[pos] = os;
-    if (a.hwc_cur) a.hwc_srt[pos] = hw;
-    if (a.quat_cur) a.quat_srt[pos] = a.quat_cur[s];
-    if (a.mask_cur) a.mask_srt[pos] = a.mask_cur[s];
   }
   for (uint32_t r = tid; r < nl; r += T) {
     const unsigned long long c = big ? gl[r] : Ls[r];
@@ -629,12 +630,13 @@ __global__ __launch_bounds__(SORT_THREADS) void k_fs_bin(SortArgs a) {
  * included) for 256 / 512 slots a block, one a thread, and 2,048 / 4,096 by
  * 1,024 threads, with 0.3 %, 7 % and 27 % of the keys changed:
  *     8,000   11.2 16.3 23.3 / 12.0 16.7 22.8
- *    30,000   11.9 19.5 29.8 / 12.6 19.3 28.3 / 15.8 24.0 38.0 / 19.4 31.3 54.5
- *   131,072                    15.5 26.2 43.5 / 18.6 30.4 51.2 / 22.8 39.4 71.4
- *   262,144                    19.2 33.6 61.5 / 19.1 33.2 57.7 / 22.9 43.6 81.2
- *   524,288                    26.0 71.5  173 / 21.1 43.7 82.2 / 25.5 52.9  102
- *   750,000                    30.8  103  276 / 31.8 79.9  173 / 28.6 62.3  125
- * 1,000,000                    40.4  160  459 / 35.2 93.5  213 / 31.7 71.3  149 */
+ *    30,000   12.2 19.3 29.4 / 12.6 19.3 28.3 / 15.4 23.6 37.4 / 21.2 32.8 57.0
+ *   131,072                    16.1 27.1 45.2 / 17.8 30.0 50.4 / 22.8 40.5 74.1
+ *   262,144                    19.1 33.8 63.0 / 19.7 33.5 57.0 / 24.8 46.0 84.5
+ *   524,288                    26.1 72.5  175 / 20.3 42.5 80.7 / 25.3 53.9  104
+ *   750,000                    31.4  104  277 / 30.6 79.7  175 / 28.8 63.9  126
+ * 1,000,000                    40.3  160  464 / 33.5 91.7  213 / 32.5 73.4  151
+ * 2,097,152                    76.5  533 1711                  / 61.8  180  433 */
 constexpr int RS_T256 = 32768, RS_T512 = 196608, RS_T2048 = 655360;
 
 static hipError_t launch_full_sort(const SortArgs& a, int par, hipStream_t s) {
@@ -666,10 +668,10 @@ hipError_t launch_sort(const SortArgs& a, bool incremental, int par, hipStream_t
     auto go = [&](auto kernel, int threads, int tile) {
       hipLaunchKernelGGL(kernel, dim3((a.n + tile - 1) / tile + extra), dim3(threads), 0, s, a, par);
     };
-    if (a.n <= RS_T256) go(k_resort<256, 1>, 256, 256);
-    else if (a.n <= RS_T512) go(k_resort<512, 1>, 512, 512);
-    else if (a.n <= RS_T2048) go(k_resort<1024, 2>, 1024, 2048);
-    else go(k_resort<1024, 4>, 1024, 4096);
+    if (a.n <= RS_T256) go(k_resort<256, 1, 1>, 256, 256);
+    else if (a.n <= RS_T512) go(k_resort<512, 1, 1>, 512, 512);
+    else if (a.n <= RS_T2048) go(k_resort<1024, 2, 1>, 1024, 2048);
+    else go(k_resort<1024, 4, 4>, 1024, 4096);
     return hipGetLastError();
   }
   if (a.turn.params) launch_turn_lifters(a.turn, s);
