@@ -1458,11 +1458,20 @@ __global__ __launch_bounds__(64 * LIST2_WAVES) __attribute__((amdgpu_waves_per_e
  * past the table, its row was cut off there, or j's list overflowed. */
 __device__ __forceinline__ bool listed_back(const uint32_t* __restrict__ list32, const uint32_t* __restrict__ nn, int i,
                                             int k, int j) {
-  int ours = 0, theirs = 0;
-  for (int q = 0; q < k; ++q) ours += list32[(size_t)i * LIST_STRIDE + q] == (uint32_t)j ? 1 : 0;
-  const int m = (int)min(nn[j], (uint32_t)LIST_STRIDE);
-  for (int q = 0; q < m; ++q) theirs += list32[(size_t)j * LIST_STRIDE + q] == (uint32_t)i ? 1 : 0;
-  return ours < theirs;
+  auto named = [&](int row, uint32_t other) {   /* bit q: entry q of the row's list names it */
+    const uint4* const l = reinterpret_cast<const uint4*>(list32 + (size_t)row * LIST_STRIDE);
+    uint32_t m = 0u;
+#pragma unroll
+    for (int q = 0; q < LIST_STRIDE / 4; ++q) {
+      const uint4 v = l[q];
+      m |= ((v.x == other ? 1u : 0u) | (v.y == other ? 2u : 0u) | (v.z == other ? 4u : 0u) | (v.w == other ? 8u : 0u))
+           << (4 * q);
+    }
+    return m;
+  };
+  const uint32_t ours = named(i, (uint32_t)j) & ((1u << k) - 1u);
+  const uint32_t m = nn[j], theirs = named(j, (uint32_t)i) & (m < 32u ? (1u << m) - 1u : 0xFFFFFFFFu);
+  return __popc(ours) < __popc(theirs);
 }
 
 /* The separating-plane test of the pairs listed by PPB consecutive
@@ -1497,7 +1506,7 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
   static_assert(PPB * LIST_STRIDE <= 65536, "slots of a block fit 16 bits");
   const DevParams& P = *Pp;
   __shared__ uint16_t items[PPB * LIST_STRIDE], left[PPB * LIST_STRIDE];
-  __shared__ uint32_t nitems, nleft, nout, qbase;
+  __shared__ uint32_t nitems, nask, nleft, nout, qbase;
   const int lane = threadIdx.x & 63;
   const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
   const int base = xcd_block(blockIdx.x, gridDim.x) * PPB;
@@ -1529,7 +1538,7 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
     p.vbB = p.hb.vbound * P.vbound_scale;
     return p;
   };
-  if (threadIdx.x == 0) { nitems = 0u; nleft = 0u; nout = 0u; }
+  if (threadIdx.x == 0) { nitems = 0u; nask = 0u; nleft = 0u; nout = 0u; }
   __syncthreads();
   /* two threads a particle, 16 list entries each in four loads */
   const bool over = qcount[POLY_OVERFLOW * POLY_QSTRIDE] != 0u;
@@ -1548,13 +1557,17 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
       if (4 * q < m) v = *reinterpret_cast<const uint4*>(list32 + (size_t)i * LIST_STRIDE + k0 + 4 * q);
       js[4 * q] = v.x; js[4 * q + 1] = v.y; js[4 * q + 2] = v.z; js[4 * q + 3] = v.w;
     }
-    uint32_t want = 0u;
+    uint32_t want = 0u, ask = 0u;   /* entries to test, entries to look up first */
 #pragma unroll
     for (int q = 0; q < LIST_STRIDE / 2; ++q) {
-      bool w = q < m && js[q] > (uint32_t)i;
-      if ((look || over) && q < m && !w)
-        w = (look || nn[js[q]] > (uint32_t)LIST_STRIDE) && !listed_back(list32, nn, i, k0 + q, (int)js[q]);
+      const bool w = q < m && js[q] > (uint32_t)i;
       want |= (w ? 1u : 0u) << q;
+      if ((look || over) && q < m && !w) ask |= (look || nn[js[q]] > (uint32_t)LIST_STRIDE ? 1u : 0u) << q;
+    }
+    while (ask) {
+      const int q = __ffs(ask) - 1;
+      ask &= ask - 1u;
+      left[atomicAdd(&nask, 1u)] = (uint16_t)((t >> 1) * LIST_STRIDE + k0 + q);
     }
     const int own = __popc(want);
     int incl = own;
@@ -1573,6 +1586,16 @@ __global__ __launch_bounds__(256) void k_poly_pairs(const DevParams* __restrict_
     }
   }
   __syncthreads();
+  if (nask != 0u) {   /* a thread per entry, not per particle: 16 us of a launch while one did its own */
+    for (uint32_t q0 = 0u; q0 < nask; q0 += 256u) {
+      const uint32_t q = q0 + threadIdx.x;
+      const uint32_t e = q < nask ? left[q] : 0u;
+      const int i = base + (int)(e / LIST_STRIDE), k = (int)(e % LIST_STRIDE);
+      const bool w = q < nask && !listed_back(list32, nn, i, k, (int)list32[(size_t)i * LIST_STRIDE + k]);
+      push(items, &nitems, w, e);
+    }
+    __syncthreads();
+  }
   const uint32_t cnt = nitems;
   for (uint32_t q0 = 0u; q0 < cnt; q0 += 256u) {
     const uint32_t q = q0 + threadIdx.x;

@@ -3,9 +3,10 @@ contact, against the FP32 restatement, which computes every listed entry on
 its own: more z than x cells (hulls whose hash passes the cell table list
 their neighbours and are not listed back, and rows that end past it are
 dropped), grids two or three cells thin (two rows of a stencil share cells,
-and a partner is listed twice), and hulls outside the grid.  Both list
-kernels (24,577 hulls and more take the second).  Forces and states within
-the build's 1e-5 bar (bit-equal away from the quaternion's sine and cosine)."""
+and a partner is listed twice), hulls outside the grid, and packs whose lists
+overflow.  Both list kernels (24,577 hulls and more take the second).  Forces
+and states within the build's 1e-5 bar (bit-equal away from the quaternion's
+sine and cosine)."""
 import numpy as np
 import pytest
 
@@ -59,17 +60,19 @@ def unmatched(lists, counts):
 CASES = [((4, 4, 7), None, 0), ((2, 2, 5), None, 0), ((4, 4, 2), None, 0), ((2, 4, 4), None, 0), ((3, 3, 3), None, 0),
          ((5, 2, 6), None, 0), ((6, 5, 1), None, 0), ((1, 6, 6), None, 0), ((5, 5, 5), None, 24), ((4, 4, 7), None, 24),
          ((10, 10, 42), 24576, 40), ((10, 10, 42), 24577, 40), ((70, 60, 2), 26000, 0)]
+CASES = [c + (0.55,) for c in CASES] + [((6, 6, 6), None, 0, 0.45), ((4, 4, 7), None, 8, 0.45), ((13, 13, 16), None, 0, 0.45)]
 
 
-@pytest.mark.parametrize("cells,n,outside", CASES)
-def test_forces_and_states_equal_the_oracle(cells, n, outside):
-    print(f"[case] grid {cells} n={n} outside={outside}", flush=True)
-    deck = grid_deck(cells, n, outside)
+@pytest.mark.parametrize("cells,n,outside,spacing", CASES)
+def test_forces_and_states_equal_the_oracle(cells, n, outside, spacing):
+    print(f"[case] grid {cells} n={n} outside={outside} spacing={spacing}", flush=True)
+    deck = grid_deck(cells, n, outside, spacing)
     dev, ora = make_pair(deck)
     try:
         lo, no = ora.contacts()
         one, twice = unmatched(lo, no)
         assert one + twice > 0 or cells in ((3, 3, 3), (6, 5, 1))
+        assert spacing > 0.5 or no.max() > 32
         lg, ng = dev.debug_contacts()
         assert np.array_equal(ng, no)
         for i in np.nonzero(no)[0]:
