@@ -173,7 +173,7 @@ __device__ __forceinline__ int wave_find_unchanged(const uint8_t* __restrict__ c
  * read while the one EARLY before it is stored.  (Stream by stream, each load
  * behind the previous store, took 5-7 us of a 13-15 us block.)  The largest
  * tile leaves one block a CU at a million slots, so all four of a thread's
- * slots are read at the start, at 92 VGPRs: 28.6 us for the settled silo's
+ * slots are read at the start, at 92 VGPRs: 27.3 us for the settled silo's
  * sort against 33.7 with one early and 32.1 with 512 slots a block.  Two
  * blocks a CU hide each other's waits, and one early slot is the better
  * choice for 2,048.  The output's keys are kept in LDS for the cell bounds.
@@ -226,18 +226,22 @@ __global__ __launch_bounds__(T) void k_resort(SortArgs a, int par) {
     const int s = s0 + min(it * T + tid, cnt - 1);
     return State{a.pos_cur[s], a.vel_cur[s], a.omg_cur[s], a.hwc_cur ? a.hwc_cur[s] : 0u};
   };
-  State st[EARLY];   /* items it .. it + EARLY - 1 */
+  uint8_t cf[ITEMS];
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int s = s0 + min(it * T + tid, cnt - 1);
+    ok[it] = a.okeys[s];
+    cf[it] = a.changed[s];
+  }
+  State st[EARLY];   /* items it .. it + EARLY - 1; behind the keys, which are waited for first */
 #pragma unroll
   for (int e = 0; e < EARLY; ++e) st[e] = state_of(e);
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
     const int t = it * T + tid;
     const bool mine = t < cnt;
-    const int s = s0 + (mine ? t : cnt - 1);
-    ok[it] = a.okeys[s];
-    const uint8_t cf = a.changed[s];
     if (!mine) ok[it] = 0xFFFFFFFFu;
-    ch[it] = !mine || cf != 0;
+    ch[it] = !mine || cf[it] != 0;
     if (mine) okey_l[t] = ok[it];
     cand[t] = 0;
     bal[it] = __ballot(!ch[it]);
